@@ -33,6 +33,7 @@ HIP_DEV = ["--offload-arch=" + ARCH, "-Xclang", "-target-feature", "-Xclang", "-
 # contraction); the fused FP32/FP16 kernels may contract.
 UNITS = [
     ("kernels_generic.hip", ["-O3", "-ffp-contract=off"] + HIP_DEV),
+    ("kernels_passes.hip", ["-O3", "-ffp-contract=off"] + HIP_DEV),
     ("kernels_fused.hip", ["-O3", "-ffp-contract=fast"] + HIP_DEV),
     ("kernels_batch.hip", ["-O3", "-ffp-contract=off"] + HIP_DEV),
     ("mlp.hip", ["-O3", "-ffp-contract=off"] + HIP_DEV),

@@ -11,9 +11,11 @@
 #include <vector>
 
 #include "../../include/mplb.h"
+#include "boxidx.h"
 #include "case.h"
 #include "fused.h"
 #include "glibc_rand.h"
+#include "passes.h"
 
 using namespace mplb;
 
@@ -397,6 +399,65 @@ int setup_device(mplb_case* c) {
     return 0;
 }
 
+// A boundary list whose condition changes populations (see boundaries_t)
+bool list_active(const FieldCfg& fc, int b) {
+    const int t = fc.bctype[b];
+    if (t == BD_PERIODIC || t == BD_FEP || t == BD_UHF || t == BD_FGT) return false;
+    return !(t == BD_FU && fc.mp.model != M_LIMRT);   // fixedU.c:10: liMRT only
+}
+
+// The fused passes take a case when f is updated, every active list is bounceBack, fixedT
+// or fixedRandomT without hazards inside it, and no node is on two of a field's active
+// lists: such a list's result depends on pulled populations and on earlier lists only, so
+// it can be formed outside the population buffer.  Other cases (frozen f, fixedU, outflow,
+// overlapping lists) run one kernel per routine.
+int setup_passes(mplb_case* c) {
+    const Mesh& m = c->mesh;
+    if (!c->update[0] || m.N >= (int64_t(1) << 31) - 256 || m.bd.size() > 254) return 0;
+    std::vector<uint8_t> order[2], any(m.N, 0);
+    bool lists[2] = {false, false};
+    for (int f = 0; f < 2; f++) {
+        if (!c->fc[f].present || !c->update[f]) continue;
+        order[f].assign(m.N, 255);
+        for (size_t b = 0; b < m.bd.size(); b++) {
+            if (!list_active(c->fc[f], (int)b) || m.bd[b].empty()) continue;
+            const int t = c->fc[f].bctype[b];
+            if ((t != BD_BBACK && t != BD_FT && t != BD_FRDT) || c->bd[b].sequential[f]) return 0;
+            if (f == 0 && t != BD_BBACK) return 0;
+            lists[f] = true;
+            for (int32_t id : m.bd[b]) {
+                if (order[f][id] != 255) return 0;
+                order[f][id] = (uint8_t)b;
+                any[id] = 1;
+            }
+        }
+    }
+    // neighbours are computed from coordinates where the lattice is a box in box order; a
+    // lattice read from files may have odd links or listed nodes off the surface
+    bool box = m.structured;
+    if (box && !m.points.empty()) {
+        const int64_t nxy = (int64_t)m.nx * m.ny;
+        for (int64_t id = 0; id < m.N && box; id++) {
+            const int i = (int)(id % m.nx), j = (int)((id / m.nx) % m.ny), k = (int)(id / nxy);
+            if (i == 0 || i == m.nx - 1 || j == 0 || j == m.ny - 1 || (m.d == 3 && (k == 0 || k == m.nz - 1))) continue;
+            box = !any[id];
+            for (int q = 0; q < m.Q && box; q++) {
+                const int* cq = m.lbmodel == 0 ? D2Q9::t.c[q] : D3Q15::t.c[q];
+                box = m.nb[id * m.Q + q] == id - cq[0] - (int64_t)cq[1] * m.nx - cq[2] * nxy;
+            }
+        }
+    }
+    c->pass_faces = box ? odd_faces(m, any) : kAllTable;
+    for (int f = 0; f < 2; f++) {
+        if (!lists[f]) continue;
+        HIPCHK(c, hipMalloc(&c->order[f], m.N));
+        HIPCHK(c, hipMemcpy(c->order[f], order[f].data(), m.N, hipMemcpyHostToDevice));
+    }
+    if (c->fc[1].present && c->update[1]) HIPCHK(c, hipMalloc(&c->sumg, c->scalar_bytes * m.N));
+    c->passes = true;
+    return 0;
+}
+
 template <typename T>
 DevState<T> state(mplb_case* c) {
     DevState<T> s;
@@ -484,27 +545,33 @@ int stream_t(mplb_case* c, int field) {
     return 0;
 }
 
+// List b of a field as its next application sees it (counts a fixedRandomT step)
+BdList next_list(mplb_case* c, int field, size_t b) {
+    FieldCfg& fc = c->fc[field];
+    const int t = fc.bctype[b];
+    BdList bl{};
+    bl.nodes = c->bd[b].nodes;
+    bl.n = c->bd[b].n;
+    bl.type = t;
+    bl.sequential = c->bd[b].sequential[field];
+    for (int j = 0; j < 3; j++) bl.value[j] = fc.bcval[b][j];
+    bl.pert = fc.pert[b];
+    bl.rnd = c->rnd;
+    bl.rnd_off = c->bd[b].rnd_off[field];
+    bl.draw = (t == BD_FRDT) ? (fc.localT[b] < fc.psteps[b] ? 1 : 0) : 0;
+    if (t == BD_FRDT) fc.localT[b]++;
+    return bl;
+}
+
 template <typename T>
 int boundaries_t(mplb_case* c, int field) {
     if (!c->fc[field].present || !c->update[field]) return 0;
     FieldCfg& fc = c->fc[field];
     TimedRegion tr(c, TM_BOUNDARY);
     for (size_t b = 0; b < c->bd.size(); b++) {
-        const int t = fc.bctype[b];
-        if (t == BD_PERIODIC || t == BD_FEP || t == BD_UHF || t == BD_FGT) continue;
-        if (t == BD_FU && fc.mp.model != M_LIMRT) continue;   // fixedU.c:10: liMRT only
-        BdList bl{};
-        bl.nodes = c->bd[b].nodes;
-        bl.n = c->bd[b].n;
-        bl.type = t;
-        bl.sequential = c->bd[b].sequential[field];
-        for (int j = 0; j < 3; j++) bl.value[j] = fc.bcval[b][j];
-        bl.pert = fc.pert[b];
-        bl.rnd = c->rnd;
-        bl.rnd_off = c->bd[b].rnd_off[field];
-        bl.draw = (t == BD_FRDT) ? (fc.localT[b] < fc.psteps[b] ? 1 : 0) : 0;
+        if (!list_active(fc, (int)b)) continue;
+        const BdList bl = next_list(c, field, b);
         GenericOps<T>::boundary(c->mesh.lbmodel, c->stream, c->eos, fc.mp, state<T>(c), (T*)c->f[field], bl, c->rho0);
-        if (t == BD_FRDT) fc.localT[b]++;
     }
     return 0;
 }
@@ -656,10 +723,89 @@ int one_step_t(mplb_case* c) {
     return 0;
 }
 
+// m steps of multiPhasePP.c:157-241 in fused passes (kernels_passes.hip), from and to the
+// per-routine state; level0 is the time level before the first of them
+template <typename T>
+void run_passes_t(mplb_case* c, int m, int level0) {
+    const Mesh& ms = c->mesh;
+    const bool thermal = c->fc[1].present && c->update[1];
+    collision_t<T>(c, 0);
+    collision_t<T>(c, 1);
+    PassArgs<T> a{};
+    a.nx = ms.nx;
+    a.ny = ms.ny;
+    a.nz = ms.nz;
+    a.N = ms.N;
+    a.nxy = (int64_t)ms.nx * ms.ny;
+    a.face_table = c->pass_faces;
+    a.nb = c->nb;
+    a.onbnd = c->onbnd;
+    a.order[0] = c->order[0];
+    a.order[1] = c->order[1];
+    a.eos = c->eos;
+    a.fp = c->fc[0].mp;
+    a.gp = c->fc[1].mp;
+    a.rho0 = T(c->rho0);
+    a.rho = (T*)c->rho;
+    a.temp = (T*)c->temp;
+    a.U = (T*)c->U;
+    a.Fi = (T*)c->Fi;
+    a.Ft = (T*)c->Ft;
+    a.ss = (T*)c->ss;
+    a.psi = (T*)c->psi;
+    a.sumg = (T*)c->sumg;
+    for (int i = 0; i < m; i++) {
+        a.fin = (const T*)c->f[0];
+        a.fout = (T*)c->f_alt[0];
+        a.gin = (const T*)c->f[1];
+        a.gout = (T*)c->f_alt[1];
+        a.first_call = level0 + 1 + i == 0 ? 1 : 0;
+        for (int fld = 0; fld < (thermal ? 2 : 1); fld++) {
+            if (!c->order[fld]) continue;
+            TimedRegion tr(c, TM_BOUNDARY);
+            for (size_t b = 0; b < c->bd.size(); b++)
+                if (list_active(c->fc[fld], (int)b))
+                    PassOps<T>::boundary(ms.lbmodel, c->stream, a, fld, (int)b, next_list(c, fld, b));
+        }
+        {
+            TimedRegion tr(c, TM_MACRO);
+            PassOps<T>::density(ms.lbmodel, c->stream, a, thermal);
+        }
+        if (thermal) {
+            TimedRegion tr(c, TM_HEAT);
+            PassOps<T>::heat(ms.lbmodel, c->stream, a);
+        }
+        {
+            TimedRegion tr(c, TM_COLLIDE);
+            PassOps<T>::collide(ms.lbmodel, c->stream, a, thermal, i == m - 1);
+        }
+        for (int fld = 0; fld < (thermal ? 2 : 1); fld++) std::swap(c->f[fld], c->f_alt[fld]);
+    }
+    c->psi_valid = true;
+}
+
 template <typename T>
 int steps_t(mplb_case* c, int nsteps, int* done) {
     int n = 0;
-    while (n < nsteps && update_time(c)) {
+    bool more = true;
+    while (c->passes && more && n < nsteps) {
+        // the steps up to and including the next write step go out as one run
+        const int level0 = c->current;
+        int m = 0;
+        bool write = false;
+        while (n + m < nsteps && !write && (more = update_time(c))) {
+            m++;
+            write = c->stp == c->write_interval;
+        }
+        if (m) run_passes_t<T>(c, m, level0);
+        n += m;
+        const int rc = write ? write_step_t<T>(c) : 0;
+        if (rc) {
+            if (done) *done = n;
+            return rc;
+        }
+    }
+    while (!c->passes && n < nsteps && update_time(c)) {
         int rc = one_step_t<T>(c);
         n++;
         if (rc) {
@@ -789,11 +935,7 @@ int mplb_case_open(const char* case_dir, const mplb_opts* opts, mplb_case** out)
     }
     rc = setup_device(c);
     if (rc) return rc;
-    if (c->fused) {
-        rc = fused_create(c);
-        if (rc) return rc;
-    }
-    return 0;
+    return c->fused ? fused_create(c) : setup_passes(c);
 }
 
 int mplb_case_close(mplb_case* c) {
@@ -802,7 +944,7 @@ int mplb_case_close(mplb_case* c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     if (c->fused) fused_destroy(c);
     void* ptrs[] = {c->f[0], c->f[1], c->f_alt[0], c->f_alt[1], c->rho, c->temp, c->p, c->U, c->Fi, c->Ft, c->ss, c->psi,
-                    c->nb, c->onbnd, c->rnd, c->red, c->nanc, c->rho_snap};
+                    c->nb, c->onbnd, c->rnd, c->red, c->nanc, c->rho_snap, c->order[0], c->order[1], c->sumg};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (auto& b : c->bd) {

@@ -79,6 +79,12 @@ struct mplb_case {
     void* rho_snap = nullptr;                   // density snapshot of mplb_density_change
     bool snap_valid = false;
 
+    // fused passes of the per-routine arithmetic (kernels_passes.hip)
+    bool passes = false;
+    int pass_faces = 0;                         // faces read through the neighbour table
+    uint8_t* order[2] = {nullptr, nullptr};     // per field: each node's boundary list (255: none)
+    void* sumg = nullptr;
+
     // fused structured-box path
     bool fused = false;
     void* fz = nullptr;                         // fused-state handle (kernels_fused.hip)

@@ -25,6 +25,7 @@
 #include <unordered_map>
 #include <vector>
 
+#include "boxidx.h"
 #include "case.h"
 #include "fused.h"
 #include "physics.h"
@@ -184,15 +185,6 @@ __device__ inline void stf_ref(void* p, int64_t i, int q, float v, float R, floa
     else ((_Float16*)p)[i] = (_Float16)dev;
 }
 
-struct NodePos {
-    int i, j, k;
-    int64_t id;
-    bool surface;       // on the box surface
-    bool table;         // on a face whose links must be read from the neighbour table
-    bool valid;
-    unsigned X[3], Y[3], Z[3];   // wrapped coordinates u-1, u, u+1 premultiplied by the strides
-};
-
 // psi = potential(rho, T) (potential.c:7-13) in FP32 with the loop-invariant factors taken
 // from the host for the van der Waals EOS (one division instead of three); other EOS
 // types use the shared form.
@@ -209,58 +201,6 @@ __device__ inline float fpot(const FArgs& a, float rho, float T) {
         return sqrt_fast(2.f * (p - rho * float(kCs2)) * a.vinv_g);
     }
     return potential<float>(a.eos, rho, T);
-}
-
-// Block b covers the 256 consecutive node ids [256 b, 256 b + 256).
-template <class L>
-__device__ inline NodePos node_pos(const FArgs& a) {
-    NodePos p;
-    const unsigned id = blockIdx.x * 256u + threadIdx.x;     // N < 2^31
-    const unsigned nxy = (unsigned)a.nxy, nx = (unsigned)a.nx;
-    p.id = id;
-    p.valid = p.id < a.N;
-    const unsigned k = id / nxy, r = id - k * nxy, j = r / nx;
-    p.k = (int)k;
-    p.j = (int)j;
-    p.i = (int)(r - j * nx);
-    const bool x0 = p.i == 0, x1 = p.i == a.nx - 1, y0 = p.j == 0, y1 = p.j == a.ny - 1;
-    const bool z0 = L::D == 3 && p.k == 0, z1 = L::D == 3 && p.k == a.nz - 1;
-    p.surface = x0 || x1 || y0 || y1 || z0 || z1;
-    const int m = a.face_table;
-    p.table = (x0 && (m & 1)) || (x1 && (m & 2)) || (y0 && (m & 4)) || (y1 && (m & 8)) || (z0 && (m & 16)) ||
-              (z1 && (m & 32));
-    // periodic wrap with duplicate end nodes: u - 1 at 0 is n - 2, u + 1 at n - 1 is 1
-    p.X[0] = x0 ? nx - 2 : p.i - 1;
-    p.X[1] = p.i;
-    p.X[2] = x1 ? 1 : p.i + 1;
-    p.Y[0] = (y0 ? a.ny - 2 : p.j - 1) * nx;
-    p.Y[1] = j * nx;
-    p.Y[2] = (y1 ? 1 : p.j + 1) * nx;
-    if (L::D == 3) {
-        p.Z[0] = (z0 ? a.nz - 2 : p.k - 1) * nxy;
-        p.Z[1] = k * nxy;
-        p.Z[2] = (z1 ? 1 : p.k + 1) * nxy;
-    } else {
-        p.Z[0] = p.Z[1] = p.Z[2] = 0;
-    }
-    return p;
-}
-
-// upstream node x - c_q (lbstream.c:16-62: a missing link keeps the node's own value)
-template <class L>
-__device__ inline unsigned upstream(const FArgs& a, const NodePos& p, int q) {
-    if (p.table) {
-        const int s = a.nb[q * a.N + p.id];
-        return s == -1 ? (unsigned)p.id : (unsigned)s;
-    }
-    return p.X[1 - L::t.c[q][0]] + p.Y[1 - L::t.c[q][1]] + p.Z[1 - L::t.c[q][2]];
-}
-
-// downstream node x + c_q (the interaction-force and stencil neighbour), -1 if missing
-template <class L>
-__device__ inline int64_t downstream(const FArgs& a, const NodePos& p, int q) {
-    if (p.table) return a.nb[L::t.rev[q] * a.N + p.id];
-    return (int64_t)(p.X[1 + L::t.c[q][0]] + p.Y[1 + L::t.c[q][1]] + p.Z[1 + L::t.c[q][2]]);
 }
 
 // REF: f stored against per-node references (FP16N); otherwise shift holds the storage
@@ -2111,49 +2051,10 @@ int fused_create(mplb_case* c) {
             }
         }
     }
-    // Faces read through the neighbour table: together they hold every node whose links
-    // are not the duplicate-node periodic wrap or that carries a boundary condition.  A
-    // node on an edge lies on two faces, and either one covers it, so the cheapest cover is
-    // taken: a y or z face is nx consecutive nodes per row (few wavefronts), while an x face
-    // puts one table lane into a wavefront of every row, which then pulls twice.  (The
-    // walled planes of a column have odd links along their edges: covered by all six faces
-    // every wavefront of a 128-wide column took both paths, 1.29 ms per step at 128 x 128 x
-    // 384 with heat transfer against 0.56 with the two walls alone.)
     {
-        const int nx = m.nx, ny = m.ny, nz = m.nz;
-        const int64_t nxy = (int64_t)nx * ny;
-        auto wrapc = [](int u, int n) { return u < 0 ? u + (n - 1) : (u > n - 1 ? u - (n - 1) : u); };
-        bool seen[64] = {false};           // face sets of the nodes that need the table
-        for (int64_t id = 0; id < N; id++) {
-            const int i = (int)(id % nx), j = (int)((id / nx) % ny), k = (int)(id / nxy);
-            int faces = (i == 0 ? 1 : 0) | (i == nx - 1 ? 2 : 0) | (j == 0 ? 4 : 0) | (j == ny - 1 ? 8 : 0);
-            if (m.d == 3) faces |= (k == 0 ? 16 : 0) | (k == nz - 1 ? 32 : 0);
-            if (!faces || seen[faces]) continue;
-            bool differs = bcf[id] != FB_NONE || bcg[id] != FB_NONE;
-            for (int q = 0; q < Q && !differs; q++) {
-                const int* cq = m.lbmodel == 0 ? D2Q9::t.c[q] : D3Q15::t.c[q];
-                const int64_t want = wrapc(i - cq[0], nx) + (int64_t)wrapc(j - cq[1], ny) * nx +
-                                     (m.d == 3 ? (int64_t)wrapc(k - cq[2], nz) * nxy : 0);
-                if (m.nb[id * Q + q] != want) differs = true;
-            }
-            if (differs) seen[faces] = true;
-        }
-        // wavefronts that a face puts on the table path
-        const int64_t rows = (int64_t)ny * nz, wx = (nx + 63) / 64;
-        const int64_t cost[6] = {rows, rows, wx * nz, wx * nz, wx * ny, wx * ny};
-        int best = 0;
-        int64_t best_cost = -1;
-        for (int mask = 0; mask < 64; mask++) {
-            bool covers = true;
-            int64_t w = 0;
-            for (int f = 1; f < 64 && covers; f++) covers = !seen[f] || (f & mask);
-            for (int b = 0; b < 6; b++) w += (mask >> b & 1) ? cost[b] : 0;
-            if (covers && (best_cost < 0 || w < best_cost)) {
-                best = mask;
-                best_cost = w;
-            }
-        }
-        z->face_table = best;
+        std::vector<uint8_t> bc(N);
+        for (int64_t id = 0; id < N; id++) bc[id] = bcf[id] != FB_NONE || bcg[id] != FB_NONE;
+        z->face_table = odd_faces(m, bc);
     }
     // single-pass kernel: isothermal D3Q15 with every link the periodic wrap and no
     // boundary node (MPLB_FUSED_KERNEL=twopass keeps the two-pass kernels)

@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include "kernels.h"
+#include "node.h"
 
 namespace mplb {
 
@@ -38,295 +39,97 @@ __global__ void k_psi(int64_t N, EosParams e, const T* __restrict__ rho, const T
     psi[id] = potential<T>(e, rho[id], temp[id]);
 }
 
+// psi at the downstream nodes x + c_k of node id; false when a link is missing (its entry
+// is the node's own psi)
+template <class L, typename T>
+__device__ inline bool psi_stencil(const DevState<T>& st, int64_t id, T* psin) {
+    bool full = true;
+#pragma unroll
+    for (int k = 1; k < L::Q; k++) {
+        const int nid = st.nb[L::t.rev[k] * st.N + id];
+        full = full && nid != -1;
+        psin[k] = st.psi[nid == -1 ? id : (int64_t)nid];
+    }
+    return full;
+}
+
 // interForce.c:16-39 with interactionForce.c:47-79
 template <class L, typename T>
 __global__ void k_inter_force(DevState<T> st, EosParams e, T rho0) {
     const int64_t N = st.N;
     const int64_t id = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (id >= N) return;
-    T F[3] = {T(0.0), T(0.0), T(0.0)};
-    T Ff[3] = {T(0), T(0), T(0)};
+    T psin[L::Q], Ff[3], Ft[3];
     const bool interior = st.onbnd[id] == 0;
-    if (interior) {
-#pragma unroll
-        for (int k = 1; k < L::Q; k++) {
-            const int nid = st.nb[L::t.rev[k] * N + id];
-            const T alpha = T(L::t.w[k]) * st.psi[nid];
-#pragma unroll
-            for (int i = 0; i < 3; i++) {
-                const int c = L::t.c[k][i];
-                if (c == 1) F[i] += alpha;
-                else if (c == -1) F[i] += -alpha;
-            }
-        }
-        const T beta = -T(e.G) * st.psi[id];
-#pragma unroll
-        for (int i = 0; i < 3; i++) Ff[i] = F[i] * beta;
-    }
-    const T r = st.rho[id];
+    if (interior) psi_stencil<L, T>(st, id, psin);
+    node_force<L, T>(e, psin, st.psi[id], interior, Ff);
+    node_total_force<T>(e, Ff, st.rho[id], rho0, interior, Ft);
 #pragma unroll
     for (int j = 0; j < 3; j++) {
         st.Fi[j * N + id] = Ff[j];
-        T ft = Ff[j] + (r - rho0) * T(e.g[j]);
-        if (interior) ft += T(e.fext[j]);
-        st.Ft[j * N + id] = ft;
+        st.Ft[j * N + id] = Ft[j];
     }
 }
 
-// liMRTSurfaceTension.c:11-132 (D2Q9) / xuMRTSurfaceTension.c:57-122 (D3Q15)
+// surface-tension moments of node id (zero next to missing links)
 template <class L, typename T>
 __device__ inline void surface_tension(const DevState<T>& st, const EosParams& e, const ModelParams& mp,
                                        int64_t id, T* C) {
-    const int64_t N = st.N;
-    const T psi = st.psi[id];
-    int noneigh = 0;
-#pragma unroll
-    for (int k = 1; k < L::Q; k++)
-        if (st.nb[k * N + id] == -1) noneigh++;
+    T psin[L::Q];
 #pragma unroll
     for (int k = 0; k < L::Q; k++) C[k] = T(0);
-    if (noneigh != 0) return;
-    T Qt[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-#pragma unroll
-    for (int k = 1; k < L::Q; k++) {
-        const int nid = st.nb[L::t.rev[k] * N + id];
-        const T alpha = T(L::t.w[k]) * (st.psi[nid] - psi);
-#pragma unroll
-        for (int i = 0; i < L::D; i++)
-#pragma unroll
-            for (int j = (L::D == 2 ? 0 : i); j < L::D; j++) {
-                const int cc = L::t.c[k][i] * L::t.c[k][j];
-                if (cc == 1) Qt[i][j] += alpha;
-                else if (cc == -1) Qt[i][j] += -alpha;
-            }
-    }
-    const T G = T(e.G), kap = T(mp.kappa);
-#pragma unroll
-    for (int i = 0; i < L::D; i++)
-#pragma unroll
-        for (int j = (L::D == 2 ? 0 : i); j < L::D; j++) Qt[i][j] = Qt[i][j] * T(0.5) * psi * G * kap;
-    if (L::D == 2) {
-        C[1] = T(1.5) * T(mp.Lambda[1]) * (Qt[0][0] + Qt[1][1]);
-        C[2] = T(-1.5) * T(mp.Lambda[2]) * (Qt[0][0] + Qt[1][1]);
-        C[7] = -T(mp.Lambda[8]) * (Qt[0][0] - Qt[1][1]);
-        C[8] = -T(mp.Lambda[8]) * Qt[0][1];
-    } else {
-        C[1] = T(4.0) * T(mp.Lambda[1]) * (Qt[0][0] + Qt[1][1] + Qt[2][2]) / T(5.0);
-        const T l10 = -T(mp.Lambda[10]);
-        C[9] = l10 * (T(2) * Qt[0][0] - Qt[1][1] - Qt[2][2]);
-        C[10] = l10 * (Qt[1][1] - Qt[2][2]);
-        C[11] = l10 * Qt[0][1];
-        C[12] = l10 * Qt[1][2];
-        C[13] = l10 * Qt[0][2];
-    }
+    if (psi_stencil<L, T>(st, id, psin)) node_surface_tension<L, T>(e, mp, psin, st.psi[id], C);
 }
 
-// liMRTCollision.c:33-106 with liMRTForce.c:13-42 (D2Q9)
 template <class L, typename T>
 __global__ void k_collide_limrt(DevState<T> st, EosParams e, ModelParams mp, T* __restrict__ f) {
     const int64_t N = st.N;
     const int64_t id = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (id >= N) return;
-    T fv[L::Q], m[L::Q], meq[L::Q], S[L::Q], C[L::Q];
+    T fv[L::Q], C[L::Q];
     load_pops<L, T>(f, N, id, fv);
-    const T rho = st.rho[id];
     const T U[3] = {st.U[id], st.U[N + id], st.U[2 * N + id]};
-    T umag = 0;
-#pragma unroll
-    for (int k = 0; k < 3; k++) umag += U[k] * U[k];
-    meq[0] = rho;
-    meq[1] = rho * (T(-2) + T(3) * umag);
-    meq[2] = rho * (T(1) - T(3) * umag);
-    meq[3] = rho * U[0];
-    meq[4] = rho * (-U[0]);
-    meq[5] = rho * U[1];
-    meq[6] = rho * (-U[1]);
-    meq[7] = rho * (U[0] * U[0] - U[1] * U[1]);
-    meq[8] = rho * U[0] * U[1];
-    moments<L, T>(fv, m);
     const T F[3] = {st.Ft[id], st.Ft[N + id], st.Ft[2 * N + id]};
-    const T Fi0 = st.Fi[id], Fi1 = st.Fi[N + id];
-    const T psi = st.psi[id];
-    const T sigma = T(mp.sigma);
-    const T L1 = T(mp.Lambda[1]), L2 = T(mp.Lambda[2]);
-    S[0] = 0;
-    S[1] = T(6) * (U[0] * F[0] + U[1] * F[1]) +
-           T(12) * sigma * (Fi0 * Fi0 + Fi1 * Fi1) / (psi * psi * ((T(1) / L1) - T(0.5)));
-    S[2] = T(-6) * (U[0] * F[0] + U[1] * F[1]) -
-           T(12) * sigma * (Fi0 * Fi0 + Fi1 * Fi1) / (psi * psi * ((T(1) / L2) - T(0.5)));
-    S[3] = F[0];
-    S[4] = -F[0];
-    S[5] = F[1];
-    S[6] = -F[1];
-    S[7] = T(2) * (U[0] * F[0] - U[1] * F[1]);
-    S[8] = U[0] * F[1] + U[1] * F[0];
     if (mp.surf) surface_tension<L, T>(st, e, mp, id, C);
-#pragma unroll
-    for (int k = 0; k < L::Q; k++) {
-        const T lam = T(mp.Lambda[k]);
-        m[k] = m[k] - lam * (m[k] - meq[k]) + (T(1) - T(0.5) * lam) * S[k];
-        if (mp.surf) m[k] = m[k] + C[k];
-    }
-    populations<L, T>(m, fv);
+    node_collide_limrt<L, T>(mp, fv, st.rho[id], U, F, st.Fi[id], st.Fi[N + id], st.psi[id], C);
     store_pops<L, T>(f, N, id, fv);
 }
 
-// xuMRTCollision.c:42-92 with xuMRTEquilibriumMS.c:23-51 and xuMRTForce.c:18-69 (D3Q15)
 template <class L, typename T>
 __global__ void k_collide_xumrt(DevState<T> st, EosParams e, ModelParams mp, T* __restrict__ f, T rho0) {
     const int64_t N = st.N;
     const int64_t id = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (id >= N) return;
-    T fv[L::Q], m[L::Q], meq[L::Q], S[L::Q], C[L::Q];
+    T fv[L::Q], C[L::Q];
     load_pops<L, T>(f, N, id, fv);
     const T U[3] = {st.U[id], st.U[N + id], st.U[2 * N + id]};
-    const T rho = st.rho[id];
-    T umag = 0;
-#pragma unroll
-    for (int k = 0; k < 3; k++) umag += U[k] * U[k];
-    meq[0] = rho;
-    meq[1] = rho * (T(-1.0) + umag);
-    meq[2] = rho * (T(1.0) - T(5.0) * umag);
-    meq[3] = rho * U[0];
-    meq[4] = rho * T(-7.0) * U[0] / T(3.0);
-    meq[5] = rho * U[1];
-    meq[6] = rho * T(-7.0) * U[1] / T(3.0);
-    meq[7] = rho * U[2];
-    meq[8] = rho * T(-7.0) * U[2] / T(3.0);
-    meq[9] = rho * (T(2.0) * U[0] * U[0] - U[1] * U[1] - U[2] * U[2]);
-    meq[10] = rho * (U[1] * U[1] - U[2] * U[2]);
-    meq[11] = rho * U[0] * U[1];
-    meq[12] = rho * U[1] * U[2];
-    meq[13] = rho * U[0] * U[2];
-    meq[14] = 0;
-    moments<L, T>(fv, m);
-    T F[3];
-#pragma unroll
-    for (int j = 0; j < 3; j++) F[j] = st.Fi[j * N + id] + (rho - rho0) * T(e.g[j]);
-    const T psi = st.psi[id];
-    const T uDotF = U[0] * F[0] + U[1] * F[1] + U[2] * F[2];
-    T fmag = 0;
-#pragma unroll
-    for (int k = 0; k < 3; k++) fmag += F[k] * F[k];
-    const T sigma = T(mp.sigma), L1 = T(mp.Lambda[1]);
-    S[0] = 0;
-    S[1] = T(2.0) * uDotF + (T(6.0) * sigma * fmag) / (psi * psi * ((T(1) / L1) - T(0.5)));
-    S[2] = T(-10.0) * uDotF;
-    S[3] = F[0];
-    S[4] = T(-7.0) * F[0] / T(3.0);
-    S[5] = F[1];
-    S[6] = T(-7.0) * F[1] / T(3.0);
-    S[7] = F[2];
-    S[8] = T(-7.0) * F[2] / T(3.0);
-    S[9] = T(4.0) * U[0] * F[0] - T(2.0) * U[1] * F[1] - T(2.0) * U[2] * F[2];
-    S[10] = T(2.0) * U[1] * F[1] - T(2.0) * U[2] * F[2];
-    S[11] = U[0] * F[1] + U[1] * F[0];
-    S[12] = U[1] * F[2] + U[2] * F[1];
-    S[13] = U[0] * F[2] + U[2] * F[0];
-    S[14] = 0;
+    const T Fi[3] = {st.Fi[id], st.Fi[N + id], st.Fi[2 * N + id]};
     if (mp.surf) surface_tension<L, T>(st, e, mp, id, C);
-#pragma unroll
-    for (int k = 0; k < L::Q; k++) {
-        const T lam = T(mp.Lambda[k]);
-        m[k] = m[k] - lam * (m[k] - meq[k]) + (T(1) - T(0.5) * lam) * S[k];
-        if (mp.surf) m[k] = m[k] + C[k];
-    }
-    populations<L, T>(m, fv);
+    node_collide_xumrt<L, T>(e, mp, fv, st.rho[id], U, Fi, st.psi[id], rho0, C);
     store_pops<L, T>(f, N, id, fv);
 }
 
-// liTempMRTCollision.c:31-84 with liTempMRTEquilibriumMS.c:20-41, liTempMRTSource.c:17-24
 template <class L, typename T>
 __global__ void k_collide_litemp(DevState<T> st, ModelParams mp, T* __restrict__ g) {
     const int64_t N = st.N;
     const int64_t id = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (id >= N) return;
-    T gv[L::Q], n[L::Q], neq[L::Q];
+    T gv[L::Q];
     load_pops<L, T>(g, N, id, gv);
-    const T temp = st.temp[id];
     const T U[3] = {st.U[id], st.U[N + id], st.U[2 * N + id]};
-    neq[0] = temp;
-    neq[1] = T(-2.0) * temp;
-    neq[2] = T(2.0) * temp;
-    neq[3] = temp * U[0];
-    neq[4] = temp * (-U[0]);
-    neq[5] = temp * U[1];
-    neq[6] = temp * (-U[1]);
-    neq[7] = 0;
-    neq[8] = 0;
-    moments<L, T>(gv, n);
-    const T n4 = n[4], n6 = n[6];
-#pragma unroll
-    for (int k = 0; k < L::Q; k++) {
-        const T lam = T(mp.Lambda[k]);
-        const T gam = (k == 0) ? st.ss[id] : T(0);
-        n[k] = n[k] - lam * (n[k] - neq[k]) + gam;
-    }
-    n[3] = n[3] + (T(1) - T(mp.Lambda[3]) / T(2)) * T(mp.Lambda[4]) * n4;
-    n[5] = n[5] + (T(1) - T(mp.Lambda[5]) / T(2)) * T(mp.Lambda[6]) * n6;
-    populations<L, T>(n, gv);
+    node_collide_litemp<L, T>(mp, gv, st.temp[id], U, st.ss[id]);
     store_pops<L, T>(g, N, id, gv);
 }
 
-// myMRTCollision.c:35-212 with myMRTEquilibriumMS.c:20-77 and sparseMatVecMult.c:11-28:
-// Q = diag(Lambda) + Q34, Q56 (, Q78), Q_aux = I - Q/2; n <- n - Q (n - n_eq) + Q_aux Gamma.
 template <class L, typename T>
 __global__ void k_collide_my(DevState<T> st, ModelParams mp, T* __restrict__ g) {
     const int64_t N = st.N;
     const int64_t id = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (id >= N) return;
-    T gv[L::Q], n[L::Q], neq[L::Q], aux1[L::Q], aux2[L::Q];
+    T gv[L::Q];
     load_pops<L, T>(g, N, id, gv);
-    const T temp = st.temp[id];
     const T U[3] = {st.U[id], st.U[N + id], st.U[2 * N + id]};
-#pragma unroll
-    for (int k = 0; k < L::Q; k++) neq[k] = T(0);
-    neq[0] = temp;
-    neq[1] = T(mp.alpha1) * temp;
-    neq[2] = T(mp.alpha2) * temp;
-    if (L::D == 2) {
-        neq[3] = temp * U[0];
-        neq[4] = temp * (-U[0]);
-        neq[5] = temp * U[1];
-        neq[6] = temp * (-U[1]);
-    } else {
-        neq[3] = temp * U[0];
-        neq[4] = -(temp * U[0]);
-        neq[5] = temp * U[1];
-        neq[6] = -(temp * U[1]);
-        neq[7] = temp * U[2];
-        neq[8] = -(temp * U[2]);
-    }
-    moments<L, T>(gv, n);
-    // relaxation matrix entries (myMRTCollision.c:39-127), computed as the reference does
-    T Qd[L::Q], Qa[L::Q];
-#pragma unroll
-    for (int k = 0; k < L::Q; k++) {
-        Qd[k] = T(mp.Lambda[k]);
-        Qa[k] = T(1.0) + T(-0.5) * Qd[k];
-    }
-    const int npair = L::D == 2 ? 2 : 3;
-    T Qo[3], Qao[3];
-#pragma unroll
-    for (int pr = 0; pr < 3; pr++) {
-        const int a = 3 + 2 * pr, b = 4 + 2 * pr;
-        Qo[pr] = Qd[b] * (Qd[a] / T(2.0) - T(1.0));
-        Qao[pr] = T(-0.5) * Qo[pr];
-    }
-#pragma unroll
-    for (int k = 0; k < L::Q; k++) aux2[k] = n[k] - neq[k];
-#pragma unroll
-    for (int k = 0; k < L::Q; k++) aux1[k] = Qd[k] * aux2[k];
-#pragma unroll
-    for (int pr = 0; pr < npair; pr++) aux1[3 + 2 * pr] = aux1[3 + 2 * pr] + Qo[pr] * aux2[4 + 2 * pr];
-    const T gam0 = st.ss[id];
-#pragma unroll
-    for (int k = 0; k < L::Q; k++) aux2[k] = Qa[k] * (k == 0 ? gam0 : T(0));
-#pragma unroll
-    for (int pr = 0; pr < npair; pr++) aux2[3 + 2 * pr] = aux2[3 + 2 * pr] + Qao[pr] * T(0);
-#pragma unroll
-    for (int k = 0; k < L::Q; k++) n[k] = n[k] - aux1[k] + aux2[k];
-    populations<L, T>(n, gv);
+    node_collide_my<L, T>(mp, gv, st.temp[id], U, st.ss[id]);
     store_pops<L, T>(g, N, id, gv);
 }
 
@@ -350,20 +153,11 @@ template <class L, typename T>
 __device__ inline void bc_bounceback(const DevState<T>& st, T* f, int64_t id) {
     const int64_t N = st.N;
     T v[L::Q];
-    int miss[L::Q];
+    bool miss[L::Q];
     load_pops<L, T>(f, N, id, v);
 #pragma unroll
     for (int k = 0; k < L::Q; k++) miss[k] = st.nb[k * N + id] == -1;
-#pragma unroll
-    for (int k = 0; k < L::Q; k++) {
-        const int r = L::t.rev[k];
-        if (miss[k]) {
-            v[k] = v[r];
-        } else if (!miss[r] && k >= 1 && k <= L::naxis) {
-            v[k] = T(0.5) * v[k] + T(0.5) * v[r];
-            v[r] = v[k];
-        }
-    }
+    node_bounce_back<L, T>(v, miss);
     store_pops<L, T>(f, N, id, v);
 }
 
@@ -514,10 +308,9 @@ __global__ void k_density(DevState<T> st, const T* __restrict__ f) {
     const int64_t N = st.N;
     const int64_t id = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (id >= N) return;
-    T r = 0;
-#pragma unroll
-    for (int k = 0; k < L::Q; k++) r += f[k * N + id];
-    st.rho[id] = r;
+    T fv[L::Q];
+    load_pops<L, T>(f, N, id, fv);
+    st.rho[id] = node_sum<L, T>(fv);
 }
 
 // macroVelocity.c:17-50 with liMRTVelocity.c:11-50 / xuMRTVelocity.c:19-50
@@ -534,16 +327,7 @@ __global__ void k_velocity(DevState<T> st, EosParams e, int fmodel, const T* __r
     for (int j = 0; j < 3; j++)
         F[j] = fmodel == M_LIMRT ? st.Ft[j * N + id] : st.Fi[j * N + id] + (rho - rho0) * T(e.g[j]);
 #pragma unroll
-    for (int j = 0; j < 3; j++) {
-        T lv = 0;
-#pragma unroll
-        for (int k = 0; k < L::Q; k++) {
-            const int c = L::t.c[k][j];
-            if (c == 1) lv += fv[k];
-            else if (c == -1) lv += -fv[k];
-        }
-        st.U[j * N + id] = (lv + F[j] * T(0.5)) / rho;
-    }
+    for (int j = 0; j < 3; j++) st.U[j * N + id] = node_velocity<L, T>(fv, rho, F[j], j);
 }
 
 // macroTemperature.c:15-63 with myMRTTemperature.c:16-30 / liTempMRTTemperature.c:16-20
@@ -552,34 +336,11 @@ __global__ void k_temperature(DevState<T> st, int gmodel, const T* __restrict__ 
     const int64_t N = st.N;
     const int64_t id = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (id >= N) return;
-    T t = 0;
-#pragma unroll
-    for (int k = 0; k < L::Q; k++) t += g[k * N + id];
+    T gv[L::Q];
+    load_pops<L, T>(g, N, id, gv);
+    T t = node_sum<L, T>(gv);
     if (gmodel == M_MYMRT) t = t + T(0.5) * st.ss[id];
     st.temp[id] = t;
-}
-
-// finiteDifference/{scalarGradient,invScalarGradient,vectorDivergence}.c along one axis.
-template <typename T>
-__device__ inline T fd_axis(const T* q, int a, int b, int64_t id, bool inv, bool* has) {
-    *has = true;
-    if (a != -1 && b != -1) {
-        const T qa = inv ? T(1.0) / q[a] : q[a];
-        const T qb = inv ? T(1.0) / q[b] : q[b];
-        return T(0.5) * (qa - qb);
-    }
-    if (a == -1 && b != -1) {
-        const T qi = inv ? T(1.0) / q[id] : q[id];
-        const T qb = inv ? T(1.0) / q[b] : q[b];
-        return qi - qb;
-    }
-    if (a != -1 && b == -1) {
-        const T qa = inv ? T(1.0) / q[a] : q[a];
-        const T qi = inv ? T(1.0) / q[id] : q[id];
-        return qa - qi;
-    }
-    *has = false;
-    return T(0);
 }
 
 // heatSource.c:26-170: S = -lambda (grad T . grad 1/rho)/Cv + div U T (1 - dp/dT/(rho Cv)),
@@ -590,35 +351,23 @@ __global__ void k_heat_source(DevState<T> st, EosParams e, ModelParams mp, int f
     const int64_t id = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (id >= N) return;
     const T rho = st.rho[id], temp = st.temp[id];
-    const T Cv = T(e.Cv);
-    const T L3 = T(mp.Lambda[3]);
-    T lambda;
-    if (mp.model == M_MYMRT) {
-        if (L::D == 2)
-            lambda = rho * Cv * (T(1) / L3 - T(0.5)) * (T(4.0) + T(3.0) * T(mp.alpha1) + T(2.0) * T(mp.alpha2)) / T(6.0);
-        else
-            lambda = rho * Cv * (T(1) / L3 - T(0.5)) * (T(6.0) + T(11.0) * T(mp.alpha1) + T(mp.alpha2)) / T(9.0);
-    } else {
-        lambda = rho * Cv * (T(1) / L3 - T(0.5));
-    }
     T gT[3] = {0, 0, 0}, gR[3] = {0, 0, 0};
     T divU = 0;
 #pragma unroll
     for (int ax = 0; ax < L::D; ax++) {
         const int a = st.nb[L::fd_plus[ax] * N + id];
         const int b = st.nb[L::fd_minus[ax] * N + id];
-        bool has;
-        gT[ax] = fd_axis<T>(st.temp, a, b, id, false, &has);
-        gR[ax] = fd_axis<T>(st.rho, a, b, id, true, &has);
-        const T dv = fd_axis<T>(st.U + ax * N, a, b, id, false, &has);
-        if (has) divU += dv;
+        const bool ha = a != -1, hb = b != -1;
+        const int64_t ia = ha ? (int64_t)a : id, ib = hb ? (int64_t)b : id;
+        const T* Uax = st.U + ax * N;
+        gT[ax] = node_fd<T>(st.temp[ia], ha, st.temp[ib], hb, temp, false);
+        gR[ax] = node_fd<T>(st.rho[ia], ha, st.rho[ib], hb, rho, true);
+        divU += node_fd<T>(Uax[ia], ha, Uax[ib], hb, Uax[id], false);
     }
     T dot = 0;
 #pragma unroll
     for (int k = 0; k < 3; k++) dot += gT[k] * gR[k];
-    T dpdT = p_eos<T>(e, rho, T(1.1) * temp) - p_eos<T>(e, rho, T(0.9) * temp);
-    dpdT = dpdT / (T(0.2) * temp);
-    const T s = -lambda * dot / Cv + divU * temp * (T(1.0) - dpdT / (rho * Cv));
+    const T s = node_heat<L, T>(e, mp, rho, temp, dot, divU);
     if (mp.model == M_MYMRT) {
         st.ss[id] = s;
     } else {

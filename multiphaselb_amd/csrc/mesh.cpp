@@ -292,4 +292,46 @@ std::string build_box(Mesh& m, double spot_radius, const double spot_centre[2]) 
     return "";
 }
 
+// A node on an edge lies on two faces, and either one covers it, so the cheapest cover is
+// taken: a y or z face is nx consecutive nodes per row (few wavefronts), while an x face
+// puts one table lane into a wavefront of every row, which then pulls twice.  (The walled
+// planes of a column have odd links along their edges: covered by all six faces every
+// wavefront of a 128-wide column took both paths, 1.29 ms per step at 128 x 128 x 384 with
+// heat transfer in FP32 against 0.56 with the two walls alone.)
+int odd_faces(const Mesh& m, const std::vector<uint8_t>& bc) {
+    const int nx = m.nx, ny = m.ny, nz = m.nz;
+    const int64_t nxy = (int64_t)nx * ny;
+    bool seen[64] = {false};               // face sets of the nodes that need the table
+    for (int64_t id = 0; id < m.N; id++) {
+        const int i = (int)(id % nx), j = (int)((id / nx) % ny), k = (int)(id / nxy);
+        int faces = (i == 0 ? 1 : 0) | (i == nx - 1 ? 2 : 0) | (j == 0 ? 4 : 0) | (j == ny - 1 ? 8 : 0);
+        if (m.d == 3) faces |= (k == 0 ? 16 : 0) | (k == nz - 1 ? 32 : 0);
+        if (!faces || seen[faces]) continue;
+        bool differs = bc[id] != 0;
+        for (int q = 0; q < m.Q && !differs; q++) {
+            const int* cq = m.lbmodel == 0 ? kC2[q] : kC3[q];
+            const int64_t want = wrap_dup(i - cq[0], nx) + (int64_t)wrap_dup(j - cq[1], ny) * nx +
+                                 (m.d == 3 ? (int64_t)wrap_dup(k - cq[2], nz) * nxy : 0);
+            if (m.nb[id * m.Q + q] != want) differs = true;
+        }
+        if (differs) seen[faces] = true;
+    }
+    // wavefronts that a face puts on the table path
+    const int64_t rows = (int64_t)ny * nz, wx = (nx + 63) / 64;
+    const int64_t cost[6] = {rows, rows, wx * nz, wx * nz, wx * ny, wx * ny};
+    int best = 63;
+    int64_t best_cost = -1;
+    for (int mask = 0; mask < 64; mask++) {
+        bool covers = true;
+        int64_t w = 0;
+        for (int f = 1; f < 64 && covers; f++) covers = !seen[f] || (f & mask);
+        for (int b = 0; b < 6; b++) w += (mask >> b & 1) ? cost[b] : 0;
+        if (covers && (best_cost < 0 || w < best_cost)) {
+            best = mask;
+            best_cost = w;
+        }
+    }
+    return best;
+}
+
 }  // namespace mplb

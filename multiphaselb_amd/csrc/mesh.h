@@ -37,4 +37,10 @@ std::string read_lattice(Mesh& m, const std::string& dir);
 // nodes: coordinate u in [-1, n] maps to u in [0, n-1] with period n-1.
 inline int wrap_dup(int u, int n) { return u < 0 ? u + (n - 1) : (u > n - 1 ? u - (n - 1) : u); }
 
+// Faces of a structured box (bits x0 x1 y0 y1 z0 z1) that kernels read through the
+// neighbour table: together they hold every surface node whose links are not the
+// duplicate-node periodic wrap or that bc (one flag per node) marks as carrying a boundary
+// condition.
+int odd_faces(const Mesh& m, const std::vector<uint8_t>& bc);
+
 }  // namespace mplb
