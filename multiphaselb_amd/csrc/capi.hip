@@ -16,6 +16,7 @@
 #include "fused.h"
 #include "glibc_rand.h"
 #include "passes.h"
+#include "transfer.h"
 
 using namespace mplb;
 
@@ -861,6 +862,11 @@ int copy_field(mplb_case* c, const std::string& name, double* host, size_t n, bo
     if (field_layout(c, name, &d, &comps)) return fail(c, MPLB_E_ARG, "Unknown field " + name);
     const int64_t N = c->mesh.N;
     if (n != (size_t)(N * comps)) return fail(c, MPLB_E_ARG, "Field " + name + ": wrong element count");
+    if (stage_wanted(N, comps)) {
+        const int rc = stage_transfer(c, d, N, comps, host, to_device);
+        if (!rc && to_device && (name == "rho" || name == "T")) c->psi_valid = false;
+        return rc;
+    }
     std::vector<T> buf((size_t)N * comps);
     if (to_device) {
         for (int64_t i = 0; i < N; i++)
@@ -943,6 +949,7 @@ int mplb_case_close(mplb_case* c) {
     // teardown: failures here have nobody left to report to
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     if (c->fused) fused_destroy(c);
+    stage_free(c);
     void* ptrs[] = {c->f[0], c->f[1], c->f_alt[0], c->f_alt[1], c->rho, c->temp, c->p, c->U, c->Fi, c->Ft, c->ss, c->psi,
                     c->nb, c->onbnd, c->rnd, c->red, c->nanc, c->rho_snap, c->order[0], c->order[1], c->sumg};
     for (void* p : ptrs)

@@ -40,6 +40,10 @@ struct Timer {
 
 }  // namespace mplb
 
+namespace mplb {
+struct HostStage;
+}
+
 struct mplb_case {
     mplb_opts opts{};
     std::string dir;
@@ -88,6 +92,8 @@ struct mplb_case {
     // fused structured-box path
     bool fused = false;
     void* fz = nullptr;                         // fused-state handle (kernels_fused.hip)
+
+    mplb::HostStage* stage = nullptr;           // pinned buffers of large field transfers
 
     // timers
     bool timing = false;

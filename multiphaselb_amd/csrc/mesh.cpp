@@ -302,20 +302,26 @@ int odd_faces(const Mesh& m, const std::vector<uint8_t>& bc) {
     const int nx = m.nx, ny = m.ny, nz = m.nz;
     const int64_t nxy = (int64_t)nx * ny;
     bool seen[64] = {false};               // face sets of the nodes that need the table
-    for (int64_t id = 0; id < m.N; id++) {
-        const int i = (int)(id % nx), j = (int)((id / nx) % ny), k = (int)(id / nxy);
+    auto visit = [&](int i, int j, int k) {
         int faces = (i == 0 ? 1 : 0) | (i == nx - 1 ? 2 : 0) | (j == 0 ? 4 : 0) | (j == ny - 1 ? 8 : 0);
         if (m.d == 3) faces |= (k == 0 ? 16 : 0) | (k == nz - 1 ? 32 : 0);
-        if (!faces || seen[faces]) continue;
+        if (!faces || seen[faces]) return;
+        const int64_t id = i + (int64_t)j * nx + k * nxy;
         bool differs = bc[id] != 0;
         for (int q = 0; q < m.Q && !differs; q++) {
             const int* cq = m.lbmodel == 0 ? kC2[q] : kC3[q];
             const int64_t want = wrap_dup(i - cq[0], nx) + (int64_t)wrap_dup(j - cq[1], ny) * nx +
                                  (m.d == 3 ? (int64_t)wrap_dup(k - cq[2], nz) * nxy : 0);
-            if (m.nb[id * m.Q + q] != want) differs = true;
+            differs = m.nb[id * m.Q + q] != want;
         }
         if (differs) seen[faces] = true;
-    }
+    };
+    for (int k = 0; k < nz; k++)
+        for (int j = 0; j < ny; j++) {
+            const bool whole = j == 0 || j == ny - 1 || (m.d == 3 && (k == 0 || k == nz - 1));
+            const int step = whole || nx == 1 ? 1 : nx - 1;
+            for (int i = 0; i < nx; i += step) visit(i, j, k);
+        }
     // wavefronts that a face puts on the table path
     const int64_t rows = (int64_t)ny * nz, wx = (nx + 63) / 64;
     const int64_t cost[6] = {rows, rows, wx * nz, wx * nz, wx * ny, wx * ny};
