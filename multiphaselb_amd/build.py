@@ -34,11 +34,13 @@ HIP_DEV = ["--offload-arch=" + ARCH, "-Xclang", "-target-feature", "-Xclang", "-
 UNITS = [
     ("kernels_generic.hip", ["-O3", "-ffp-contract=off"] + HIP_DEV),
     ("kernels_passes.hip", ["-O3", "-ffp-contract=off"] + HIP_DEV),
+    ("kernels_tiles.hip", ["-O3", "-ffp-contract=off"] + HIP_DEV),
     ("kernels_fused.hip", ["-O3", "-ffp-contract=fast"] + HIP_DEV),
     ("kernels_batch.hip", ["-O3", "-ffp-contract=off"] + HIP_DEV),
     ("mlp.hip", ["-O3", "-ffp-contract=off"] + HIP_DEV),
     ("warm.hip", ["-O3", "-ffp-contract=off"] + HIP_DEV),
     ("fieldio.hip", ["-O2", "-ffp-contract=off"] + HIP_DEV),
+    ("tiles.hip", ["-O2", "-ffp-contract=off"] + HIP_DEV),
     ("transfer.hip", ["-O2", "-ffp-contract=off"] + HIP_DEV),
     ("capi.hip", ["-O2", "-ffp-contract=off"] + HIP_DEV),
     ("dict.cpp", ["-O2", "-ffp-contract=off"]),

@@ -16,6 +16,7 @@
 #include "fused.h"
 #include "glibc_rand.h"
 #include "passes.h"
+#include "tiles.h"
 #include "transfer.h"
 
 using namespace mplb;
@@ -456,7 +457,7 @@ int setup_passes(mplb_case* c) {
     }
     if (c->fc[1].present && c->update[1]) HIPCHK(c, hipMalloc(&c->sumg, c->scalar_bytes * m.N));
     c->passes = true;
-    return 0;
+    return tiles_create(c);
 }
 
 template <typename T>
@@ -724,12 +725,18 @@ int one_step_t(mplb_case* c) {
     return 0;
 }
 
-// m steps of multiPhasePP.c:157-241 in fused passes (kernels_passes.hip), from and to the
-// per-routine state; level0 is the time level before the first of them
+// m steps of multiPhasePP.c:157-241 in fused passes (kernels_passes.hip) or, on small
+// lattices, tiles (kernels_tiles.hip), from and to the per-routine state; level0 is the time level before the first of them
 template <typename T>
 void run_passes_t(mplb_case* c, int m, int level0) {
     const Mesh& ms = c->mesh;
     const bool thermal = c->fc[1].present && c->update[1];
+    if (c->tiles) {
+        ensure_psi<T>(c);
+        TimedRegion tr(c, TM_COLLIDE);
+        tiles_run<T>(c, m, level0);
+        return;
+    }
     collision_t<T>(c, 0);
     collision_t<T>(c, 1);
     PassArgs<T> a{};
@@ -950,6 +957,7 @@ int mplb_case_close(mplb_case* c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     if (c->fused) fused_destroy(c);
     stage_free(c);
+    tiles_destroy(c);
     void* ptrs[] = {c->f[0], c->f[1], c->f_alt[0], c->f_alt[1], c->rho, c->temp, c->p, c->U, c->Fi, c->Ft, c->ss, c->psi,
                     c->nb, c->onbnd, c->rnd, c->red, c->nanc, c->rho_snap, c->order[0], c->order[1], c->sumg};
     for (void* p : ptrs)

@@ -42,6 +42,7 @@ struct Timer {
 
 namespace mplb {
 struct HostStage;
+struct Tiles;
 }
 
 struct mplb_case {
@@ -88,6 +89,11 @@ struct mplb_case {
     int pass_faces = 0;                         // faces read through the neighbour table
     uint8_t* order[2] = {nullptr, nullptr};     // per field: each node's boundary list (255: none)
     void* sumg = nullptr;
+
+    // several steps per launch on small lattices (tiles.hip): rho, T, U, Fi, Ft, ss and psi
+    // of the level being written
+    mplb::Tiles* tiles = nullptr;
+    void* alt[7] = {nullptr};
 
     // fused structured-box path
     bool fused = false;
