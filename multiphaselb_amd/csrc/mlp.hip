@@ -18,6 +18,7 @@
 // counter, so one captured graph is replayed for every iteration.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -55,6 +56,14 @@ struct Gemm {
 };
 
 __device__ inline __bf16 bf(float x) { return (__bf16)x; }
+
+// The two-launch path keeps every matrix operand in the order its lanes load it: 16 rows x
+// 32 K values are 1 KB in one piece, 16 bytes per lane.  (Rows of K values one after the
+// other made each load touch sixteen half cache lines; a workgroup streams all the weights
+// through one CU, which is bound by the lines it can have in flight.)
+__host__ __device__ inline size_t frag(int row, int k, int K) {
+    return ((size_t)(row / 16) * (K / kKStep) + k / kKStep) * 512 + ((k % kKStep) / 8 * 16 + row % 16) * 8 + k % 8;
+}
 
 // Wave w of the workgroup computes the 32 x 32 block (m0, n0) as 2 x 2 MFMA tiles of
 // 16 x 16; lane l supplies row l % 16 of each A tile and row l % 16 of each Bt tile,
@@ -228,6 +237,7 @@ struct RefreshAll {
     int din[kRefreshLayers], dinp[kRefreshLayers], dout[kRefreshLayers];
     __bf16* Wb[kRefreshLayers];
     __bf16* Wbt[kRefreshLayers];
+    int pieces;                        // operands in the two-launch path's order (frag)
 };
 
 __global__ void k_refresh_all(RefreshAll a) {
@@ -238,12 +248,399 @@ __global__ void k_refresh_all(RefreshAll a) {
     const int i = (int)(g - a.start[l]), dout = a.dout[l], dinp = a.dinp[l];
     const int r = i / dout, c = i - r * dout;
     const __bf16 v = bf(r < a.din[l] ? a.W[l][(size_t)r * dout + c] : 0.f);
-    a.Wb[l][(size_t)r * dout + c] = v;
-    a.Wbt[l][(size_t)c * dinp + r] = v;
+    a.Wb[l][a.pieces ? frag(r, c, dout) : (size_t)r * dout + c] = v;
+    a.Wbt[l][a.pieces ? frag(c, r, dinp) : (size_t)c * dinp + r] = v;
 }
 
 __global__ void k_advance(int* counter) {
     if (threadIdx.x == 0 && blockIdx.x == 0) *counter += 1;
+}
+
+// ---------------------------------------------------------------------------
+// The network in two launches.  Every row of a batch goes through the layers on its own,
+// so one workgroup takes 16 rows through the whole forward pass, the loss and the backward
+// pass to the first layer (k_rows), activations and dL/dz staying in LDS; what couples the
+// rows, the weight and bias gradients, follows in one launch over all layers with Adam and
+// the refresh of the BF16 weight copies in its epilogue (k_weights).
+//
+// Bound: latency.  The products of a whole iteration (0.26 GFLOP at batch 256) are a
+// fraction of a microsecond of the chip's matrix rate, but a row workgroup streams all the
+// weights (0.6 MB of BF16) through one CU, layer after layer.  One launch per product, loss
+// term, bias and update cost 21 launches of about 5 us, 131 us per iteration of the
+// 9-256-256-256-128 network at batch 256; k_rows and k_weights take 19.1 and 7.1 us.  Each product
+// accumulates its K values in ascending steps of 32 in one MFMA chain whatever the tile, so
+// results equal the one-launch-per-product kernels' bit for bit.
+constexpr int kNetLayers = 8;
+constexpr int kRows = 16;              // rows of a workgroup of k_rows
+constexpr int kRowThreads = 1024;      // 16 waves: one 16-column tile each of a 256-wide layer
+constexpr int kHelpers = 8;            // helper workgroups per XCD (backward pass)
+constexpr int kRowPad = 8;             // BF16 elements of padding per LDS row
+
+struct Net {
+    int L, B, rows;                    // rows: rows of X that exist (gather without idx)
+    int w[kNetLayers + 1], wp[kNetLayers + 1];
+    int wmax;                          // widest padded level
+    const __bf16* Wb[kNetLayers];      // rows: inputs (frag)
+    const __bf16* Wbt[kNetLayers];     // rows: outputs (frag)
+    const float* bias[kNetLayers];
+    const float* X;
+    const float* T;
+    const int* idx;
+    int* counter;                      // [0] iteration of the next k_rows, [1] of the last one
+    float* y;                          // forward only
+    float* rowsum;
+    __bf16* abt[kNetLayers];           // BF16 activations of levels 0..L-1, rows: channels (frag)
+    __bf16* dzt[kNetLayers + 1];       // BF16 dL/dz of levels 1..L, rows: channels (frag)
+    float* dz32[kNetLayers + 1];       // [B][w]
+    // KEEP: the row-major copies mplb_mlp_tensor hands out
+    __bf16* ab[kNetLayers];
+    float* a32[kNetLayers + 1];
+    __bf16* dzb[kNetLayers + 1];
+};
+
+// LDS of k_rows in bytes: two operand buffers and, with the backward pass, the FP32
+// activations of the hidden levels and the output
+size_t rows_lds(int L, const int* w, const int* wp, bool bwd) {
+    int wmax = 0, hidden = 0;
+    for (int l = 0; l <= L; l++) wmax = wp[l] > wmax ? wp[l] : wmax;
+    for (int l = 1; l < L; l++) hidden += w[l];
+    return sizeof(__bf16) * 2 * kRows * (wmax + kRowPad) + sizeof(float) * kRows * (bwd ? hidden + w[L] + 1 : 0);
+}
+
+// K steps [k0, K) of one 16 x 16 tile, K in ascending steps of 32: a, this lane's row of a
+// row-major operand, or (FRAG) its place in the tile's pieces; bt, its place in the other
+// operand's pieces
+template <bool FRAG>
+__device__ inline f32x4 row_tile(const __bf16* a, const __bf16* bt, int k0, int K, f32x4 acc) {
+#pragma unroll 8
+    for (int k = k0; k < K; k += kKStep)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)(a + (FRAG ? k / kKStep * 512 : k)),
+                                                      *(const bf16x8*)(bt + k / kKStep * 512), acc, 0, 0, 0);
+    return acc;
+}
+
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+
+// The workgroup meets with its LDS writes done; global loads and stores stay in flight
+// (nothing of them is read by another wave).  A fence would wait for the transposed stores
+// of the layer and for the next layer's weights.
+__device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// BWD: with loss and backward pass; KEEP: also the row-major intermediates.  A wave's first
+// tile of a layer takes its weights from registers, loaded while the layer before it was
+// finished (they do not depend on the rows).  At batch 256: 33.7 us with the weights loaded
+// when a layer began, a fence per layer and the targets read at the loss, 30.7 us with all
+// three ahead, 20.5 us with the operands in load order (frag), 19.1 us with the helper
+// workgroups.
+template <bool BWD, bool KEEP>
+__global__ void __launch_bounds__(kRowThreads) k_rows(Net g) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    if (BWD && (int)blockIdx.x >= g.B / kRows) {
+        // helper workgroup: touches its slice of every layer's weights, in the order of use, so
+        // that they are in this XCD's L2 when its row workgroups come to them (the update that
+        // wrote them ran on all XCDs)
+        const int part = ((int)blockIdx.x - g.B / kRows) / 8;
+        unsigned seen = 0;
+        for (int i = 0; i < 2 * g.L - 1; i++) {
+            const int l = i < g.L ? i : 2 * g.L - 1 - i;
+            const uint4* p = (const uint4*)(i < g.L ? g.Wbt[l] : g.Wb[l]);
+            const int n = g.wp[l] * g.w[l + 1] / 8;
+            for (int e = part * kRowThreads + threadIdx.x; e < n; e += kHelpers * kRowThreads) seen |= p[e].x;
+        }
+        asm volatile("" ::"v"(seen));
+        return;
+    }
+    const int ld = g.wmax + kRowPad;
+    __bf16* buf = (__bf16*)lds;                          // [2][kRows][ld]
+    float* act = (float*)(buf + 2 * kRows * ld);         // hidden levels, [kRows][w] each, then [kRows][w_L + 1]
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int r = lane & 15, kq = (lane >> 4) * 8, m0 = (lane >> 4) * 4;
+    const int b0 = blockIdx.x * kRows, B = g.B;
+    constexpr int kWaves = kRowThreads / 64, kHeld = 8, kTargets = 4;
+    bf16x8 held[kHeld];
+    float held_bias = 0.f;
+    // weights (and bias) of this wave's first tile of a layer
+    auto fetch = [&](const __bf16* bt, const float* bias, int N, int K) __attribute__((always_inline)) {
+        if (wave >= N / 16) return;
+        const __bf16* p = bt + (size_t)wave * 16 * K + lane * 8;
+#pragma unroll
+        for (int i = 0; i < kHeld; i++)
+            if (i * kKStep < K) held[i] = *(const bf16x8*)(p + i * 512);
+        if (bias) held_bias = bias[wave * 16 + r];
+    };
+    auto first_tile = [&](const __bf16* a, const __bf16* bt, int K) __attribute__((always_inline)) {
+        f32x4 acc{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < kHeld; i++)
+            if (i * kKStep < K)
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)(a + i * kKStep), held[i], acc, 0, 0, 0);
+        return row_tile<false>(a, bt, kHeld * kKStep, K, acc);
+    };
+    fetch(g.Wbt[0], g.bias[0], g.w[1], g.wp[0]);
+    const int* idx = g.idx ? g.idx + (size_t)g.counter[0] * B : nullptr;
+    auto row_of = [&](int m) { return idx ? idx[b0 + m] : b0 + m; };
+    const int nout = g.w[g.L];
+    for (int e = threadIdx.x; e < kRows * kInPad; e += kRowThreads) {
+        const int m = e / kInPad, c = e % kInPad, row = row_of(m);
+        const float x = c < g.w[0] && row < g.rows ? g.X[(size_t)row * g.w[0] + c] : 0.f;
+        buf[m * ld + c] = bf(x);
+        if (BWD) g.abt[0][frag(c, b0 + m, B)] = bf(x);
+        if (KEEP) g.ab[0][(size_t)(b0 + m) * kInPad + c] = bf(x);
+    }
+    float target[kTargets];
+    if constexpr (BWD) {
+#pragma unroll
+        for (int j = 0; j < kTargets; j++) {
+            const int e = threadIdx.x + j * kRowThreads;
+            if (e < kRows * nout) target[j] = g.T[(size_t)row_of(e / nout) * nout + e % nout];
+        }
+    }
+    lds_barrier();
+    int cur = 0;
+    float* level = act;                                  // FP32 activations of level l + 1
+    for (int l = 0; l < g.L; l++) {
+        const int N = g.w[l + 1], K = g.wp[l];
+        const bool last = l == g.L - 1;
+        const int stride = last ? N + 1 : N;             // (the output's rows are read by one lane each)
+        const __bf16* a = buf + (cur * kRows + r) * ld + kq;
+        __bf16* to = buf + (1 - cur) * kRows * ld;
+        for (int nt = wave; nt < N / 16; nt += kWaves) {
+            const int n = nt * 16 + r;
+            const __bf16* bt = g.Wbt[l] + (size_t)nt * 16 * K + lane * 8;
+            f32x4 acc{0.f, 0.f, 0.f, 0.f};
+            float bias;
+            if (nt == wave) {
+                acc = first_tile(a, bt, K);
+                bias = held_bias;
+                if (!last) fetch(g.Wbt[l + 1], g.bias[l + 1], g.w[l + 2], g.wp[l + 1]);
+                else if (BWD && l > 0) fetch(g.Wb[l], nullptr, g.wp[l], g.w[l + 1]);
+            } else {
+                acc = row_tile<false>(a, bt, 0, K, acc);
+                bias = g.bias[l][n];
+            }
+            bf16x4 t;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int m = m0 + e;
+                float v = acc[e] + bias;
+                if (!last) {
+                    v = tanhf(v);
+                    t[e] = bf(v);
+                    to[m * ld + n] = t[e];
+                    if (KEEP) g.ab[l + 1][(size_t)(b0 + m) * N + n] = t[e];
+                    if (KEEP) g.a32[l + 1][(size_t)(b0 + m) * N + n] = v;
+                } else if (!BWD || KEEP) {
+                    if (b0 + m < B) g.y[(size_t)(b0 + m) * N + n] = v;
+                }
+                if (BWD) level[m * stride + n] = v;
+            }
+            if (BWD && !last) *(bf16x4*)(g.abt[l + 1] + frag(n, b0 + m0, B)) = t;
+        }
+        // a wave without a tile in this layer may have one in the next
+        if (wave >= N / 16) {
+            if (!last) fetch(g.Wbt[l + 1], g.bias[l + 1], g.w[l + 2], g.wp[l + 1]);
+            else if (BWD && l > 0) fetch(g.Wb[l], nullptr, g.wp[l], g.w[l + 1]);
+        }
+        cur = 1 - cur;
+        if (BWD && !last) level += kRows * N;
+        lds_barrier();
+    }
+    if constexpr (BWD) {
+        // dL/dy of L = sum (y - t)^2 / (B n); level holds y, then the differences
+        const int n = nout;
+        const float scale = 2.0f / ((float)B * (float)n);
+        __bf16* to = buf + cur * kRows * ld;
+        auto loss_at = [&](int e, float t) __attribute__((always_inline)) {
+            const int m = e / n, c = e - m * n;
+            const float d = level[m * (n + 1) + c] - t;
+            const float dz = scale * d;
+            level[m * (n + 1) + c] = d;
+            to[m * ld + c] = bf(dz);
+            g.dz32[g.L][(size_t)(b0 + m) * n + c] = dz;
+            if (KEEP) g.dzb[g.L][(size_t)(b0 + m) * n + c] = bf(dz);
+        };
+#pragma unroll
+        for (int j = 0; j < kTargets; j++) {
+            const int e = threadIdx.x + j * kRowThreads;
+            if (e < kRows * n) loss_at(e, target[j]);
+        }
+        for (int e = threadIdx.x + kTargets * kRowThreads; e < kRows * n; e += kRowThreads)
+            loss_at(e, g.T[(size_t)row_of(e / n) * n + e % n]);
+        lds_barrier();
+        for (int e = threadIdx.x; e < kRows * n; e += kRowThreads) {
+            const int c = e / kRows, m = e % kRows;
+            g.dzt[g.L][frag(c, b0 + m, B)] = to[m * ld + c];
+        }
+        // row sums of squared errors: 256 partial sums over every 256th column, added in
+        // order, by one lane per row of the last wave (which for a 256-wide layer has a tile of
+        // its own to finish, so the sums come after the backward pass)
+        const float* diff = level;
+        for (int l = g.L - 1; l > 0; l--) {
+            const int N = g.wp[l], K = g.w[l + 1];
+            level -= kRows * N;
+            const __bf16* a = buf + (cur * kRows + r) * ld + kq;
+            __bf16* out = buf + (1 - cur) * kRows * ld;
+            for (int nt = wave; nt < N / 16; nt += kWaves) {
+                const int c = nt * 16 + r;
+                const __bf16* bt = g.Wb[l] + (size_t)nt * 16 * K + lane * 8;
+                f32x4 acc{0.f, 0.f, 0.f, 0.f};
+                if (nt == wave) {
+                    acc = first_tile(a, bt, K);
+                    if (l > 1) fetch(g.Wb[l - 1], nullptr, g.wp[l - 1], g.w[l]);
+                } else {
+                    acc = row_tile<false>(a, bt, 0, K, acc);
+                }
+                bf16x4 t;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int m = m0 + e;
+                    const float x = level[m * N + c];
+                    const float dz = acc[e] * (1.0f - x * x);
+                    t[e] = bf(dz);
+                    out[m * ld + c] = t[e];
+                    g.dz32[l][(size_t)(b0 + m) * N + c] = dz;
+                    if (KEEP) g.dzb[l][(size_t)(b0 + m) * N + c] = t[e];
+                }
+                *(bf16x4*)(g.dzt[l] + frag(c, b0 + m0, B)) = t;
+            }
+            if (wave >= N / 16 && l > 1) fetch(g.Wb[l - 1], nullptr, g.wp[l - 1], g.w[l]);
+            cur = 1 - cur;
+            lds_barrier();
+        }
+        if (wave == 0 && lane < kRows) {
+            const float* d = diff + lane * (n + 1);
+            float sum = 0.f;
+            if (n <= 256) {
+#pragma unroll 16
+                for (int i = 0; i < n; i++) sum += d[i] * d[i];
+            } else {
+                for (int i = 0; i < 256; i++) {
+                    float s = 0.f;
+                    for (int c = i; c < n; c += 256) s += d[c] * d[c];
+                    sum += s;
+                }
+            }
+            g.rowsum[b0 + lane] = sum;
+        }
+        if (blockIdx.x == 0 && threadIdx.x == 0 && g.idx) g.counter[1] += 1;
+    }
+}
+
+// one Adam update of parameter i with gradient gi (bias correction at step t)
+struct Adam {
+    float *p, *m, *v;
+    float lr, b1, b2, eps;
+};
+__device__ inline float adam_update(const Adam& a, int64_t i, float gi, float t) {
+    const float mi = a.b1 * a.m[i] + (1.f - a.b1) * gi;
+    const float vi = a.b2 * a.v[i] + (1.f - a.b2) * gi * gi;
+    a.m[i] = mi;
+    a.v[i] = vi;
+    const float mh = mi / (1.f - powf(a.b1, t));
+    const float vh = vi / (1.f - powf(a.b2, t));
+    const float p = a.p[i] - a.lr * mh / (sqrtf(vh) + a.eps);
+    a.p[i] = p;
+    return p;
+}
+
+// Weight and bias gradients of every layer: blocks [0, 1) the loss, then per layer 64-column
+// bias blocks, then 32 x 32 weight tiles (four waves of one 16 x 16 tile each).
+struct Grads {
+    int L, B;
+    int w[kNetLayers + 1], wp[kNetLayers + 1];
+    int bias0[kNetLayers + 1], tile0[kNetLayers + 1];    // first block of a layer's biases / tiles
+    const __bf16* abt[kNetLayers];
+    const __bf16* dzt[kNetLayers + 1];
+    const float* dz32[kNetLayers + 1];
+    __bf16* Wb[kNetLayers];
+    __bf16* Wbt[kNetLayers];
+    int64_t woff[kNetLayers], boff[kNetLayers];
+    float* grad;                       // written when not training
+    const float* rowsum;
+    int* counter;
+    float* hist;
+    float* loss;
+    Adam adam;
+};
+
+template <bool TRAIN>
+__global__ void __launch_bounds__(256) k_weights(Grads g) {
+    const int blk = blockIdx.x, B = g.B;
+    const int it = TRAIN ? g.counter[1] : 0;
+    const float t = (float)(it + 1);
+    if (blk == 0) {
+        __shared__ float rs[1024];
+        double s = 0;
+        for (int b1 = 0; b1 < B; b1 += 1024) {
+            const int n = B - b1 < 1024 ? B - b1 : 1024;
+            for (int i = threadIdx.x; i < n; i += 256) rs[i] = g.rowsum[b1 + i];
+            __syncthreads();
+            if (threadIdx.x == 0) {
+#pragma unroll 8
+                for (int i = 0; i < n; i++) s += rs[i];
+            }
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) {
+            const float L = (float)(s / ((double)B * (double)g.w[g.L]));
+            *g.loss = L;
+            if (g.hist) g.hist[it] = L;
+            if (TRAIN) g.counter[0] += 1;
+        }
+        return;
+    }
+    if (blk < g.tile0[0]) {
+        int l = 0;
+        while (blk >= g.bias0[l + 1]) l++;
+        // as k_bias_grad
+        __shared__ float part[4][64];
+        const float* dz = g.dz32[l + 1];
+        const int n = g.w[l + 1], cl = threadIdx.x & 63, k = threadIdx.x >> 6;
+        const int c = (blk - g.bias0[l]) * 64 + cl;
+        float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
+        if (c < n) {
+            int b = k;
+#pragma unroll 4
+            for (; b + 12 < B; b += 16) {
+                s0 += dz[(size_t)b * n + c];
+                s1 += dz[(size_t)(b + 4) * n + c];
+                s2 += dz[(size_t)(b + 8) * n + c];
+                s3 += dz[(size_t)(b + 12) * n + c];
+            }
+            for (; b < B; b += 4) s0 += dz[(size_t)b * n + c];
+        }
+        part[k][cl] = (s0 + s1) + (s2 + s3);
+        __syncthreads();
+        if (k == 0 && c < n) {
+            const float db = ((part[0][cl] + part[1][cl]) + part[2][cl]) + part[3][cl];
+            if (TRAIN) adam_update(g.adam, g.boff[l] + c, db, t);
+            else g.grad[g.boff[l] + c] = db;
+        }
+        return;
+    }
+    int l = 0;
+    while (blk >= g.tile0[l + 1]) l++;
+    const int dout = g.w[l + 1], dinp = g.wp[l], din = g.w[l];
+    const int nt = dout / 32, tile = blk - g.tile0[l];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15;
+    const int mt0 = tile / nt * 32 + (wave >> 1) * 16, n = tile % nt * 32 + (wave & 1) * 16 + r;
+    const f32x4 acc = row_tile<true>(g.abt[l] + (size_t)mt0 * B + lane * 8, g.dzt[l + 1] + (size_t)(n - r) * B + lane * 8,
+                                     0, B, f32x4{0.f, 0.f, 0.f, 0.f});
+    const int m0 = mt0 + (lane >> 4) * 4;
+    bf16x4 wt;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const int m = m0 + e;
+        if (TRAIN) {
+            float p = 0.f;
+            if (m < din) p = adam_update(g.adam, g.woff[l] + (int64_t)m * dout + n, acc[e], t);
+            wt[e] = bf(p);
+            g.Wb[l][frag(m, n, dout)] = wt[e];
+        } else if (m < din) {
+            g.grad[g.woff[l] + (int64_t)m * dout + n] = acc[e];
+        }
+    }
+    if (TRAIN) *(bf16x4*)(g.Wbt[l] + frag(n, m0, dinp)) = wt;
 }
 
 __global__ void k_set_int(int* p, int v) {
@@ -272,7 +669,10 @@ struct mplb_mlp {
     std::vector<__bf16*> dzb, dzt;
     float* rowsum = nullptr;
     float* loss = nullptr;
-    int* counter = nullptr;
+    int* counter = nullptr;                     // [2]
+    size_t lds_fwd = 0, lds_bwd = 0;            // LDS of k_rows; 0: one launch per product
+    float* Y = nullptr;                         // outputs of a forward call
+    size_t Y_cap = 0;
     std::vector<void*> owned;
     // training data resident on the device
     float *X = nullptr, *T = nullptr;
@@ -321,6 +721,7 @@ void refresh(mplb_mlp* n) {
     if (n->L <= kRefreshLayers) {
         RefreshAll a{};
         a.L = n->L;
+        a.pieces = n->lds_bwd != 0;
         for (int l = 0; l < n->L; l++) {
             a.start[l + 1] = a.start[l] + (int64_t)n->wp[l] * n->w[l + 1];
             a.W[l] = n->p + n->woff[l];
@@ -410,6 +811,73 @@ void backward(mplb_mlp* n) {
     }
 }
 
+// The two-launch path takes networks whose row workgroup fits its LDS; wider or deeper ones
+// keep one launch per product.
+constexpr size_t kRowsLds = 150 * 1024;
+
+Net net_args(mplb_mlp* n) {
+    Net g{};
+    g.L = n->L;
+    g.B = n->B;
+    g.rows = n->B;
+    for (int l = 0; l <= n->L; l++) {
+        g.w[l] = n->w[l];
+        g.wp[l] = n->wp[l];
+        g.wmax = std::max(g.wmax, n->wp[l]);
+        g.dzt[l] = n->dzt[l];
+        g.dz32[l] = n->dz32[l];
+        g.dzb[l] = n->dzb[l];
+        g.a32[l] = n->a32[l];
+    }
+    for (int l = 0; l < n->L; l++) {
+        g.Wb[l] = n->Wb[l];
+        g.Wbt[l] = n->Wbt[l];
+        g.bias[l] = n->p + n->boff[l];
+        g.abt[l] = n->abt[l];
+        g.ab[l] = n->ab[l];
+    }
+    g.X = n->X;
+    g.T = n->T;
+    g.counter = n->counter;
+    g.y = n->y;
+    g.rowsum = n->rowsum;
+    return g;
+}
+
+Grads grad_args(mplb_mlp* n, int* blocks) {
+    Grads g{};
+    g.L = n->L;
+    g.B = n->B;
+    for (int l = 0; l <= n->L; l++) {
+        g.w[l] = n->w[l];
+        g.wp[l] = n->wp[l];
+        g.dzt[l] = n->dzt[l];
+        g.dz32[l] = n->dz32[l];
+    }
+    int at = 1;
+    for (int l = 0; l < n->L; l++) {
+        g.abt[l] = n->abt[l];
+        g.Wb[l] = n->Wb[l];
+        g.Wbt[l] = n->Wbt[l];
+        g.woff[l] = n->woff[l];
+        g.boff[l] = n->boff[l];
+        g.bias0[l] = at;
+        at += (n->w[l + 1] + 63) / 64;
+    }
+    g.bias0[n->L] = at;
+    for (int l = 0; l < n->L; l++) {
+        g.tile0[l] = at;
+        at += n->wp[l] / 32 * (n->w[l + 1] / 32);
+    }
+    g.tile0[n->L] = at;
+    g.grad = n->g;
+    g.rowsum = n->rowsum;
+    g.counter = n->counter;
+    g.loss = n->loss;
+    *blocks = at;
+    return g;
+}
+
 }  // namespace
 
 extern "C" {
@@ -469,15 +937,27 @@ int mplb_mlp_create(int nlayers, const int* widths, int batch, int device, mplb_
     rc |= alloc(n, &n->tgt, (size_t)batch * n->w[nlayers]);
     rc |= alloc(n, &n->rowsum, (size_t)batch);
     rc |= alloc(n, &n->loss, 1);
-    rc |= alloc(n, &n->counter, 1);
-    return rc ? MPLB_E_HIP : 0;
+    rc |= alloc(n, &n->counter, 2);
+    if (rc) return MPLB_E_HIP;
+    const size_t lds = rows_lds(nlayers, n->w.data(), n->wp.data(), true);
+    if (nlayers <= kNetLayers && lds <= kRowsLds) {
+        n->lds_bwd = lds;
+        n->lds_fwd = rows_lds(nlayers, n->w.data(), n->wp.data(), false);
+        MCHK(n, hipFuncSetAttribute((const void*)k_rows<false, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)kRowsLds));
+        MCHK(n, hipFuncSetAttribute((const void*)k_rows<true, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)kRowsLds));
+        MCHK(n, hipFuncSetAttribute((const void*)k_rows<true, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)kRowsLds));
+    }
+    return 0;
 }
 
 int mplb_mlp_close(mplb_mlp* n) {
     if (!n) return MPLB_E_ARG;
     if (n->stream) (void)hipStreamSynchronize(n->stream);
     for (void* q : n->owned) (void)hipFree(q);
-    void* extra[] = {n->X, n->T, n->idx, n->hist};
+    void* extra[] = {n->X, n->T, n->idx, n->hist, n->Y};
     for (void* q : extra)
         if (q) (void)hipFree(q);
     if (n->stream) (void)hipStreamDestroy(n->stream);
@@ -517,6 +997,26 @@ int mplb_mlp_forward(mplb_mlp* n, const float* x, int rows, float* y) {
     if (!n || !x || !y || rows < 0) return MPLB_E_ARG;
     MCHK(n, hipSetDevice(n->dev));
     const int din = n->w[0], dout = n->w[n->L], B = n->B;
+    if (n->lds_bwd) {
+        constexpr int kChunk = 65536;          // rows on the device at a time
+        const size_t most = (size_t)std::min(rows, kChunk);
+        int rc = ensure(n, &n->X, &n->X_cap, most * din);
+        if (!rc) rc = ensure(n, &n->Y, &n->Y_cap, most * dout);
+        if (rc) return rc;
+        Net g = net_args(n);
+        g.y = n->Y;
+        for (int r0 = 0; r0 < rows; r0 += kChunk) {
+            g.B = g.rows = std::min(kChunk, rows - r0);
+            MCHK(n, hipMemcpyAsync(n->X, x + (size_t)r0 * din, sizeof(float) * g.rows * din, hipMemcpyHostToDevice,
+                                   n->stream));
+            k_rows<false, false><<<(unsigned)((g.rows + kRows - 1) / kRows), kRowThreads, n->lds_fwd, n->stream>>>(g);
+            MCHK(n, hipGetLastError());
+            MCHK(n, hipMemcpyAsync(y + (size_t)r0 * dout, n->Y, sizeof(float) * g.rows * dout, hipMemcpyDeviceToHost,
+                                   n->stream));
+            MCHK(n, hipStreamSynchronize(n->stream));
+        }
+        return 0;
+    }
     int rc = ensure(n, &n->X, &n->X_cap, (size_t)B * din);
     if (rc) return rc;
     std::vector<float> xb((size_t)B * din), yb((size_t)B * dout);
@@ -546,12 +1046,19 @@ int mplb_mlp_gradient(mplb_mlp* n, const float* x, const float* t, float* loss, 
     if (rc) return rc;
     MCHK(n, hipMemcpyAsync(n->X, x, sizeof(float) * B * din, hipMemcpyHostToDevice, n->stream));
     MCHK(n, hipMemcpyAsync(n->T, t, sizeof(float) * B * dout, hipMemcpyHostToDevice, n->stream));
-    k_gather<<<B, 64, 0, n->stream>>>(n->X, n->T, nullptr, nullptr, B, din, dout, n->ab[0], n->abt[0], n->tgt);
-    float* keep = n->hist;
-    n->hist = nullptr;
-    forward(n);
-    backward(n);
-    n->hist = keep;
+    if (n->lds_bwd) {
+        int blocks = 0;
+        const Grads g = grad_args(n, &blocks);
+        k_rows<true, true><<<(unsigned)(B / kRows + 8 * kHelpers), kRowThreads, n->lds_bwd, n->stream>>>(net_args(n));
+        k_weights<false><<<(unsigned)blocks, 256, 0, n->stream>>>(g);
+    } else {
+        k_gather<<<B, 64, 0, n->stream>>>(n->X, n->T, nullptr, nullptr, B, din, dout, n->ab[0], n->abt[0], n->tgt);
+        float* keep = n->hist;
+        n->hist = nullptr;
+        forward(n);
+        backward(n);
+        n->hist = keep;
+    }
     MCHK(n, hipGetLastError());
     if (loss) MCHK(n, hipMemcpyAsync(loss, n->loss, sizeof(float), hipMemcpyDeviceToHost, n->stream));
     if (grad) MCHK(n, hipMemcpyAsync(grad, n->g, sizeof(float) * ngrad, hipMemcpyDeviceToHost, n->stream));
@@ -577,19 +1084,32 @@ int mplb_mlp_train(mplb_mlp* n, const float* X, const float* T, int nsamples, co
     // every call is a fresh Adam run: the iteration counter (index table, loss history,
     // bias-correction step count) restarts and the first and second moments are zeroed
     hipLaunchKernelGGL(k_set_int, 1, 1, 0, n->stream, n->counter, 0);
+    hipLaunchKernelGGL(k_set_int, 1, 1, 0, n->stream, n->counter + 1, -1);
     MCHK(n, hipMemsetAsync(n->m, 0, sizeof(float) * n->P, n->stream));
     MCHK(n, hipMemsetAsync(n->v, 0, sizeof(float) * n->P, n->stream));
     MCHK(n, hipStreamSynchronize(n->stream));
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     MCHK(n, hipStreamBeginCapture(n->stream, hipStreamCaptureModeThreadLocal));
-    k_gather<<<B, 64, 0, n->stream>>>(n->X, n->T, n->idx, n->counter, B, din, dout, n->ab[0], n->abt[0], n->tgt);
-    forward(n);
-    backward(n);
-    k_adam<<<(unsigned)((n->P + 255) / 256), 256, 0, n->stream>>>(n->p, n->g, n->m, n->v, n->P, lr, beta1, beta2, eps,
-                                                                   n->counter);
-    refresh(n);
-    k_advance<<<1, 64, 0, n->stream>>>(n->counter);
+    if (n->lds_bwd) {
+        int blocks = 0;
+        Grads gr = grad_args(n, &blocks);
+        gr.hist = n->hist;
+        gr.adam = Adam{n->p, n->m, n->v, lr, beta1, beta2, eps};
+        Net g = net_args(n);
+        g.idx = n->idx;
+        g.rows = nsamples;
+        k_rows<true, false><<<(unsigned)(B / kRows + 8 * kHelpers), kRowThreads, n->lds_bwd, n->stream>>>(g);
+        k_weights<true><<<(unsigned)blocks, 256, 0, n->stream>>>(gr);
+    } else {
+        k_gather<<<B, 64, 0, n->stream>>>(n->X, n->T, n->idx, n->counter, B, din, dout, n->ab[0], n->abt[0], n->tgt);
+        forward(n);
+        backward(n);
+        k_adam<<<(unsigned)((n->P + 255) / 256), 256, 0, n->stream>>>(n->p, n->g, n->m, n->v, n->P, lr, beta1, beta2,
+                                                                       eps, n->counter);
+        refresh(n);
+        k_advance<<<1, 64, 0, n->stream>>>(n->counter);
+    }
     MCHK(n, hipStreamEndCapture(n->stream, &graph));
     MCHK(n, hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
     for (int it = 0; it < iters; it++) MCHK(n, hipGraphLaunch(exec, n->stream));
@@ -639,8 +1159,10 @@ int mplb_mlp_tensor(mplb_mlp* n, const char* name, int j, float* out, size_t cou
     if (is_bf) {
         std::vector<uint16_t> h(count);
         MCHK(n, hipMemcpy(h.data(), src, 2 * count, hipMemcpyDeviceToHost));
+        const int cols = !std::strcmp(name, "wb") ? n->w[j + 1] : 0;
         for (size_t i = 0; i < count; i++) {
-            const uint32_t u = (uint32_t)h[i] << 16;
+            const size_t at = n->lds_bwd && cols ? frag((int)(i / cols), (int)(i % cols), cols) : i;
+            const uint32_t u = (uint32_t)h[at] << 16;
             std::memcpy(&out[i], &u, 4);
         }
     } else {
