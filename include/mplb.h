@@ -213,7 +213,7 @@ int64_t mplb_batch_case_steps(const mplb_batch* b, int i);
  * chosen_block is the two-pass block size (also used by the measurement passes).
  * mplb_batch_set_launch selects the two-pass kernels by hand, mplb_batch_set_march the
  * single-pass kernel (rows per item; 0 = two-pass); both kernels give identical results.
- * New batches use the single-pass kernel with 32 rows when every case fits. */
+ * New batches use the single-pass kernel with 8 rows when every case fits. */
 int mplb_batch_tune(mplb_batch* b, int steps_per_trial, int* chosen_block, int* chosen_xcd_order);
 int mplb_batch_set_launch(mplb_batch* b, int block, int xcd_order);
 int mplb_batch_set_march(mplb_batch* b, int rows);

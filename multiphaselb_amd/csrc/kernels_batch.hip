@@ -48,13 +48,22 @@ struct BCase {
     int state;            // 0 active, 1 converged, 2 diverged (NaN)
 };
 
+// Model constants in the arithmetic type, converted on the host: a conversion in the kernel
+// leaves a value that is the same for every lane in a vector register for the whole march.
+template <typename T>
+struct BPar {
+    T lam[9];
+    T sigma, G, g[2], fext[2];
+    T R, M, a, b;
+};
+
 struct BArgs {
+    BPar<double> pd;
+    BPar<float> pf;
     const BCase* cases;
     const int2* work;     // (case, first local node) per workgroup; case -1 = padding
     int64_t P;            // plane pitch (total padded nodes)
     EosParams eos;
-    double lam[9];
-    double sigma;
     const void* fin;      // populations (storage type)
     void* fout;
     void* psi;            // compute type
@@ -65,6 +74,12 @@ struct BArgs {
     const _Float16* rin;
     _Float16* rout;
 };
+
+template <typename T>
+__device__ inline const BPar<T>& par(const BArgs& a) {
+    if constexpr (sizeof(T) == 8) return a.pd;
+    else return a.pf;
+}
 
 // Work item of the single-pass kernel: rows [y0, y1) of up to four cases of the same
 // nx x ny (workgroup lane t serves case slot t / nx, column t % nx); ncase 0 = padding.
@@ -207,16 +222,16 @@ __device__ inline T bdiv(T x, T y) {
 }
 
 template <typename T>
-__device__ inline T bpotential(const EosParams& e, T rho, T temp) {
+__device__ inline T bpotential(const BArgs& a, T rho, T temp) {
     if constexpr (sizeof(T) == 4) {
-        if (e.type == EOS_VDW) {
-            const float M = (float)e.M;
-            const float p = rho * (float)e.R * temp * __builtin_amdgcn_rcpf(M - rho * (float)e.b) -
-                            (float)e.a * __builtin_amdgcn_rcpf(M * M) * rho * rho;
-            return __builtin_amdgcn_sqrtf(2.f * (p - rho * (float)kCs2) * __builtin_amdgcn_rcpf((float)e.G));
+        if (a.eos.type == EOS_VDW) {
+            const BPar<float>& e = a.pf;
+            const float p = rho * e.R * temp * __builtin_amdgcn_rcpf(e.M - rho * e.b) -
+                            e.a * __builtin_amdgcn_rcpf(e.M * e.M) * rho * rho;
+            return __builtin_amdgcn_sqrtf(2.f * (p - rho * (float)kCs2) * __builtin_amdgcn_rcpf(e.G));
         }
     }
-    return potential<T>(e, rho, temp);
+    return potential<T>(a.eos, rho, temp);
 }
 
 template <typename T>
@@ -257,18 +272,17 @@ __global__ void k_batch_psi(BArgs a) {
     if (!p.valid) return;
     T v[9];
     const T rho = load_state<S, T, MODE>(a, bc, p, v);
-    ((T*)a.psi)[p.gid] = bpotential<T>(a.eos, rho, T(bc.T));
+    ((T*)a.psi)[p.gid] = bpotential<T>(a, rho, T(bc.T));
 }
 
 // Interaction force (interForce.c:16-39, interactionForce.c:47-79; every node of a fully
 // periodic box is interior), velocity (liMRTVelocity.c:11-50) and the liMRT collision
 // (liMRTCollision.c:33-106 with liMRTForce.c:13-42), written to the other buffer.  The
 // expressions keep the per-routine FP64 kernels' association order.
-// One node: v holds its pulled populations (density rho), psic its psi and psin[q] the
-// psi of x + c_q; the post-collision populations go to node gid of the other buffer.
-template <typename S, typename T, int MODE>
-__device__ inline void collide_site(const BArgs& a, const BCase& bc, T* v, const T rho, const T psic, const T* psin,
-                                    int64_t gid) {
+// One node: v holds its pulled populations (density rho) on entry and the post-collision
+// ones on exit, psic its psi and psin[q] the psi of x + c_q.
+template <typename T, int MODE>
+__device__ inline void collide_site(const BArgs& a, T* v, const T rho, const T psic, const T* psin) {
     T F[2] = {T(0.0), T(0.0)};
     constexpr Pairs<D2Q9> PR = make_pairs<D2Q9>();
     if constexpr (sizeof(T) == 8) {
@@ -295,11 +309,12 @@ __device__ inline void collide_site(const BArgs& a, const BCase& bc, T* v, const
             }
         }
     }
-    const T beta = -T(a.eos.G) * psic;
+    const BPar<T>& c = par<T>(a);
+    const T beta = -c.G * psic;
     const T Fi[2] = {F[0] * beta, F[1] * beta};
     T Ft[2];
 #pragma unroll
-    for (int d = 0; d < 2; d++) Ft[d] = Fi[d] + (rho - T(0)) * T(a.eos.g[d]) + T(a.eos.fext[d]);
+    for (int d = 0; d < 2; d++) Ft[d] = Fi[d] + (rho - T(0)) * c.g[d] + c.fext[d];
     T U[2] = {T(0), T(0)};
     if (MODE == FROM_PULL) {
 #pragma unroll
@@ -336,8 +351,8 @@ __device__ inline void collide_site(const BArgs& a, const BCase& bc, T* v, const
     meq[8] = rho * U[0] * U[1];
     if constexpr (sizeof(T) == 8) moments<D2Q9, T>(v, m);
     else moments_sym<D2Q9, T>(v, m);
-    const T sigma = T(a.sigma);
-    const T L1 = T(a.lam[1]), L2 = T(a.lam[2]);
+    const T sigma = c.sigma;
+    const T L1 = c.lam[1], L2 = c.lam[2];
     const T uF = U[0] * Ft[0] + U[1] * Ft[1];
     const T fi2 = Fi[0] * Fi[0] + Fi[1] * Fi[1];
     Sf[0] = 0;
@@ -353,7 +368,7 @@ __device__ inline void collide_site(const BArgs& a, const BCase& bc, T* v, const
         // the oracle's order: post-collision moments, then populations rebuilt from them
 #pragma unroll
         for (int q = 0; q < 9; q++) {
-            const T l = T(a.lam[q]);
+            const T l = c.lam[q];
             m[q] = m[q] - l * (m[q] - meq[q]) + (T(1) - T(0.5) * l) * Sf[q];
         }
         populations<D2Q9, T>(m, v);
@@ -361,15 +376,11 @@ __device__ inline void collide_site(const BArgs& a, const BCase& bc, T* v, const
         // the moment change added to the pulled populations (no per-step rebuild)
 #pragma unroll
         for (int q = 0; q < 9; q++) {
-            const T l = T(a.lam[q]);
+            const T l = c.lam[q];
             m[q] = (T(1) - T(0.5) * l) * Sf[q] - l * (m[q] - meq[q]);
         }
         populations_add_sym<D2Q9, T>(m, v);
     }
-    T rinv;
-    const T R = put_ref<S, T>(a, gid, rho, rinv);
-#pragma unroll
-    for (int q = 0; q < 9; q++) stf<S, T>(bc, a.fout, q * a.P + gid, q, v[q], R, rinv);
 }
 
 template <typename S, typename T, int MODE>
@@ -383,7 +394,11 @@ __global__ void k_batch_collide(BArgs a) {
     T psin[9];
 #pragma unroll
     for (int q = 1; q < 9; q++) psin[q] = psi[p.off + p.X[1 + D2Q9::t.c[q][0]] + p.Y[1 + D2Q9::t.c[q][1]]];
-    collide_site<S, T, MODE>(a, bc, v, rho, psi[p.gid], psin, p.gid);
+    collide_site<T, MODE>(a, v, rho, psi[p.gid], psin);
+    T rinv;
+    const T R = put_ref<S, T>(a, p.gid, rho, rinv);
+#pragma unroll
+    for (int q = 0; q < 9; q++) stf<S, T>(bc, a.fout, q * a.P + p.gid, q, v[q], R, rinv);
 }
 
 __device__ inline int wrap_dup(int u, int n) { return u < 0 ? u + (n - 1) : (u > n - 1 ? u - (n - 1) : u); }
@@ -396,14 +411,31 @@ __device__ inline int wrap_dup(int u, int n) { return u < 0 ? u + (n - 1) : (u >
 // psi never goes to memory.  Per node and step the populations are read once and written
 // once.  LDS hazards: row y + 1 goes to slot (y + 2 - y0) & 3, which no lane reads while
 // colliding row y - 1 or y, and one barrier per row publishes it.
+// Bound: memory (256 cases of 64 to 256 nodes in FP32: 1.10 x the 72 B per node and step at
+// 3.9 TB/s, VALU issue 45% busy).  Six waves per SIMD in FP32 and FP16 (79 VGPRs), four in
+// FP64 (127): with the model constants converted in the kernel they held 20 vector registers
+// and, with 64-bit addresses, the FP32 kernel ran four, 197 us per step at 32 rows per item
+// against 152.  Issuing row y + 2's pulls before row y collides (108 VGPRs) was slower, 171
+// against 160 us at 8 rows, and plain stores instead of non-temporal ones 158 against 150.
 // wave priority while a row's populations are pulled (as in the 3D single pass: loads
 // go out ahead of other waves' collisions; 0.9% faster in FP64, neutral in FP32)
 #ifndef MPLB_BATCH_PRIO
 #define MPLB_BATCH_PRIO 2
 #endif
-template <typename S, typename T>
+// Population q of a node, addressed by the node's byte offset in its plane: the plane's
+// address is the same for the whole workgroup and stays in scalar registers, so a load is
+// one 32-bit add.  WIDE keeps 64-bit offsets for batches whose planes reach 4 GiB.
+template <bool WIDE>
+using off_t_ = typename std::conditional<WIDE, uint64_t, uint32_t>::type;
+
+// LDS writes done and the workgroup met; loads and stores of populations stay in flight (no
+// wave reads what another one stores within a step)
+__device__ inline void ring_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+template <typename S, typename T, bool WIDE>
 __device__ inline void march_item(const BArgs& a, const MItem& it, T (*ring)[kMarchLanes]) {
     if (it.ncase == 0) return;
+    using off = off_t_<WIDE>;
     const int t = threadIdx.x;
     const int nx = it.nx;
     const int slot = t / nx, x = t - slot * nx;
@@ -413,9 +445,10 @@ __device__ inline void march_item(const BArgs& a, const MItem& it, T (*ring)[kMa
     const int ny = act ? bc.ny : 3;
     const int sb = slot * nx;
     const unsigned X[3] = {(unsigned)(x == 0 ? nx - 2 : x - 1), (unsigned)x, (unsigned)(x == nx - 1 ? 1 : x + 1)};
+    const off base = (off)bc.off;
     T fc[9], fn[9];
     // populations and psi of raw row yr (y0 - 1 <= yr <= y1)
-    auto row = [&](int yr) {
+    auto row = [&](int yr) __attribute__((always_inline)) {
         if (!act) return;
         if (MPLB_BATCH_PRIO) __builtin_amdgcn_s_setprio(MPLB_BATCH_PRIO);
         const int yw = wrap_dup(yr, ny);
@@ -423,10 +456,11 @@ __device__ inline void march_item(const BArgs& a, const MItem& it, T (*ring)[kMa
                                (unsigned)((yw == ny - 1 ? 1 : yw + 1) * nx)};
 #pragma unroll
         for (int q = 0; q < 9; q++) {
-            const int64_t node = bc.off + X[1 - D2Q9::t.c[q][0]] + Y[1 - D2Q9::t.c[q][1]];
-            fn[q] = ldf<S, T>(a.fin, q * a.P + node, wref_of<S, T>(a, bc, node, q));
+            const off node = base + (X[1 - D2Q9::t.c[q][0]] + Y[1 - D2Q9::t.c[q][1]]);
+            const char* plane = (const char*)a.fin + (int64_t)q * a.P * sizeof(S);
+            fn[q] = ldf<S, T>(plane + node * (off)sizeof(S), 0, wref_of<S, T>(a, bc, node, q));
         }
-        ring[(yr - it.y0 + 1) & 3][t] = bpotential<T>(a.eos, density<T>(fn), T(bc.T));
+        ring[(yr - it.y0 + 1) & 3][t] = bpotential<T>(a, density<T>(fn), T(bc.T));
         if (MPLB_BATCH_PRIO) __builtin_amdgcn_s_setprio(0);
     };
     row(it.y0 - 1);
@@ -435,26 +469,34 @@ __device__ inline void march_item(const BArgs& a, const MItem& it, T (*ring)[kMa
     for (int q = 0; q < 9; q++) fc[q] = fn[q];
     for (int y = it.y0; y < it.y1; y++) {
         row(y + 1);
-        __syncthreads();
+        ring_barrier();
         if (act) {
             T psin[9];
 #pragma unroll
             for (int q = 1; q < 9; q++)
                 psin[q] = ring[(y + D2Q9::t.c[q][1] - it.y0 + 1) & 3][sb + X[1 + D2Q9::t.c[q][0]]];
-            collide_site<S, T, FROM_PULL>(a, bc, fc, density<T>(fc), ring[(y - it.y0 + 1) & 3][t], psin,
-                                          bc.off + (int64_t)y * nx + x);
+            const T rho = density<T>(fc);
+            collide_site<T, FROM_PULL>(a, fc, rho, ring[(y - it.y0 + 1) & 3][t], psin);
+            const off node = base + (off)((unsigned)y * (unsigned)nx + (unsigned)x);
+            T rinv;
+            const T R = put_ref<S, T>(a, (int64_t)node, rho, rinv);
+#pragma unroll
+            for (int q = 0; q < 9; q++) {
+                char* plane = (char*)a.fout + (int64_t)q * a.P * sizeof(S);
+                stf<S, T>(bc, plane + node * (off)sizeof(S), 0, q, fc[q], R, rinv);
+            }
         }
 #pragma unroll
         for (int q = 0; q < 9; q++) fc[q] = fn[q];
     }
 }
 
-template <typename S, typename T>
+template <typename S, typename T, bool WIDE>
 __global__ void __launch_bounds__(kMarchLanes) k_batch_march(BArgs a, const MItem* items, int per, int nitems) {
     __shared__ T ring[4][kMarchLanes];
     const int wi = (int)((blockIdx.x & 7u) * (unsigned)per + (blockIdx.x >> 3));
     if (wi >= nitems) return;
-    march_item<S, T>(a, items[wi], ring);
+    march_item<S, T, WIDE>(a, items[wi], ring);
 }
 
 // The same steps from one persistent launch (cooperative, so every workgroup is resident
@@ -477,7 +519,7 @@ __global__ void __launch_bounds__(kMarchLanes) k_batch_persist(BArgs a, const MI
         a.rout = (s & 1) ? r0 : r1;
         for (unsigned v = blockIdx.x; v < total; v += gridDim.x) {
             const int wi = (int)((v & 7u) * (unsigned)per + (v >> 3));
-            if (wi < nitems) march_item<S, T>(a, items[wi], ring);
+            if (wi < nitems) march_item<S, T, true>(a, items[wi], ring);
             __syncthreads();      // the next item's rows reuse the LDS ring
         }
         if (s + 1 < nsteps) grid.sync();
@@ -522,7 +564,7 @@ __global__ void k_batch_pressure(BArgs a) {
     const Pos p = pos(a, bc);
     if (!p.valid) return;
     const T* psi = (const T*)a.psi;
-    const T G = T(a.eos.G);
+    const T G = par<T>(a).G;
     const T ps = psi[p.gid];
     T pr = ((const T*)a.rho)[p.gid] * T(kCs2) + T(0.5) * G * ps * ps;
     const T xa = psi[p.off + p.X[2] + p.Y[1]], xb = psi[p.off + p.X[0] + p.Y[1]];
@@ -534,7 +576,7 @@ __global__ void k_batch_pressure(BArgs a) {
     T g2 = 0;
 #pragma unroll
     for (int k = 0; k < 3; k++) g2 += grad[k] * grad[k];
-    pr = pr + T(2.0) * G * G * T(a.sigma) * g2;
+    pr = pr + T(2.0) * G * G * par<T>(a).sigma * g2;
     ((T*)a.p)[p.gid] = pr;
 }
 
@@ -548,7 +590,7 @@ __global__ void k_batch_rho_psi(BArgs a) {
     pull<S, T>(a, bc, p, a.fin, v);
     const T rho = density<T>(v);
     ((T*)a.rho)[p.gid] = rho;
-    ((T*)a.psi)[p.gid] = bpotential<T>(a.eos, rho, T(bc.T));
+    ((T*)a.psi)[p.gid] = bpotential<T>(a, rho, T(bc.T));
 }
 
 __global__ void k_fill_u32(unsigned* p, int n, unsigned v) {
@@ -590,7 +632,11 @@ struct mplb_batch {
     int nmwork = 0;                     // launch grid of k_batch_march (8 x mper)
     int mper = 0;
     bool march_ok = true;               // every case is at most kMarchLanes wide
-    int mrows = 32;                     // rows per march item; 0: the two-pass kernels
+    // rows per march item; 0: the two-pass kernels.  Eight by default: items enough for several
+    // rounds of workgroups, whose uneven ends then cost little, against two more rows pulled
+    // per item, which are L2 hits.  256 cases of 64 to 256 nodes, us per step at 8 / 16 / 32 / 64
+    // rows: FP32 150 / 154 / 152 / 214, FP64 274 / 286 / 317 / 298, FP16N 136 / 139 / 141 / 192
+    int mrows = 8;
     bool persist = false;               // single pass: one persistent launch per run of steps
     bool initialized = false;
     bool fields_valid = false;
@@ -621,8 +667,22 @@ BArgs bargs(mplb_batch* b) {
     a.work = b->d_work;
     a.P = b->P;
     a.eos = b->eos;
-    for (int q = 0; q < 9; q++) a.lam[q] = b->lam[q];
-    a.sigma = b->sigma;
+    auto fill = [&](auto& p) {
+        using V = std::remove_reference_t<decltype(p.sigma)>;
+        for (int q = 0; q < 9; q++) p.lam[q] = (V)b->lam[q];
+        p.sigma = (V)b->sigma;
+        p.G = (V)b->eos.G;
+        for (int d = 0; d < 2; d++) {
+            p.g[d] = (V)b->eos.g[d];
+            p.fext[d] = (V)b->eos.fext[d];
+        }
+        p.R = (V)b->eos.R;
+        p.M = (V)b->eos.M;
+        p.a = (V)b->eos.a;
+        p.b = (V)b->eos.b;
+    };
+    fill(a.pd);
+    fill(a.pf);
     a.psi = b->psi;
     a.rho = b->rho;
     a.p = b->p;
@@ -732,8 +792,13 @@ void launch_steps(mplb_batch* b, int nsteps) {
         a.rout = b->rb;
         if (b->mrows > 0) {
             if (b->nmwork > 0)
-                k_batch_march<S, T><<<(unsigned)b->nmwork, kMarchLanes, 0, b->stream>>>(a, b->d_mwork, b->mper,
-                                                                                      b->nmwork);
+            {
+                const dim3 g((unsigned)b->nmwork);
+                if ((uint64_t)b->P * sizeof(S) < (uint64_t(1) << 32))
+                    k_batch_march<S, T, false><<<g, kMarchLanes, 0, b->stream>>>(a, b->d_mwork, b->mper, b->nmwork);
+                else
+                    k_batch_march<S, T, true><<<g, kMarchLanes, 0, b->stream>>>(a, b->d_mwork, b->mper, b->nmwork);
+            }
         } else if (b->nwork > 0) {
             k_batch_psi<S, T, FROM_PULL><<<grid, block, 0, b->stream>>>(a);
             k_batch_collide<S, T, FROM_PULL><<<grid, block, 0, b->stream>>>(a);
