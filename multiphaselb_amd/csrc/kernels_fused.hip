@@ -44,6 +44,7 @@ struct FArgs {
     int face_table;                             // faces (x0 x1 y0 y1 z0 z1 bits) read through the table
     const int* nb;                              // [Q][N]
     const uint8_t* onbnd;
+    int lists_f, lists_g;                       // nodes carry boundary codes
     const uint8_t* bcf;                         // per-node boundary code, f (surface nodes)
     const uint8_t* bcg;                         // low 4 bits: code; fixedRandomT: list slot in the high 4
     const float* bcTw;                          // per-node wall temperature (g)
@@ -203,19 +204,22 @@ __device__ inline float fpot(const FArgs& a, float rho, float T) {
     return potential<float>(a.eos, rho, T);
 }
 
+// upstream nodes of a node's populations
+template <class L>
+__device__ inline void upstreams(const FArgs& a, const NodePos& p, unsigned* up) {
+#pragma unroll
+    for (int q = 0; q < L::Q; q++) up[q] = upstream<L>(a, p, q);
+}
+
 // REF: f stored against per-node references (FP16N); otherwise shift holds the storage
 // shifts
 template <class L, typename S, bool REF>
-__device__ inline void pull(const FArgs& a, const NodePos& p, const void* src, const float* shift, float* v) {
+__device__ inline void pull(const FArgs& a, const unsigned* up, const void* src, const float* shift, float* v) {
 #pragma unroll
     for (int q = 0; q < L::Q; q++) {
         const void* plane = (const char*)src + (size_t)q * a.P * sizeof(S);
-        if constexpr (REF && kNodeRef<S>) {
-            const unsigned up = upstream<L>(a, p, q);
-            v[q] = ldf<S>(plane, up, f_wref<L, S>(a, up, q));
-        } else {
-            v[q] = ld<S>(plane, upstream<L>(a, p, q), shift[q]);
-        }
+        if constexpr (REF && kNodeRef<S>) v[q] = ldf<S>(plane, up[q], f_wref<L, S>(a, up[q], q));
+        else v[q] = ld<S>(plane, up[q], shift[q]);
     }
 }
 
@@ -269,20 +273,48 @@ __device__ inline void fixed_temperature(const FArgs& a, const NodePos& p, float
     }
 }
 
-template <class L, typename S>
-__device__ inline void pull_f(const FArgs& a, const NodePos& p, float* v) {
-    pull<L, S, kNodeRef<S>>(a, p, a.fin, a.fshift, v);
-    if (p.table && a.bcf[p.id] == FB_BBACK) bounce_back<L>(a, p, v);
+// The boundary condition of a pulled node
+template <class L>
+__device__ inline void bound_f(const FArgs& a, const NodePos& p, float* v) {
+    if (a.lists_f && p.table && a.bcf[p.id] == FB_BBACK) bounce_back<L>(a, p, v);
 }
 
 template <class L, typename S>
-__device__ inline void pull_g(const FArgs& a, const NodePos& p, float* v) {
-    pull<L, S, false>(a, p, a.gin, a.gshift, v);
-    if (!p.table) return;
+__device__ inline void bound_g(const FArgs& a, const NodePos& p, float* v) {
+    if (!a.lists_g || !p.table) return;
     const uint8_t bc = a.bcg[p.id];
     const uint8_t code = bc & 0xF;
     if (code == FB_BBACK) bounce_back<L>(a, p, v);
     else if (code == FB_FT || code == FB_FRDT) fixed_temperature<L, S>(a, p, v, code, ((a.draw >> (bc >> 4)) & 1) != 0);
+}
+
+template <class L, typename S>
+__device__ inline void pull_f(const FArgs& a, const NodePos& p, float* v) {
+    unsigned up[L::Q];
+    upstreams<L>(a, p, up);
+    pull<L, S, kNodeRef<S>>(a, up, a.fin, a.fshift, v);
+    bound_f<L>(a, p, v);
+}
+
+template <class L, typename S>
+__device__ inline void pull_g(const FArgs& a, const NodePos& p, float* v) {
+    unsigned up[L::Q];
+    upstreams<L>(a, p, up);
+    pull<L, S, false>(a, up, a.gin, a.gshift, v);
+    bound_g<L, S>(a, p, v);
+}
+
+// Both fields, every load issued before a boundary condition branches: pulled one after the
+// other, the second field's loads wait for the first one's (a chain of latencies on the
+// nodes that read the neighbour table).
+template <class L, typename S>
+__device__ inline void pull_fg(const FArgs& a, const NodePos& p, float* v, float* w) {
+    unsigned up[L::Q];
+    upstreams<L>(a, p, up);
+    pull<L, S, kNodeRef<S>>(a, up, a.fin, a.fshift, v);
+    pull<L, S, false>(a, up, a.gin, a.gshift, w);
+    bound_f<L>(a, p, v);
+    bound_g<L, S>(a, p, w);
 }
 
 // K1
@@ -291,14 +323,14 @@ __global__ void __launch_bounds__(256) k_fused_density(FArgs a) {
     const NodePos p = node_pos<L>(a);
     if (!p.valid) return;
     float v[L::Q];
-    pull_f<L, S>(a, p, v);
-    const float rho = rho_sym<L, float>(v);
-    if (THERMAL) {
-        pull_g<L, S>(a, p, v);
-        const float sg = rho_sym<L, float>(v);
-        a.rho[p.id] = rho;
-        a.sumg[p.id] = sg;
+    if constexpr (THERMAL) {
+        float w[L::Q];
+        pull_fg<L, S>(a, p, v, w);
+        a.rho[p.id] = rho_sym<L, float>(v);
+        a.sumg[p.id] = rho_sym<L, float>(w);
     } else {
+        pull_f<L, S>(a, p, v);
+        const float rho = rho_sym<L, float>(v);
         const float T = a.Tuniform ? a.Tconst : a.Told[p.id];
         a.psi[p.id] = fpot(a, rho, T);
         if (a.out_rho) a.out_rho[p.id] = rho;
@@ -602,8 +634,9 @@ __global__ void __launch_bounds__(256) k_fused_collide(FArgs a) {
     const NodePos p = node_pos<L>(a);
     if (!p.valid) return;
     const int64_t id = p.id, N = a.N;
-    float v[L::Q];
-    pull_f<L, S>(a, p, v);
+    float v[L::Q], w[THERMAL ? L::Q : 1];
+    if constexpr (THERMAL) pull_fg<L, S>(a, p, v, w);
+    else pull_f<L, S>(a, p, v);
     const float rho = rho_sym<L, float>(v);
     const float psic = a.psi[id];
     const bool interior = !p.table || a.onbnd[id] == 0;
@@ -634,11 +667,10 @@ __global__ void __launch_bounds__(256) k_fused_collide(FArgs a) {
         for (int q = 0; q < L::Q; q++) st<S>(a.fout, q * a.P + id, v[q], a.fshift[q]);
     }
 
-    if (THERMAL) {
-        pull_g<L, S>(a, p, v);
-        collide_g<L>(a, v, a.Tnew[id], a.S[id], U);
+    if constexpr (THERMAL) {
+        collide_g<L>(a, w, a.Tnew[id], a.S[id], U);
 #pragma unroll
-        for (int q = 0; q < L::Q; q++) st<S>(a.gout, q * a.P + id, v[q], a.gshift[q]);
+        for (int q = 0; q < L::Q; q++) st<S>(a.gout, q * a.P + id, w[q], a.gshift[q]);
         a.Unew[id] = U[0];
         a.Unew[N + id] = U[1];
         a.Unew[2 * N + id] = U[2];
@@ -1542,6 +1574,7 @@ struct Fused {
     float* T[2] = {nullptr, nullptr};
     float* U[2] = {nullptr, nullptr};
     int cur = 0;                   // T[cur], U[cur] hold the current time level
+    int lists[2] = {0, 0};         // boundary codes are set in f / g
     uint8_t* bcf = nullptr;
     uint8_t* bcg = nullptr;
     float* bcTw = nullptr;
@@ -1604,6 +1637,8 @@ FArgs make_args(mplb_case* c) {
     a.face_table = z->face_table;
     a.nb = c->nb;
     a.onbnd = c->onbnd;
+    a.lists_f = z->lists[0];
+    a.lists_g = z->lists[1];
     a.bcf = z->bcf;
     a.bcg = z->bcg;
     a.bcTw = z->bcTw;
@@ -2031,6 +2066,7 @@ int fused_create(mplb_case* c) {
             const int t = fc.bctype[b];
             uint8_t code = t == BD_BBACK ? FB_BBACK : t == BD_FT ? FB_FT : t == BD_FRDT ? FB_FRDT : FB_NONE;
             if (code == FB_NONE) continue;
+            z->lists[f] = 1;
             int cnt = 0;
             const uint8_t slot = code == FB_FRDT ? (uint8_t)(z->frdt_lists.size() << 4) : 0;
             for (int32_t id : m.bd[b]) {
