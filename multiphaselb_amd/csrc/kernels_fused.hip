@@ -102,17 +102,14 @@ __device__ inline float ld(const void* p, int64_t i, float shift) {
     }
 }
 
-#ifndef MPLB_NT_STORE
-#define MPLB_NT_STORE 1
-#endif
-
-template <typename S>
+// Population stores: NT = non-temporal (stores_nt has the rule)
+template <typename S, bool NT = true>
 __device__ inline void st(void* p, int64_t i, float v, float shift) {
     if constexpr (sizeof(S) == 2) {
-        if (MPLB_NT_STORE) __builtin_nontemporal_store((_Float16)(v - shift), (_Float16*)p + i);
+        if constexpr (NT) __builtin_nontemporal_store((_Float16)(v - shift), (_Float16*)p + i);
         else ((_Float16*)p)[i] = (_Float16)(v - shift);
     } else {
-        if (MPLB_NT_STORE) __builtin_nontemporal_store(v, (float*)p + i);
+        if constexpr (NT) __builtin_nontemporal_store(v, (float*)p + i);
         else ((float*)p)[i] = v;
     }
 }
@@ -178,11 +175,11 @@ __device__ inline float put_ref(const FArgs& a, int64_t id, float rho, float& ri
 }
 
 // FP16N: stores f population q of a node (reference R and 1 / R = rinv from put_ref)
-template <class L>
+template <class L, bool NT = true>
 __device__ inline void stf_ref(void* p, int64_t i, int q, float v, float R, float rinv) {
     const float wref = (float)L::t.omega[q] * R;
     const float dev = (v - wref) * ((float)(1.0 / L::t.omega[q]) * rinv);
-    if (MPLB_NT_STORE) __builtin_nontemporal_store((_Float16)dev, (_Float16*)p + i);
+    if constexpr (NT) __builtin_nontemporal_store((_Float16)dev, (_Float16*)p + i);
     else ((_Float16*)p)[i] = (_Float16)dev;
 }
 
@@ -629,7 +626,7 @@ __device__ inline void collide_g(const FArgs& a, float* v, float T, float Sv, co
 }
 
 // K2
-template <class L, typename S, bool THERMAL>
+template <class L, typename S, bool THERMAL, bool NT>
 __global__ void __launch_bounds__(256) k_fused_collide(FArgs a) {
     const NodePos p = node_pos<L>(a);
     if (!p.valid) return;
@@ -661,16 +658,16 @@ __global__ void __launch_bounds__(256) k_fused_collide(FArgs a) {
         float rinv;
         const float R = put_ref<S>(a, id, rho, rinv);
 #pragma unroll
-        for (int q = 0; q < L::Q; q++) stf_ref<L>(a.fout, q * a.P + id, q, v[q], R, rinv);
+        for (int q = 0; q < L::Q; q++) stf_ref<L, NT>(a.fout, q * a.P + id, q, v[q], R, rinv);
     } else {
 #pragma unroll
-        for (int q = 0; q < L::Q; q++) st<S>(a.fout, q * a.P + id, v[q], a.fshift[q]);
+        for (int q = 0; q < L::Q; q++) st<S, NT>(a.fout, q * a.P + id, v[q], a.fshift[q]);
     }
 
     if constexpr (THERMAL) {
         collide_g<L>(a, w, a.Tnew[id], a.S[id], U);
 #pragma unroll
-        for (int q = 0; q < L::Q; q++) st<S>(a.gout, q * a.P + id, w[q], a.gshift[q]);
+        for (int q = 0; q < L::Q; q++) st<S, NT>(a.gout, q * a.P + id, w[q], a.gshift[q]);
         a.Unew[id] = U[0];
         a.Unew[N + id] = U[1];
         a.Unew[2 * N + id] = U[2];
@@ -817,7 +814,7 @@ __device__ inline float stored_pull(raw_t<S> v, const unsigned* r, int q, const 
 #define MPLB_PULL_PRIO 2
 #endif
 
-template <class L, typename S, bool OUT>
+template <class L, typename S, bool OUT, bool NT>
 __global__ void __launch_bounds__(256)
     __attribute__((amdgpu_waves_per_eu(sizeof(S) == 2 ? MPLB_MARCH_WAVES_H : MPLB_MARCH_WAVES))) k_fused_march(FArgs a) {
     __shared__ float ring[4][MSLOT];
@@ -910,10 +907,10 @@ __global__ void __launch_bounds__(256)
                 float rinv;
                 const float R = put_ref<S>(a, id, rho, rinv);
 #pragma unroll
-                for (int q = 0; q < L::Q; q++) stf_ref<L>(a.fout, q * a.P + id, q, fc[q], R, rinv);
+                for (int q = 0; q < L::Q; q++) stf_ref<L, NT>(a.fout, q * a.P + id, q, fc[q], R, rinv);
             } else {
 #pragma unroll
-                for (int q = 0; q < L::Q; q++) st<S>(a.fout, q * a.P + id, fc[q], a.fshift[q]);
+                for (int q = 0; q < L::Q; q++) st<S, NT>(a.fout, q * a.P + id, fc[q], a.fshift[q]);
             }
             if (OUT) {
                 const int64_t N = a.N;
@@ -941,7 +938,7 @@ __global__ void __launch_bounds__(256)
 #define MPLB_MARCH_PF_WAVES 2
 #endif
 
-template <class L, typename S, bool OUT>
+template <class L, typename S, bool OUT, bool NT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MPLB_MARCH_PF_WAVES)))
 k_fused_march_pf(FArgs a) {
     static_assert(!kNodeRef<S>, "FP32 or FP16S storage");
@@ -1049,7 +1046,7 @@ k_fused_march_pf(FArgs a) {
         if (owner) {
             const int64_t id = (int64_t)x + (int64_t)y * a.nx + (int64_t)z * a.nxy;
 #pragma unroll
-            for (int q = 0; q < L::Q; q++) st<S>(a.fout, q * a.P + id, fc[q], a.fshift[q]);
+            for (int q = 0; q < L::Q; q++) st<S, NT>(a.fout, q * a.P + id, fc[q], a.fshift[q]);
             if (OUT) {
                 const int64_t N = a.N;
                 a.out_rho[id] = rho;
@@ -1140,7 +1137,7 @@ __device__ inline void tring1(int r, int& px, int& py) {
 
 __device__ inline int tslot(int zr) { return (zr + 3) % 3; }
 
-template <class L, typename S, bool OUT>
+template <class L, typename S, bool OUT, bool NT>
 __global__ void __launch_bounds__(TNT) __attribute__((amdgpu_waves_per_eu(MPLB_TMARCH_WAVES))) k_fused_tmarch(FArgs a) {
     __shared__ float s_rho[3][TNR], s_T[3][TNR], s_U[3][3][TNR];
     __shared__ float s_psi[3][TNP];
@@ -1319,14 +1316,14 @@ __global__ void __launch_bounds__(TNT) __attribute__((amdgpu_waves_per_eu(MPLB_T
                 float rinv;
                 const float R = put_ref<S>(a, id, rho, rinv);
 #pragma unroll
-                for (int q = 0; q < L::Q; q++) stf_ref<L>(a.fout, pidx(a, q, (unsigned)id), q, f0[q], R, rinv);
+                for (int q = 0; q < L::Q; q++) stf_ref<L, NT>(a.fout, pidx(a, q, (unsigned)id), q, f0[q], R, rinv);
             } else {
 #pragma unroll
-                for (int q = 0; q < L::Q; q++) st<S>(a.fout, pidx(a, q, (unsigned)id), f0[q], a.fshift[q]);
+                for (int q = 0; q < L::Q; q++) st<S, NT>(a.fout, pidx(a, q, (unsigned)id), f0[q], a.fshift[q]);
             }
             collide_g<L>(a, g0, T0, s0, U);
 #pragma unroll
-            for (int q = 0; q < L::Q; q++) st<S>(a.gout, pidx(a, q, (unsigned)id), g0[q], a.gshift[q]);
+            for (int q = 0; q < L::Q; q++) st<S, NT>(a.gout, pidx(a, q, (unsigned)id), g0[q], a.gshift[q]);
             a.Tnew[id] = T0;
             a.Unew[id] = U[0];
             a.Unew[N + id] = U[1];
@@ -1386,7 +1383,7 @@ __device__ inline void stage_pull(const FArgs& a, int x, int y, int z, float (*s
     }
 }
 
-template <class L, bool OUT>
+template <class L, bool OUT, bool NT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MPLB_MARCH_LDS_WAVES)))
 k_fused_march_lds(FArgs a) {
     __shared__ float stage0[L::Q][LST], stage1[L::Q][LST];
@@ -1484,7 +1481,7 @@ k_fused_march_lds(FArgs a) {
         if (!owner) return;
         const int64_t id = (int64_t)x + (int64_t)y * a.nx + (int64_t)z * a.nxy;
 #pragma unroll
-        for (int q = 0; q < L::Q; q++) st<float>(a.fout, q * a.P + id, fc[q], 0.f);
+        for (int q = 0; q < L::Q; q++) st<float, NT>(a.fout, q * a.P + id, fc[q], 0.f);
     };
     // Plane zr is staged in stage0 when zr - z0 is odd (z0 - 1, z0 + 1, ...), in stage1
     // when it is even; the loop takes two planes per trip so that both are named
@@ -1598,6 +1595,7 @@ struct Fused {
     bool t_uniform = false;        // the isothermal temperature field is one value (t_const)
     float t_const = 0.f;
     int mtx = 0, mtiles = 0, mitems = 0, mper = 0, mzc = 0;
+    bool nt = true;              // population stores are non-temporal
 };
 
 Fused* F(mplb_case* c) { return (Fused*)c->fz; }
@@ -1695,30 +1693,47 @@ FArgs make_args(mplb_case* c) {
 }
 
 // The single-pass kernel (D3Q15, FP32 or FP16 storage)
-template <class L, typename S, bool OUT>
+template <class L, typename S, bool OUT, bool NT>
 void launch_march(mplb_case* c, const FArgs& a) {
     if constexpr (L::D == 3) {
         const dim3 grid(8u * (unsigned)a.mper);
         if constexpr (std::is_same<S, float>::value) {
             if (F(c)->march_lds) {
-                k_fused_march_lds<L, OUT><<<grid, 256, 0, c->stream>>>(a);
+                k_fused_march_lds<L, OUT, NT><<<grid, 256, 0, c->stream>>>(a);
                 return;
             }
         }
         if constexpr (!kNodeRef<S>) {
             if (F(c)->march_pf) {
-                k_fused_march_pf<L, S, OUT><<<grid, 256, 0, c->stream>>>(a);
+                k_fused_march_pf<L, S, OUT, NT><<<grid, 256, 0, c->stream>>>(a);
                 return;
             }
         }
-        k_fused_march<L, S, OUT><<<grid, 256, 0, c->stream>>>(a);
+        k_fused_march<L, S, OUT, NT><<<grid, 256, 0, c->stream>>>(a);
     }
+}
+
+template <class L, typename S, bool OUT>
+void launch_march(mplb_case* c, const FArgs& a) {
+    if (OUT || F(c)->nt) launch_march<L, S, OUT, true>(c, a);
+    else launch_march<L, S, OUT, OUT>(c, a);
 }
 
 // The thermal single-pass kernel (D3Q15, FP32 or FP16 storage)
 template <class L, typename S, bool OUT>
 void launch_tmarch(mplb_case* c, const FArgs& a) {
-    if constexpr (L::D == 3) k_fused_tmarch<L, S, OUT><<<dim3(8u * (unsigned)a.mper), TNT, 0, c->stream>>>(a);
+    if constexpr (L::D == 3) {
+        const dim3 grid(8u * (unsigned)a.mper);
+        if (OUT || F(c)->nt) k_fused_tmarch<L, S, OUT, true><<<grid, TNT, 0, c->stream>>>(a);
+        else k_fused_tmarch<L, S, OUT, OUT><<<grid, TNT, 0, c->stream>>>(a);
+    }
+}
+
+template <class L, typename S, bool THERMAL>
+void launch_collide(mplb_case* c, const FArgs& a) {
+    const dim3 grid((unsigned)a.nblocks);
+    if (F(c)->nt) k_fused_collide<L, S, THERMAL, true><<<grid, 256, 0, c->stream>>>(a);
+    else k_fused_collide<L, S, THERMAL, false><<<grid, 256, 0, c->stream>>>(a);
 }
 
 template <class L, typename S>
@@ -1735,12 +1750,12 @@ void launch_step(mplb_case* c, FArgs a, bool thermal, bool outputs) {
     } else if (thermal) {
         k_fused_density<L, S, true><<<grid, block, 0, c->stream>>>(a);
         k_fused_heat<L><<<grid, block, 0, c->stream>>>(a);
-        k_fused_collide<L, S, true><<<grid, block, 0, c->stream>>>(a);
+        launch_collide<L, S, true>(c, a);
     } else if (F(c)->march) {
         launch_march<L, S, false>(c, a);
     } else {
         k_fused_density<L, S, false><<<grid, block, 0, c->stream>>>(a);
-        k_fused_collide<L, S, false><<<grid, block, 0, c->stream>>>(a);
+        launch_collide<L, S, false>(c, a);
     }
 }
 
@@ -1788,7 +1803,7 @@ void launch_step_timed(mplb_case* c, FArgs a, bool thermal, bool outputs) {
             k_fused_heat<L><<<grid, block, 0, c->stream>>>(a);
         }
         Ev e(c, 6);
-        k_fused_collide<L, S, true><<<grid, block, 0, c->stream>>>(a);
+        launch_collide<L, S, true>(c, a);
     } else if (F(c)->march) {
         Ev e(c, 6);
         launch_march<L, S, false>(c, a);
@@ -1798,7 +1813,7 @@ void launch_step_timed(mplb_case* c, FArgs a, bool thermal, bool outputs) {
             k_fused_density<L, S, false><<<grid, block, 0, c->stream>>>(a);
         }
         Ev e(c, 6);
-        k_fused_collide<L, S, false><<<grid, block, 0, c->stream>>>(a);
+        launch_collide<L, S, false>(c, a);
     }
 }
 
@@ -1926,12 +1941,12 @@ int materialize(mplb_case* c) {
         // T and U with the values they hold
         launch_tmarch<L, S, true>(c, a);
     } else if (z->thermal) {
-        k_fused_collide<L, S, true><<<grid, block, 0, c->stream>>>(a);
+        launch_collide<L, S, true>(c, a);
     } else if (z->march) {
         // the step's own kernel with outputs: it rewrites fa with the same values
         launch_march<L, S, true>(c, a);
     } else {
-        k_fused_collide<L, S, false><<<grid, block, 0, c->stream>>>(a);
+        launch_collide<L, S, false>(c, a);
     }
     if (z->thermal) {
         const int64_t N = c->mesh.N;
@@ -2024,6 +2039,26 @@ bool fused_supported(const mplb_case* c, std::string* why) {
         }
     }
     return true;
+}
+
+// Non-temporal or ordinary stores of the new populations.  Non-temporal ones are best when
+// every wavefront writes whole 64-byte sectors and the populations do not fit the 256 MiB
+// memory-side cache (256^3 FP32 0.441 against 0.460 ms per step, 192^3 thermal 0.536 against
+// 0.557, 224^3 FP16S, rows of 448 bytes, equal).
+//   - The marches write each row of the box by itself.  Rows that are not a multiple of 64
+//     bytes begin and end inside sectors: non-temporal stores send those partial sectors to
+//     HBM one by one, ordinary ones are joined with the next row's in the L2 (255^3 FP32
+//     0.714 -> 0.623 ms, FP16S 0.528 -> 0.362; 201 x 150 x 180 FP32 0.248 -> 0.219; 240^3
+//     FP16S, rows of 480 bytes, 0.336 -> 0.299).  The other kernels write 256 consecutive
+//     nodes per workgroup, whatever the rows.
+//   - Populations that fit the cache with both copies are read back from it in the next step
+//     (128^3 FP32 69 -> 50 us, 96^3 thermal 85 -> 73, 401 x 333 thermal 19.5 -> 19.0).  The
+//     thermal passes with FP16 storage are the exception (96^3 54 against 56 us, 128^3 115
+//     against 119): they are bound by their arithmetic.
+bool stores_nt(const Mesh& m, const Fused& z, size_t scalar) {
+    if ((z.march || z.tmarch) && m.nx * scalar % 64 != 0) return false;
+    if (z.thermal && z.half) return true;
+    return 2 * (z.thermal ? 2 : 1) * scalar * m.Q * (size_t)z.P > (size_t)256 << 20;
 }
 
 int fused_create(mplb_case* c) {
@@ -2130,23 +2165,23 @@ int fused_create(mplb_case* c) {
             int bpc = 0, cus = 0;
             const int halo = z->tmarch ? 4 : 2;
             if (z->tmarch && z->noderef)
-                FCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_fused_tmarch<D3Q15, h16n, false>, TNT, 0));
+                FCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_fused_tmarch<D3Q15, h16n, false, true>, TNT, 0));
             else if (z->tmarch && z->half)
-                FCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_fused_tmarch<D3Q15, _Float16, false>, TNT, 0));
+                FCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_fused_tmarch<D3Q15, _Float16, false, true>, TNT, 0));
             else if (z->tmarch)
-                FCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_fused_tmarch<D3Q15, float, false>, TNT, 0));
+                FCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_fused_tmarch<D3Q15, float, false, true>, TNT, 0));
             else if (z->march_lds)
-                FCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_fused_march_lds<D3Q15, false>, 256, 0));
+                FCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_fused_march_lds<D3Q15, false, true>, 256, 0));
             else if (z->march_pf && z->half)
-                FCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_fused_march_pf<D3Q15, _Float16, false>, 256, 0));
+                FCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_fused_march_pf<D3Q15, _Float16, false, true>, 256, 0));
             else if (z->march_pf)
-                FCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_fused_march_pf<D3Q15, float, false>, 256, 0));
+                FCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_fused_march_pf<D3Q15, float, false, true>, 256, 0));
             else if (z->noderef)
-                FCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_fused_march<D3Q15, h16n, false>, 256, 0));
+                FCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_fused_march<D3Q15, h16n, false, true>, 256, 0));
             else if (z->half)
-                FCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_fused_march<D3Q15, _Float16, false>, 256, 0));
+                FCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_fused_march<D3Q15, _Float16, false, true>, 256, 0));
             else
-                FCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_fused_march<D3Q15, float, false>, 256, 0));
+                FCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_fused_march<D3Q15, float, false, true>, 256, 0));
             FCHK(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->opts.device));
             const long long resident = std::max(1LL, (long long)bpc * cus);
             int nchunks = 1;
@@ -2170,6 +2205,7 @@ int fused_create(mplb_case* c) {
             z->mper = (z->mitems + 7) / 8;
         }
     }
+    z->nt = stores_nt(m, *z, sb);
     FCHK(c, hipMalloc(&z->bcf, N));
     FCHK(c, hipMemcpy(z->bcf, bcf.data(), N, hipMemcpyHostToDevice));
     FCHK(c, hipMalloc(&z->bcg, N));
