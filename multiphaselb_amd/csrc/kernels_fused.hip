@@ -2157,11 +2157,14 @@ int fused_create(mplb_case* c) {
             const int tmx = z->tmarch ? TMX : MX, tmy = z->tmarch ? TMY : MY;
             z->mtx = (m.nx + tmx - 1) / tmx;
             z->mtiles = z->mtx * ((m.ny + tmy - 1) / tmy);
-            // z chunks (of at least 8 planes) per column: the work items run in rounds of
-            // `resident` workgroups (CUs x workgroups per CU at the kernel's occupancy), so
-            // pick the count that minimises rounds x (planes per chunk + 2 halo planes)
-            // (halo: 2 planes for the isothermal kernel's psi stencil, 4 for the thermal
-            // kernel's rho/T/U stencils of the heat source under the psi stencil)
+            // z chunks per column: the work items run in rounds of `resident` workgroups (CUs
+            // x workgroups per CU at the kernel's occupancy), so pick the count that minimises
+            // rounds x (planes per chunk + halo planes) (halo: 2 planes for the isothermal
+            // kernel's psi stencil, 4 for the thermal kernel's rho/T/U stencils of the heat
+            // source under the psi stencil).  Boxes that do not fill the device end at chunks
+            // of one or two planes: their time is a workgroup's chain of planes, and the halo
+            // planes come from cache (64^3 FP32 24.4 us per step in chunks of eight, 15.0 in
+            // chunks of two; thermal 56.4 and 30.8; 49 x 101 x 49 27.8 and 16.6).
             int bpc = 0, cus = 0;
             const int halo = z->tmarch ? 4 : 2;
             if (z->tmarch && z->noderef)
@@ -2186,7 +2189,7 @@ int fused_create(mplb_case* c) {
             const long long resident = std::max(1LL, (long long)bpc * cus);
             int nchunks = 1;
             long long best = -1;
-            for (int n = 1; n <= std::max(1, m.nz / 8); n++) {
+            for (int n = 1; n <= m.nz; n++) {
                 const long long rounds = ((long long)z->mtiles * n + resident - 1) / resident;
                 const long long cost = rounds * ((m.nz + n - 1) / n + halo);
                 if (best < 0 || cost < best) {
