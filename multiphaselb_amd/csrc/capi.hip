@@ -457,6 +457,12 @@ int setup_passes(mplb_case* c) {
     }
     if (c->fc[1].present && c->update[1]) HIPCHK(c, hipMalloc(&c->sumg, c->scalar_bytes * m.N));
     c->passes = true;
+    const bool thermal = c->fc[1].present && c->update[1];
+    if (m.d == 3 && !thermal && c->pass_faces == 0) {
+        const int e = c->scalar_bytes == 8 ? PassOps<double>::march_plan(c->opts.device, m.nx, m.ny, m.nz, &c->march)
+                                           : PassOps<float>::march_plan(c->opts.device, m.nx, m.ny, m.nz, &c->march);
+        if (e) return fail(c, MPLB_E_HIP, std::string("march plan: ") + hipGetErrorString((hipError_t)e));
+    }
     return tiles_create(c);
 }
 
@@ -774,6 +780,12 @@ void run_passes_t(mplb_case* c, int m, int level0) {
             for (size_t b = 0; b < c->bd.size(); b++)
                 if (list_active(c->fc[fld], (int)b))
                     PassOps<T>::boundary(ms.lbmodel, c->stream, a, fld, (int)b, next_list(c, fld, b));
+        }
+        if (c->march.items) {
+            TimedRegion tr(c, TM_COLLIDE);
+            PassOps<T>::march(c->stream, a, c->march, i == m - 1);
+            std::swap(c->f[0], c->f_alt[0]);
+            continue;
         }
         {
             TimedRegion tr(c, TM_MACRO);

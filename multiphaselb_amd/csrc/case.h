@@ -11,6 +11,7 @@
 #include "dict.h"
 #include "kernels.h"
 #include "mesh.h"
+#include "passes.h"
 
 namespace mplb {
 
@@ -89,6 +90,7 @@ struct mplb_case {
     int pass_faces = 0;                         // faces read through the neighbour table
     uint8_t* order[2] = {nullptr, nullptr};     // per field: each node's boundary list (255: none)
     void* sumg = nullptr;
+    mplb::PassMarch march;                      // the single-pass march (isothermal periodic D3Q15)
 
     // several steps per launch on small lattices (tiles.hip): rho, T, U, Fi, Ft, ss and psi
     // of the level being written

@@ -37,6 +37,11 @@ struct PassArgs {
     int first_call;              // liTempMRT heat source S_old = 0
 };
 
+// Work split of the single-pass march over a fully periodic D3Q15 box (items 0: not used)
+struct PassMarch {
+    int mtx = 0, tiles = 0, items = 0, per = 0, zc = 0;
+};
+
 template <typename T>
 struct PassOps {
     // boundary condition of one list of field fld (0 f, 1 g): the nodes' pulled and
@@ -49,6 +54,10 @@ struct PassOps {
     // force, velocity and the collisions of the next step; last: no collision, the
     // post-stream populations and every macroscopic field instead
     static void collide(int model, hipStream_t s, const PassArgs<T>& a, bool thermal, bool last);
+    // density and collide passes of an isothermal step in one (the plan stays empty where the
+    // two passes are the better choice)
+    static int march_plan(int device, int nx, int ny, int nz, PassMarch* p);
+    static void march(hipStream_t s, const PassArgs<T>& a, const PassMarch& p, bool last);
 };
 
 }  // namespace mplb
