@@ -2041,6 +2041,37 @@ bool fused_supported(const mplb_case* c, std::string* why) {
     return true;
 }
 
+// Both copies of the populations fit the 256 MiB memory-side cache
+bool in_cache(const Mesh& m, const Fused& z, size_t scalar) {
+    return 2 * (z.thermal ? 2 : 1) * scalar * m.Q * (size_t)z.P <= (size_t)256 << 20;
+}
+
+// Whether the single pass is faster than the two (thermal: three) passes, which read the
+// populations twice but leave no lane idle: a march's wavefronts are rows of 64 sites, so on
+// Nx of fill = Nx / (64 x columns) the rest idles.  Per step, single pass against passes:
+//   FP32       0.346 against 0.445 ms on 320 x 200^2 (fill 1), 0.315 / 0.316 on 208^3 (0.81),
+//              0.333 / 0.287 on 200^3 (0.78), 0.195 / 0.145 on 66 x 200 x 300 (0.52).  Rows that
+//              share 64-byte sectors need more (330 x 200^2, 0.86: 0.532 / 0.465; 180^3, 0.94:
+//              equal; 250^3, 0.98: 0.524 / 0.551).  In cache the passes' launches and psi
+//              cost more than the lanes (130^3, 0.68: 65 / 84 us; 75 x 90 x 120, 0.59: 31 / 36).
+//   FP16S      0.237 / 0.292 on 320 x 200^2, 91 / 96 us on 160^3 (0.83), 0.230 / 0.207 on 208^3,
+//              0.151 / 0.130 on 201 x 150 x 180 (0.79).
+//   FP16N      0.317 / 0.353 on 320 x 200^2, 0.196 / 0.191 on 190^3 (0.99), 0.390 / 0.378 on 240^3
+//              (0.94), 0.263 / 0.225 on 200^3: the references' loads make its pulls dear.
+//   thermal    FP32 0.863 / 1.052 on 320 x 200^2, 0.335 / 0.353 on 160^3, 0.872 / 0.753 on 208^3,
+//              0.551 / 0.480 on 201 x 150 x 180; with FP16 storage the three passes are faster
+//              everywhere (FP16S 255^3 1.024 / 0.945, 160^3 0.305 / 0.230).
+// Below 2^20 nodes a march is a short chain of planes with most of the device idle: the passes
+// are as fast or faster, but for FP32 (64^3 thermal 29.5 / 25.9 us, FP16S 13.3 / 12.2, FP16N
+// 15.8 / 12.8, FP32 13.8 / 13.3; 49 x 101 x 49 FP32 15.1 / 16.4).
+bool march_pays(const Mesh& m, const Fused& z, size_t scalar) {
+    const double fill = m.nx / (64.0 * ((m.nx + 63) / 64));
+    const bool sectors = m.nx * scalar % 64 == 0;
+    if (!z.thermal && !z.half) return in_cache(m, z, scalar) || fill >= (sectors ? 0.8 : 0.9);
+    if (z.thermal && z.half) return false;
+    return m.N >= 1 << 20 && fill >= (z.noderef ? 0.95 : 0.83);
+}
+
 // Non-temporal or ordinary stores of the new populations.  Non-temporal ones are best when
 // every wavefront writes whole 64-byte sectors and the populations do not fit the 256 MiB
 // memory-side cache (256^3 FP32 0.441 against 0.460 ms per step, 192^3 thermal 0.536 against
@@ -2058,7 +2089,7 @@ bool fused_supported(const mplb_case* c, std::string* why) {
 bool stores_nt(const Mesh& m, const Fused& z, size_t scalar) {
     if ((z.march || z.tmarch) && m.nx * scalar % 64 != 0) return false;
     if (z.thermal && z.half) return true;
-    return 2 * (z.thermal ? 2 : 1) * scalar * m.Q * (size_t)z.P > (size_t)256 << 20;
+    return !in_cache(m, z, scalar);
 }
 
 int fused_create(mplb_case* c) {
@@ -2128,31 +2159,31 @@ int fused_create(mplb_case* c) {
         z->face_table = odd_faces(m, bc);
     }
     // single-pass kernel: isothermal D3Q15 with every link the periodic wrap and no
-    // boundary node (MPLB_FUSED_KERNEL=twopass keeps the two-pass kernels)
+    // boundary node (MPLB_FUSED_KERNEL=twopass keeps the two-pass kernels, =march takes the
+    // single pass wherever it can run; march_pays chooses otherwise)
     {
         const char* env = std::getenv("MPLB_FUSED_KERNEL");
         const bool twopass = env && std::strcmp(env, "twopass") == 0;
+        const bool pays = (env && std::strcmp(env, "march") == 0) || march_pays(m, *z, sb);
         bool any_bnd = false;
         for (int64_t id = 0; id < N && !any_bnd; id++) any_bnd = m.onbnd[id] != 0;
         const bool periodic3 = !twopass && m.lbmodel == 1 && z->face_table == 0 && !any_bnd && m.nx >= 3 && m.ny >= 3 &&
                                m.nz >= 3;
-        z->march = periodic3 && !z->thermal;
-        // thermal single pass: xuMRT f with myMRT g (the D3Q15 thermal pair).  The default
-        // with FP32 storage (1.10 against 1.38 ms per step for the three passes on the
-        // 256^3 thermal bubble); with FP16 storage the three passes are as fast or faster
-        // (FP16S 0.961 against 0.975 ms, FP16N 1.004 against 1.162).
+        // LDS-staged pulls for the isothermal single pass, FP32 storage (opt-in, MPLB_MARCH_LDS=1)
+        const char* lenv = std::getenv("MPLB_MARCH_LDS");
+        const bool iso = periodic3 && !z->thermal;
+        z->march_lds = iso && !z->half && lenv && std::strcmp(lenv, "1") == 0;
+        // pulls issued a plane ahead (FP32 and FP16S storage; opt-in, MPLB_MARCH_PF=1)
+        const char* penv = std::getenv("MPLB_MARCH_PF");
+        z->march_pf = iso && !z->march_lds && !z->noderef && penv && std::strcmp(penv, "1") == 0;
+        z->march = iso && (pays || z->march_lds || z->march_pf);
+        // thermal single pass: xuMRT f with myMRT g (the D3Q15 thermal pair).
         // MPLB_THERMAL_MARCH=1 / =0 forces the single pass / the three passes.
         const char* tenv = std::getenv("MPLB_THERMAL_MARCH");
-        const bool tpick = tenv ? std::strcmp(tenv, "1") == 0 : !z->half;
+        const bool tpick = tenv ? std::strcmp(tenv, "1") == 0 : pays;
         // (it indexes populations in 32 bits: Q x pitch below 2^32)
         z->tmarch = periodic3 && z->thermal && c->fc[1].mp.model == M_MYMRT && tpick &&
                     15 * pitch_for(N) <= (int64_t)0xFFFFFFFF;
-        // LDS-staged pulls for the isothermal single pass, FP32 storage (opt-in, MPLB_MARCH_LDS=1)
-        const char* lenv = std::getenv("MPLB_MARCH_LDS");
-        z->march_lds = z->march && !z->half && lenv && std::strcmp(lenv, "1") == 0;
-        // pulls issued a plane ahead (FP32 and FP16S storage; opt-in, MPLB_MARCH_PF=1)
-        const char* penv = std::getenv("MPLB_MARCH_PF");
-        z->march_pf = z->march && !z->march_lds && !z->noderef && penv && std::strcmp(penv, "1") == 0;
         if (z->march || z->tmarch) {
             const int tmx = z->tmarch ? TMX : MX, tmy = z->tmarch ? TMY : MY;
             z->mtx = (m.nx + tmx - 1) / tmx;

@@ -1,5 +1,6 @@
 """The z-marches split a box into chunks of planes and store the new populations either
-non-temporally or not, by the rows' size and the populations' total.  Neither changes a
+non-temporally or not, by the rows' size and the populations' total; whether a box takes
+the march or the two passes follows from its size too.  Neither of the first two changes a
 node's arithmetic: whatever the number of chunks (one, the default, one per plane) the
 fields are equal bit for bit, and boxes on both sides of the store rule (rows that end
 inside a 64-byte sector, whole sectors in populations of less and of more than 256 MiB)
@@ -34,6 +35,7 @@ def run(spec, precision, thermal, steps):
 def test_chunks_leave_the_fields_unchanged(box, precision, thermal, variant, monkeypatch):
     print("box", box, "precision", precision, "thermal", thermal, variant, flush=True)
     spec = d3(nx=box[0], ny=box[1], nz=box[2], btype=5)
+    monkeypatch.setenv("MPLB_FUSED_KERNEL", "march")
     if variant:
         monkeypatch.setenv(variant, "1")
     out = []
@@ -51,6 +53,8 @@ def test_chunks_leave_the_fields_unchanged(box, precision, thermal, variant, mon
 def test_both_kinds_of_stores_follow_the_two_pass_kernels(box, precision, monkeypatch):
     print("box", box, "precision", precision, flush=True)
     spec = d3(nx=box[0], ny=box[1], nz=box[2], btype=5)
+    picked = run(spec, precision, False, 6)          # whichever the box's size calls for
+    monkeypatch.setenv("MPLB_FUSED_KERNEL", "march")
     one = run(spec, precision, False, 6)
     monkeypatch.setenv("MPLB_FUSED_KERNEL", "twopass")
     two = run(spec, precision, False, 6)
@@ -58,3 +62,4 @@ def test_both_kinds_of_stores_follow_the_two_pass_kernels(box, precision, monkey
     assert rel(one["rho"], two["rho"]) < tol
     assert rel(one["f"], two["f"]) < tol
     assert np.max(np.abs(one["U"] - two["U"])) < 0.1 * tol
+    assert any(all(np.array_equal(picked[f], o[f]) for f in picked) for o in (one, two))
