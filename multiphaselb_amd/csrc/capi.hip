@@ -700,35 +700,26 @@ int write_step_t(mplb_case* c) {
 // multiPhasePP.c:157-241
 template <typename T>
 int one_step_t(mplb_case* c) {
-    if (c->fused) {
-        int rc = fused_step(c);
-        if (rc) return rc;
-    } else {
-        collision_t<T>(c, 0);
-        stream_t<T>(c, 0);
-        boundaries_t<T>(c, 0);
-        collision_t<T>(c, 1);
-        stream_t<T>(c, 1);
-        boundaries_t<T>(c, 1);
-        macro_density_t<T>(c);
-        if (c->opts.heat_transfer) heat_source_t<T>(c);
-        macro_temperature_t<T>(c);
-        if (!c->opts.frozen) inter_force_t<T>(c);
-        macro_velocity_t<T>(c);
-    }
-    if (c->stp == c->write_interval) {
-        if (c->fused) {
-            int rc = fused_sync_to_generic(c);
-            if (rc) return rc;
-        }
-        int rc = write_step_t<T>(c);
-        if (rc) return rc;
-        if (c->fused) {
-            rc = fused_after_write(c);
-            if (rc) return rc;
-        }
-    }
-    return 0;
+    collision_t<T>(c, 0);
+    stream_t<T>(c, 0);
+    boundaries_t<T>(c, 0);
+    collision_t<T>(c, 1);
+    stream_t<T>(c, 1);
+    boundaries_t<T>(c, 1);
+    macro_density_t<T>(c);
+    if (c->opts.heat_transfer) heat_source_t<T>(c);
+    macro_temperature_t<T>(c);
+    if (!c->opts.frozen) inter_force_t<T>(c);
+    macro_velocity_t<T>(c);
+    return c->stp == c->write_interval ? write_step_t<T>(c) : 0;
+}
+
+// the write step of a fused case
+template <typename T>
+int fused_write_t(mplb_case* c) {
+    int rc = fused_sync_to_generic(c);
+    if (!rc) rc = write_step_t<T>(c);
+    return rc ? rc : fused_after_write(c);
 }
 
 // m steps of multiPhasePP.c:157-241 in fused passes (kernels_passes.hip) or, on small
@@ -808,7 +799,7 @@ template <typename T>
 int steps_t(mplb_case* c, int nsteps, int* done) {
     int n = 0;
     bool more = true;
-    while (c->passes && more && n < nsteps) {
+    while ((c->fused || c->passes) && more && n < nsteps) {
         // the steps up to and including the next write step go out as one run
         const int level0 = c->current;
         int m = 0;
@@ -817,15 +808,17 @@ int steps_t(mplb_case* c, int nsteps, int* done) {
             m++;
             write = c->stp == c->write_interval;
         }
-        if (m) run_passes_t<T>(c, m, level0);
+        int rc = 0;
+        if (m && c->fused) rc = fused_steps(c, m, level0);
+        else if (m) run_passes_t<T>(c, m, level0);
         n += m;
-        const int rc = write ? write_step_t<T>(c) : 0;
+        if (!rc && write) rc = c->fused ? fused_write_t<T>(c) : write_step_t<T>(c);
         if (rc) {
             if (done) *done = n;
             return rc;
         }
     }
-    while (!c->passes && n < nsteps && update_time(c)) {
+    while (!c->fused && !c->passes && n < nsteps && update_time(c)) {
         int rc = one_step_t<T>(c);
         n++;
         if (rc) {

@@ -13,7 +13,8 @@ bool fused_supported(const mplb_case* c, std::string* why);
 int fused_create(mplb_case* c);
 void fused_destroy(mplb_case* c);
 int fused_after_init(mplb_case* c);
-int fused_step(mplb_case* c);
+// m steps; level0: the time level before the first of them
+int fused_steps(mplb_case* c, int m, int level0);
 // make the generic device arrays (rho, T, U, f, g ...) describe the current time level
 int fused_sync_to_generic(mplb_case* c);
 int fused_after_write(mplb_case* c);

@@ -29,6 +29,7 @@
 #include "case.h"
 #include "fused.h"
 #include "physics.h"
+#include "tiles.h"
 
 namespace mplb {
 
@@ -1518,6 +1519,263 @@ k_fused_march_lds(FArgs a) {
 
 // Post-stream, post-boundary populations of the current time level (what the
 // reference holds in f.value after updateBoundaries), FP32 SoA.
+
+// ---------------------------------------------------------------------------
+// Several steps per launch on small D2Q9 lattices.  A step of a lattice of some ten thousand
+// nodes is two or three launches of about 5 us each, whatever the nodes cost.  Here a
+// workgroup owns a block of nodes and loads with it every node that can reach it in
+// p.steps steps (two neighbours per step, pull and psi stencil; three with heat transfer),
+// one thread per node, populations in LDS, the valid set shrinking by a step's halo each
+// time.  Neighbours come from the tile's table (tiles.hip), so walls and duplicate nodes are
+// followed as the lattice has them.  FP16 storage rounds the populations at every step, as
+// the passes do: the steps a launch takes leave the fields unchanged bit for bit.
+// Bound: latency (launch, two or three barriers a step, one node's chain of arithmetic).
+struct FTileArgs {
+    TileTable t;
+    int steps;                   // of this launch
+    int first_level;             // the launch's step that is the heat source's first call (-1: none)
+    int left[16];                // fixedRandomT slots: steps that still draw, from the launch's first
+    const float* Sin;            // liTempMRT: the heat source of the level before
+};
+
+// fixed_temperature from a tile's LDS
+template <class L, int NT>
+__device__ inline void tile_fixed_temperature(const FArgs& a, int64_t id, const int* at, unsigned miss,
+                                              const int16_t* inner, int e, int total, uint8_t code, bool draws,
+                                              const float (*gs)[NT], const float* sT, const float (*sU)[NT], float* v) {
+    int draw = code == FB_FRDT ? a.rnd_off[id] : 0;
+    const float Tw0 = a.bcTw[id];
+    // (an empty statement, so that what follows from them is not kept in registers all
+    // through the step loop)
+    float a1 = a.a1, a2 = a.a2;
+    asm volatile("" : "+s"(a1), "+s"(a2), "+v"(e));
+    float minT = 0, maxT = 0;
+    if (code == FB_FRDT) {
+        const float pert = a.bcPert[id];
+        minT = Tw0 * (100.0f - pert) / 100.0f;
+        maxT = Tw0 * (100.0f + pert) / 100.0f;
+    }
+#pragma unroll
+    for (int q = 0; q < L::Q; q++) {
+        if (!(miss >> q & 1) || (miss >> L::t.rev[q] & 1)) continue;
+        const int n = at[L::t.rev[q]];
+        const float gnb = gs[q][inner[e + q * total]];
+        const float U[3] = {sU[0][n], sU[1][n], L::D == 3 ? sU[L::D - 1][n] : 0.f};
+        float geq[L::Q];
+        if (a.gmodel == 1) my_geq<L, float>(sT[n], U, a1, a2, geq);
+        else litemp_geq<L, float>(sT[n], U, geq);
+        const float eq_nb = geq[q];
+        float Tw = Tw0;
+        if (code == FB_FRDT && draws) Tw = minT + (maxT - minT) * (float)a.rnd[draw++];
+        if (a.gmodel == 1) my_geq<L, float>(Tw, U, a1, a2, geq);
+        else litemp_geq<L, float>(Tw, U, geq);
+        v[q] = geq[q] + (gnb - eq_nb);
+    }
+}
+
+// bounce_back with the links that are missing as bits
+template <class L>
+__device__ inline void tile_bounce_back(unsigned miss, float* v) {
+#pragma unroll
+    for (int q = 0; q < L::Q; q++) {
+        const int r = L::t.rev[q];
+        if (miss >> q & 1) {
+            v[q] = v[r];
+        } else if (!(miss >> r & 1) && q >= 1 && q <= L::naxis) {
+            v[q] = 0.5f * v[q] + 0.5f * v[r];
+            v[r] = v[q];
+        }
+    }
+}
+
+template <class L, typename S, bool THERMAL, int NT>
+__global__ void __launch_bounds__(NT) k_fused_tile(FArgs a, FTileArgs p) {
+    __shared__ float fs[L::Q][NT], s_psi[NT];
+    __shared__ float gs[THERMAL ? L::Q : 1][THERMAL ? NT : 1];
+    __shared__ float s_rho[THERMAL ? NT : 1], s_T[THERMAL ? NT : 1], s_U[L::D][THERMAL ? NT : 1];
+    constexpr int H = THERMAL ? 3 : 2;
+    constexpr bool HALF = sizeof(S) == 2;
+    const int i = threadIdx.x;
+    const int64_t e = (int64_t)blockIdx.x * p.t.stride + i, N = a.N;
+    const int meta = i < p.t.stride ? p.t.meta[e] : 255 << 24;
+    const int depth = meta >> 24 & 0xFF;
+    const bool interior = (meta >> 16 & 1) != 0, full = (meta >> 17 & 1) != 0;
+    int R = H * p.steps;                         // depth up to which the tile's state is valid
+    int at[L::Q];                                // upstream nodes (the node itself where the link is missing)
+    unsigned miss = 0;
+    int64_t id = 0;
+    float temp = 0.f, ss = 0.f;
+    uint8_t bf = 0, bg = 0;
+    float v[L::Q], w[THERMAL ? L::Q : 1], U[3], Fi[3], Ft[3], rho = 0.f, psi = 0.f;
+    _Float16 hf[HALF ? L::Q : 1], hg[HALF && THERMAL ? L::Q : 1], href = 0;
+    if (depth <= R) {
+        id = p.t.gid[e];
+#pragma unroll
+        for (int q = 0; q < L::Q; q++) {
+            at[q] = p.t.nb[q * p.t.total + e];
+            v[q] = ldf<S>((const char*)a.fin + (size_t)q * a.P * sizeof(S), id, f_wref<L, S>(a, id, q));
+            if constexpr (THERMAL) w[q] = ld<S>((const char*)a.gin + (size_t)q * a.P * sizeof(S), id, a.gshift[q]);
+        }
+        temp = a.Tuniform ? a.Tconst : a.Told[id];
+        if (a.lists_f) bf = a.bcf[id];
+        if constexpr (THERMAL) {
+            if (a.lists_g) bg = a.bcg[id];
+            if (a.gmodel != 1) ss = p.Sin[id];
+            s_T[i] = temp;
+#pragma unroll
+            for (int d = 0; d < L::D; d++) s_U[d][i] = a.Uold[d * N + id];
+        }
+#pragma unroll
+        for (int q = 0; q < L::Q; q++) {
+            if (at[q] == -1) {
+                at[q] = i;
+                miss |= 1u << q;
+            }
+            fs[q][i] = v[q];
+            if constexpr (THERMAL) gs[q][i] = w[q];
+        }
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int s = 0;; s++) {
+        if (depth <= R - 1) {
+#pragma unroll
+            for (int q = 0; q < L::Q; q++) v[q] = fs[q][at[q]];
+            if (bf == FB_BBACK) tile_bounce_back<L>(miss, v);
+            rho = rho_sym<L, float>(v);
+            if constexpr (THERMAL) {
+#pragma unroll
+                for (int q = 0; q < L::Q; q++) w[q] = gs[q][at[q]];
+                s_rho[i] = rho;
+                const uint8_t code = bg & 0xF;
+                if (code == FB_BBACK) tile_bounce_back<L>(miss, w);
+                else if (code != FB_NONE)
+                    tile_fixed_temperature<L, NT>(a, id, at, miss, p.t.inner, (int)e, (int)p.t.total, code,
+                                                  s < p.left[bg >> 4], gs, s_T, s_U, w);
+            } else {
+                psi = fpot(a, rho, temp);
+                s_psi[i] = psi;
+            }
+        }
+        __syncthreads();
+        if constexpr (THERMAL) {
+            if (depth <= R - 2) {
+                float dot = 0.f, divU = 0.f;
+#pragma unroll
+                for (int ax = 0; ax < L::D; ax++) {
+                    const int qa = L::fd_plus[ax], qb = L::fd_minus[ax], na = at[qa], nb = at[qb];
+                    const bool ha = !(miss >> qa & 1), hb = !(miss >> qb & 1);
+                    const float Ta = s_T[na], Tb = s_T[nb], ra = s_rho[na], rb = s_rho[nb];
+                    const float ua = s_U[ax][na], ub = s_U[ax][nb];
+                    if (ha && hb) {
+                        heat_axis(Ta, Tb, ra, rb, ua, ub, dot, divU);
+                    } else {
+                        // one-sided where one link is missing, nothing where both are (then both
+                        // neighbours are the node itself)
+                        dot += (Ta - Tb) * (1.0f / ra - 1.0f / rb);
+                        divU += ua - ub;
+                    }
+                }
+                const float src = heat_tail<L>(a, rho, temp, dot, divU);
+                float t = rho_sym<L, float>(w);
+                if (a.gmodel == 1) {
+                    ss = src;
+                    t = t + 0.5f * ss;
+                } else {
+                    const float old = s == p.first_level ? 0.f : ss;
+                    ss = src + 0.5f * (src - old);
+                }
+                temp = t;
+                psi = fpot(a, rho, t);
+                s_psi[i] = psi;
+            }
+            __syncthreads();
+        }
+        R -= H;
+        if (depth <= R) {
+            float psin[L::Q];
+            psin[0] = psi;
+#pragma unroll
+            for (int q = 1; q < L::Q; q++) {
+                const int r = L::t.rev[q];
+                psin[q] = miss >> r & 1 ? psi : s_psi[at[r]];
+            }
+            collide_node<L>(a, v, rho, psin, interior, full, U, Fi, Ft);
+            if constexpr (THERMAL) collide_g<L>(a, w, temp, ss, U);
+            // the stored values: what the next step pulls
+            if constexpr (HALF) {
+                if constexpr (kNodeRef<S>) {
+                    const float r = (rho >= kRefMin || rho != rho) ? rho : kRefMin;
+                    href = (_Float16)r;
+                    const float rr = (float)href, rinv = 1.f / rr;
+#pragma unroll
+                    for (int q = 0; q < L::Q; q++) {
+                        const float wref = (float)L::t.omega[q] * rr;
+                        hf[q] = (_Float16)((v[q] - wref) * ((float)(1.0 / L::t.omega[q]) * rinv));
+                        v[q] = fmaf((float)hf[q], wref, wref);
+                    }
+                } else {
+#pragma unroll
+                    for (int q = 0; q < L::Q; q++) {
+                        hf[q] = (_Float16)(v[q] - a.fshift[q]);
+                        v[q] = (float)hf[q] + a.fshift[q];
+                    }
+                }
+                if constexpr (THERMAL) {
+#pragma unroll
+                    for (int q = 0; q < L::Q; q++) {
+                        hg[q] = (_Float16)(w[q] - a.gshift[q]);
+                        w[q] = (float)hg[q] + a.gshift[q];
+                    }
+                }
+            }
+        }
+        if (s + 1 == p.steps) break;
+        if (depth <= R) {
+#pragma unroll
+            for (int q = 0; q < L::Q; q++) {
+                fs[q][i] = v[q];
+                if constexpr (THERMAL) gs[q][i] = w[q];
+            }
+            if constexpr (THERMAL) {
+                s_T[i] = temp;
+#pragma unroll
+                for (int d = 0; d < L::D; d++) s_U[d][i] = U[d];
+            }
+        }
+        __syncthreads();
+    }
+    // (outside the loop, which would keep the addresses in registers)
+    if (depth > 0) return;
+#pragma unroll
+    for (int q = 0; q < L::Q; q++) {
+        if constexpr (HALF) {
+            ((_Float16*)a.fout)[q * a.P + id] = hf[q];
+            if constexpr (THERMAL) ((_Float16*)a.gout)[q * a.P + id] = hg[q];
+        } else {
+            ((float*)a.fout)[q * a.P + id] = v[q];
+            if constexpr (THERMAL) ((float*)a.gout)[q * a.P + id] = w[q];
+        }
+    }
+    if constexpr (kNodeRef<S>) a.rout[id] = href;
+    a.psi[id] = psi;
+    if constexpr (THERMAL) {
+        a.Tnew[id] = temp;
+        a.S[id] = ss;
+#pragma unroll
+        for (int d = 0; d < 3; d++) a.Unew[d * N + id] = U[d];
+    }
+    if (a.out_rho) {
+        a.out_rho[id] = rho;
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            a.out_U[d * N + id] = U[d];
+            a.out_Fi[d * N + id] = Fi[d];
+            a.out_Ft[d * N + id] = Ft[d];
+        }
+    }
+}
+
 template <class L, typename S, bool G>
 __global__ void __launch_bounds__(256) k_fused_materialize(FArgs a, float* out) {
     const NodePos p = node_pos<L>(a);
@@ -1596,6 +1854,8 @@ struct Fused {
     float t_const = 0.f;
     int mtx = 0, mtiles = 0, mitems = 0, mper = 0, mzc = 0;
     bool nt = true;              // population stores are non-temporal
+    float* S = nullptr;          // tiled lattices: the second copy of the heat source
+    FTileArgs last{};            // arguments of the last tile launch
 };
 
 Fused* F(mplb_case* c) { return (Fused*)c->fz; }
@@ -1817,6 +2077,70 @@ void launch_step_timed(mplb_case* c, FArgs a, bool thermal, bool outputs) {
     }
 }
 
+constexpr int kTileThreads = 1024;     // largest tile: 4 wavefronts per SIMD, 128 VGPRs each
+
+template <class L, typename S>
+void launch_tile(mplb_case* c, const FArgs& a, const FTileArgs& p, bool thermal) {
+    if constexpr (L::D == 2) {
+        const dim3 grid((unsigned)p.t.tiles);
+        auto go = [&](auto th) {
+            constexpr bool TH = decltype(th)::value;
+            const int n = c->tiles->nodes;
+            if (n <= 256) k_fused_tile<L, S, TH, 256><<<grid, 256, 0, c->stream>>>(a, p);
+            else if (n <= 512) k_fused_tile<L, S, TH, 512><<<grid, 512, 0, c->stream>>>(a, p);
+            else k_fused_tile<L, S, TH, kTileThreads><<<grid, kTileThreads, 0, c->stream>>>(a, p);
+        };
+        if (thermal) go(std::true_type{});
+        else go(std::false_type{});
+    }
+}
+
+// m steps of a tiled lattice; level0: the time level before the first of them.  The last one
+// is a launch of its own, so that its input is there when the level is read back.
+template <class L, typename S>
+int do_tiles(mplb_case* c, int m, int level0) {
+    Fused* z = F(c);
+    for (int done = 0; done < m;) {
+        FArgs a = make_args(c);
+        a.fin = z->fa;
+        a.fout = z->fb;
+        a.gin = z->ga;
+        a.gout = z->gb;
+        FTileArgs& p = z->last;
+        p.t = c->tiles->t;
+        p.steps = m - done > 1 ? std::min(c->tiles->steps, m - done - 1) : 1;
+        p.first_level = -1 - (level0 + done) >= 0 ? -1 - (level0 + done) : -1;
+        p.Sin = (const float*)c->ss;
+        a.S = z->S;
+        // fixedRandomT (fixedRandomT.c:79): each list draws while its own localTStep < psteps
+        for (size_t s = 0; s < z->frdt_lists.size(); s++) {
+            FieldCfg& fc = c->fc[z->frdt_lists[s].first];
+            const int b = z->frdt_lists[s].second;
+            p.left[s] = fc.psteps[b] - fc.localT[b];
+            fc.localT[b] += p.steps;
+        }
+        {
+            Ev e(c, 6);
+            launch_tile<L, S>(c, a, p, z->thermal);
+        }
+        z->last_draw = 0;
+        for (size_t s = 0; s < z->frdt_lists.size(); s++) z->last_draw |= p.left[s] > 0 ? 1 << s : 0;
+        z->rho0_built = a.rho0;
+        std::swap(z->fa, z->fb);
+        std::swap(z->ra, z->rb);
+        std::swap(z->ga, z->gb);
+        if (z->thermal) {
+            z->cur = 1 - z->cur;
+            void* s = c->ss;
+            c->ss = z->S;
+            z->S = (float*)s;
+        }
+        done += p.steps;
+    }
+    z->generic_current = false;
+    return 0;
+}
+
 template <class L, typename S>
 int run_prologue(mplb_case* c) {
     // generic state (post-stream populations and macroscopic fields of the current time
@@ -1871,19 +2195,16 @@ int run_prologue(mplb_case* c) {
     return 0;
 }
 
+// one step; level: its time level
 template <class L, typename S>
-int do_step(mplb_case* c) {
+int do_step(mplb_case* c, int level) {
     Fused* z = F(c);
-    if (z->need_prologue) {
-        int rc = run_prologue<L, S>(c);
-        if (rc) return rc;
-    }
     FArgs a = make_args(c);
     a.fin = z->fa;
     a.fout = z->fb;
     a.gin = z->ga;
     a.gout = z->gb;
-    a.first_call = c->current == 0 ? 1 : 0;
+    a.first_call = level == 0 ? 1 : 0;
     // fixedRandomT (fixedRandomT.c:79): each list draws while its own localTStep < psteps
     a.draw = 0;
     for (size_t s = 0; s < z->frdt_lists.size(); s++) {
@@ -1904,7 +2225,21 @@ int do_step(mplb_case* c) {
     return 0;
 }
 
-// After do_step the buffers hold: fa = post-collision of step n+1, fb = post-collision
+template <class L, typename S>
+int do_steps(mplb_case* c, int m, int level0) {
+    if (F(c)->need_prologue) {
+        const int rc = run_prologue<L, S>(c);
+        if (rc) return rc;
+    }
+    if (c->tiles) return do_tiles<L, S>(c, m, level0);
+    for (int i = 1; i <= m; i++) {
+        const int rc = do_step<L, S>(c, level0 + i);
+        if (rc) return rc;
+    }
+    return 0;
+}
+
+// After do_steps the buffers hold: fa = post-collision of step n+1, fb = post-collision
 // of step n (input of the last K2).  Materialising level n pulls from fb.
 template <class L, typename S>
 int materialize(mplb_case* c) {
@@ -1936,7 +2271,12 @@ int materialize(mplb_case* c) {
     a.out_Fi = (float*)c->Fi;
     a.out_Ft = (float*)c->Ft;
     a.out_U = (float*)c->U;
-    if (z->thermal && z->tmarch) {
+    if (c->tiles) {
+        // the last launch, which was one step, with outputs: it rewrites fa, ga, T, U and the heat source with
+        // the values they hold
+        if (z->thermal) z->last.Sin = z->S;
+        launch_tile<L, S>(c, a, z->last, z->thermal);
+    } else if (z->thermal && z->tmarch) {
         // the step's own kernel with outputs on the last step's inputs: it rewrites fa, ga,
         // T and U with the values they hold
         launch_tmarch<L, S, true>(c, a);
@@ -2090,6 +2430,61 @@ bool stores_nt(const Mesh& m, const Fused& z, size_t scalar) {
     if ((z.march || z.tmarch) && m.nx * scalar % 64 != 0) return false;
     if (z.thermal && z.half) return true;
     return !in_cache(m, z, scalar);
+}
+
+// Time of one step in tiles, in microseconds, with a plan's blocks and steps per launch: a
+// launch with the load of its state, then per step a latency (barriers, LDS, one node's chain
+// of arithmetic) and the work of every 256 nodes; more tiles than the device holds take turns.
+// The constants fit sweeps of blocks and steps, FP32: 256^2 in blocks of 26 x 26, 22 x 22, 19 x 19
+// and 15 x 15 with 1 to 4 steps per launch 8.6, 5.4, 4.8 and 5.6 us per step, in 19 x 19 with heat
+// transfer and 2 steps 10.5, in 13 x 13 and 3 steps 12.7.  Chosen by it, us per step in tiles
+// against passes: 65^2 2.2 / 8.9, 128^2 2.5 / 9.1, 256^2 3.9 / 10.0, 401 x 333 6.3 / 12.2, 700^2 16.4 /
+// 18.6; with heat transfer 65^2 4.4 / 13.9, 128^2 5.5 / 14.0, 256^2 8.3 / 15.0, 401 x 333 15.9 / 19.8,
+// 3 x 301 column 2.9 / 17.2.  With heat transfer a box of more than about 400^2 nodes needs a second
+// round of workgroups and stays with the passes (550^2 35.1 against 27.5).
+static double tile_plan_us(const TilePlan& p, const int n[2], const Fused& z, int H, int cus) {
+    const double wait = z.thermal ? 1.3 : 0.6, work = z.thermal ? 1.2 : 0.6;
+    double sum = 0, load = 0;
+    int64_t tiles = 1, local = 1;
+    for (int d = 0; d < 2; d++) tiles *= (n[d] + p.b[d] - 1) / p.b[d];
+    for (int s = p.steps; s > 0; s--) {
+        local = 1;
+        for (int d = 0; d < 2; d++) local *= std::min(n[d], p.b[d] + 2 * H * s + 1);
+        if (local > kTileThreads) return 1e30;
+        if (s == p.steps) load = (double)local / (z.thermal ? 250 : 400);
+        sum += wait + work * (double)((local + 255) / 256);
+    }
+    const double rounds = (double)((tiles + cus - 1) / cus);
+    return (5.0 + (rounds > 1 ? 1.25 * rounds : 1.0) * (sum + load)) / p.steps;
+}
+
+// Time of one step in passes (their launches, then the nodes; the storage makes no difference
+// at these sizes): measured 10.0, 12.2 and 18.6 us on 256^2, 401 x 333 and 700^2, with heat
+// transfer 15.0, 19.8 and 36.4.
+static double tile_passes_us(const Mesh& m, const Fused& z) {
+    return z.thermal ? 11.7 + 51e-6 * (double)m.N : 9.2 + 18.5e-6 * (double)m.N;
+}
+
+// Tiles (k_fused_tile) where they are the faster way.
+static int create_tiles(mplb_case* c) {
+    Fused* z = F(c);
+    const Mesh& m = c->mesh;
+    if (z->lb != 0 || m.N > 1 << 20 || m.bd.size() >= 255) return 0;
+    const int H = z->thermal ? 3 : 2, n[2] = {m.nx, m.ny};
+    int cus = 256;
+    FCHK(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->opts.device));
+    std::vector<int> sizes;
+    for (int b = 1; b <= 128; b += b < 32 ? 1 : b < 64 ? 4 : 32) sizes.push_back(b);
+    TilePlan p = tile_choose(c, sizes, 0.95 * tile_passes_us(m, *z), [&](const TilePlan& q) {
+        return tile_plan_us(q, n, *z, H, cus);
+    });
+    tile_override(&p);
+    if (p.steps <= 0) return 0;
+    const bool lists[2] = {z->lists[0] != 0, z->lists[1] != 0};
+    const int rc = tile_tables(c, p, H * p.steps, kTileThreads, lists);
+    if (rc || !c->tiles) return rc;
+    if (z->thermal) FCHK(c, hipMalloc(&z->S, sizeof(float) * m.N));
+    return 0;
 }
 
 int fused_create(mplb_case* c) {
@@ -2251,14 +2646,14 @@ int fused_create(mplb_case* c) {
     FCHK(c, hipMalloc(&z->rnd_off, sizeof(int) * N));
     FCHK(c, hipMemcpy(z->rnd_off, off.data(), sizeof(int) * N, hipMemcpyHostToDevice));
     (void)any_frdt;
-    return 0;
+    return create_tiles(c);
 }
 
 void fused_destroy(mplb_case* c) {
     Fused* z = F(c);
     if (!z) return;
     void* ptrs[] = {z->fa, z->fb, z->ra, z->rb, z->ga, z->gb, z->rho, z->sumg, z->T[0], z->T[1], z->U[0], z->U[1],
-                    z->bcf, z->bcg, z->bcTw, z->bcPert, z->rnd_off};
+                    z->bcf, z->bcg, z->bcTw, z->bcPert, z->rnd_off, z->S};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);     // teardown: nothing left to report to
     delete z;
@@ -2309,8 +2704,8 @@ int fused_after_init(mplb_case* c) {
     return dispatch(c, [&](auto L, auto S) { return run_prologue<decltype(L), decltype(S)>(c); });
 }
 
-int fused_step(mplb_case* c) {
-    return dispatch(c, [&](auto L, auto S) { return do_step<decltype(L), decltype(S)>(c); });
+int fused_steps(mplb_case* c, int m, int level0) {
+    return dispatch(c, [&](auto L, auto S) { return do_steps<decltype(L), decltype(S)>(c, m, level0); });
 }
 
 int fused_sync_to_generic(mplb_case* c) {

@@ -1,9 +1,12 @@
-// Several time steps per launch on small lattices (kernels_tiles.hip).
+// Several time steps per launch on small lattices (kernels_tiles.hip; k_fused_tile of
+// kernels_fused.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <functional>
+#include <vector>
 
 #include "kernels.h"
 
@@ -57,6 +60,29 @@ struct TileOps {
     static void run(int model, hipStream_t s, const TileArgs<T>& a, bool thermal, int nodes);
 };
 
+// What a tiled case keeps on the device
+struct Tiles {
+    TileTable t{};
+    int nodes = 0;               // largest tile
+    int steps = 0;               // per launch
+    std::vector<void*> owned;
+};
+
+struct TilePlan {
+    int b[3] = {0, 0, 0};        // owned block
+    int steps = 0;               // per launch (0: no tiles)
+    double us = 0;               // estimated time of a step
+};
+
+// The cheapest plan under limit_us on a structured box: `us` estimates a step's time with a
+// plan of blocks of the given sizes (1e30: its tiles do not fit).
+TilePlan tile_choose(const mplb_case* c, const std::vector<int>& sizes, double limit_us,
+                     const std::function<double(const TilePlan&)>& us);
+// MPLB_TILES=bx,by,bz,steps sets the plan (steps 0: no tiles), for tests and timing sweeps
+void tile_override(TilePlan* p);
+// Builds the tables of a plan whose halo is `depth` levels (c->tiles); leaves the case
+// without when a tile has more than cap nodes.  lists: the field has boundary lists.
+int tile_tables(mplb_case* c, const TilePlan& p, int depth, int cap, const bool lists[2]);
 // Chooses tiles for a case that runs in fused passes and builds their tables (c->tiles);
 // leaves the case without when more launches over the whole lattice are the faster way.
 int tiles_create(mplb_case* c);

@@ -3,9 +3,14 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdio>
 #include <cstdlib>
+#include <memory>
+#include <new>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "case.h"
@@ -14,12 +19,6 @@
 namespace mplb {
 
 namespace {
-
-struct Plan {
-    int b[3] = {0, 0, 0};        // owned block (structured boxes); b[0] consecutive nodes otherwise
-    int steps = 0;
-    double us = 0;               // estimated time of a step
-};
 
 #define TCHK(c, call)                                                           \
     do {                                                                        \
@@ -42,7 +41,7 @@ int tile_reverse(const Mesh& m, int k) { return m.lbmodel == 0 ? D2Q9::t.rev[k] 
 // 256^2 7.9 / 12.3; with heat transfer 64^2 7.0 / 17.6, 128^2 8.8 / 18.4, 3 x 301 column 4.7 / 28.4
 // (its walls are launches of their own in passes), 3 x 3 x 301 D3Q15 column 9.9 / 40.7.  From
 // about 300^2 on the halo costs more than the launches it saves.
-double plan_us(const Plan& p, const int n[3], bool thermal, bool d3, bool fp64, int cap, int extra, int cus) {
+double plan_us(const TilePlan& p, const int n[3], bool thermal, bool d3, bool fp64, int cap, int extra, int cus) {
     const int H = thermal ? 3 : 2;
     const double scale = (d3 ? 1.7 : 1.0) * (fp64 ? 1.0 : 0.6);
     const double wait = (thermal ? 2.2 : 1.0) * scale, work = (thermal ? 2.0 : 1.05) * scale;
@@ -70,30 +69,29 @@ double passes_us(const mplb_case* c, bool thermal, bool fp64) {
     return us + (double)c->mesh.N * per / 5e6;
 }
 
-Plan choose(mplb_case* c, int cap, bool thermal, bool fp64, int extra) {
+}  // namespace
+
+TilePlan tile_choose(const mplb_case* c, const std::vector<int>& sizes, double limit_us,
+                     const std::function<double(const TilePlan&)>& us) {
     const Mesh& m = c->mesh;
-    const bool d3 = m.d == 3;
-    int cus = 256;
-    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->opts.device);
-    Plan best;
-    best.us = 0.85 * passes_us(c, thermal, fp64);
-    const int n[3] = {m.structured ? m.nx : (int)m.N, m.structured ? m.ny : 1, m.structured ? m.nz : 1};
+    TilePlan best;
+    best.us = limit_us;
     if (!m.structured) return best;      // no neighbourhood to size a block by
-    static const int sizes[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 14, 16, 20, 24, 32, 48, 64, 128};
+    const int n[3] = {m.nx, m.ny, m.nz};
     for (int bx : sizes)
         for (int by : sizes)
             for (int bz : sizes) {
-                if (!d3 && bz > 1) break;
-                Plan p;
+                if (m.d == 2 && bz > 1) break;
+                TilePlan p;
                 const int want[3] = {bx, by, bz};
                 bool ok = true;
                 for (int d = 0; d < 3; d++) {
                     p.b[d] = std::min(want[d], n[d]);
                     ok = ok && (want[d] < 2 * n[d]);
                 }
-                if (!ok || (int64_t)p.b[0] * p.b[1] * p.b[2] > cap) continue;
+                if (!ok) continue;
                 for (p.steps = 1; p.steps <= 12; p.steps++) {
-                    p.us = plan_us(p, n, thermal, d3, fp64, cap, extra, cus);
+                    p.us = us(p);
                     if (p.us >= 1e29) break;
                     if (p.us < best.us) best = p;
                 }
@@ -101,15 +99,12 @@ Plan choose(mplb_case* c, int cap, bool thermal, bool fp64, int extra) {
     return best;
 }
 
-}  // namespace
-
-// What a tiled case keeps on the device
-struct Tiles {
-    TileTable t{};
-    int nodes = 0;               // largest tile
-    int steps = 0;               // per launch
-    std::vector<void*> owned;
-};
+void tile_override(TilePlan* p) {
+    if (const char* env = std::getenv("MPLB_TILES")) {
+        if (std::sscanf(env, "%d,%d,%d,%d", &p->b[0], &p->b[1], &p->b[2], &p->steps) != 4) p->steps = 0;
+        for (int d = 0; d < 3; d++) p->b[d] = std::max(1, p->b[d]);
+    }
+}
 
 void tiles_destroy(mplb_case* c) {
     if (!c->tiles) return;
@@ -122,26 +117,77 @@ void tiles_destroy(mplb_case* c) {
     }
 }
 
+namespace {
+
+// fn(t, mark, slot) for every tile, on a few threads; mark (-1 at first) and slot are a
+// thread's own entries per node.  False: memory ran out.
+template <typename Fn>
+bool over_tiles(size_t tiles, int64_t N, const Fn& fn) {
+    std::atomic<size_t> next{0};
+    std::atomic<bool> ok{true};
+    auto work = [&] {
+        try {
+            std::vector<int> mark, slot;
+            for (size_t t; (t = next++) < tiles && ok;) {
+                if (mark.empty()) {
+                    mark.assign(N, -1);
+                    slot.assign(N, 0);
+                }
+                fn(t, mark, slot);
+            }
+        } catch (const std::bad_alloc&) {
+            ok = false;
+        }
+    };
+    std::vector<std::thread> pool;
+    for (size_t i = 1; i < std::min<size_t>(8, tiles / 8); i++) {
+        try {
+            pool.emplace_back(work);
+        } catch (const std::system_error&) {
+            break;                       // fewer threads do the same
+        }
+    }
+    work();
+    for (std::thread& t : pool) t.join();
+    return ok;
+}
+
+}  // namespace
+
 int tiles_create(mplb_case* c) {
     const Mesh& m = c->mesh;
     const bool thermal = c->fc[1].present && c->update[1], fp64 = c->scalar_bytes == 8;
     if (!c->passes || m.N > 1 << 20 || m.bd.size() > (size_t)kTileLists) return 0;
     const int cap = fp64 ? TileOps<double>::max_nodes(m.lbmodel, thermal) : TileOps<float>::max_nodes(m.lbmodel, thermal);
-    const int H = thermal ? 3 : 2, extra = c->fc[0].mp.surf ? 1 : 0, Q = m.Q;
-    Plan p = choose(c, cap, thermal, fp64, extra);
-    // MPLB_TILES=bx,by,bz,steps sets the plan (steps 0: fused passes), for tests and timing sweeps
-    if (const char* env = std::getenv("MPLB_TILES")) {
-        if (std::sscanf(env, "%d,%d,%d,%d", &p.b[0], &p.b[1], &p.b[2], &p.steps) != 4) p.steps = 0;
-        for (int d = 0; d < 3; d++) p.b[d] = std::max(1, p.b[d]);
-    }
+    const int H = thermal ? 3 : 2, extra = c->fc[0].mp.surf ? 1 : 0;
+    const int n[3] = {m.nx, m.ny, m.nz};
+    const std::vector<int> sizes = {1, 2, 3, 4, 5, 6, 8, 10, 12, 14, 16, 20, 24, 32, 48, 64, 128};
+    int cus = 256;
+    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->opts.device);
+    TilePlan p = tile_choose(c, sizes, 0.85 * passes_us(c, thermal, fp64), [&](const TilePlan& q) {
+        return plan_us(q, n, thermal, m.d == 3, fp64, cap, extra, cus);
+    });
+    tile_override(&p);
     if (p.steps <= 0) return 0;
-    const int D = H * p.steps + extra;
+    const bool lists[2] = {c->order[0] != nullptr, c->order[1] != nullptr};
+    const int rc = tile_tables(c, p, H * p.steps + extra, cap, lists);
+    if (rc || !c->tiles) return rc;
+    // second copies of the macroscopic fields: a launch reads one set and writes the other
+    const int comps[7] = {1, 1, 3, 3, 3, 1, 1};
+    for (int i = 0; i < 7; i++) TCHK(c, hipMalloc(&c->alt[i], c->scalar_bytes * comps[i] * m.N));
+    return 0;
+}
+
+int tile_tables(mplb_case* c, const TilePlan& p, int D, int cap, const bool lists[2]) {
+    const Mesh& m = c->mesh;
+    const int Q = m.Q;
+    const bool thermal = c->fc[1].present && c->update[1];
     // the g lists of fixedT nodes, whose condition reads the population that their inner
     // neighbour pulled: it must not come from a list applied before
     std::vector<int> list[2];
     for (int f = 0; f < 2; f++) {
         list[f].assign(m.N, 255);
-        if (!c->order[f]) continue;
+        if (!lists[f]) continue;
         for (size_t b = 0; b < m.bd.size(); b++) {
             const int t = c->fc[f].bctype[b];
             if (t == BD_BBACK || t == BD_FT || t == BD_FRDT)
@@ -176,55 +222,59 @@ int tiles_create(mplb_case* c) {
                                 own.back().push_back((int)(i + (int64_t)j * nx + (int64_t)k * nx * ny));
                 }
     }
-    std::vector<int> mark(m.N, -1), slot(m.N, 0);
-    std::vector<std::vector<int>> local(own.size()), level(own.size());   // nodes, and their depths
-    size_t largest = 0;
-    for (size_t t = 0; t < own.size(); t++) {
-        std::vector<int>&nodes = local[t], &depth = level[t];
-        int at = 0;
+    // tile t's nodes from local[t * cap], level d ending at ends[t * (D + 1) + d]
+    if (own.size() * (size_t)cap > size_t(1) << 26 || D > 250) return 0;
+    const std::unique_ptr<int[]> local(new int[own.size() * cap]), ends(new int[own.size() * (D + 1)]);
+    std::atomic<bool> fits{true};
+    const bool listed = over_tiles(own.size(), m.N, [&](size_t t, std::vector<int>& mark, std::vector<int>&) {
+        int *nodes = &local[t * cap], *end = &ends[t * (D + 1)], n = 0;
         auto add = [&](int64_t id) {
             if (id < 0 || mark[id] == (int)t) return;
             mark[id] = (int)t;
-            slot[id] = (int)nodes.size();
-            nodes.push_back((int)id);
-            depth.push_back(at);
+            if (n < cap) nodes[n] = (int)id;
+            n++;
         };
         for (int id : own[t]) add(id);
-        size_t from = 0;
-        for (int d = 0; d < D; d++) {
-            const size_t to = nodes.size();
-            at = d + 1;
-            for (size_t i = from; i < to; i++) {
+        int from = 0;
+        for (int d = 0; d <= D && fits; d++) {
+            if (n > cap) fits = false;
+            if (!fits) break;
+            // (in memory order, so that a wavefront's loads share sectors)
+            std::sort(nodes + from, nodes + n);
+            const int to = end[d] = n;
+            for (int i = from; i < to && d < D; i++) {
                 const int64_t id = nodes[i];
                 for (int k = 0; k < Q; k++) add(m.nb[id * Q + k]);
                 if (!fixed_t(id)) continue;
                 for (int k = 0; k < Q; k++) {
                     const int64_t in = m.nb[id * Q + tile_reverse(m, k)];
                     if (m.nb[id * Q + k] != -1 || in == -1) continue;
-                    if (list[1][in] < list[1][id]) return 0;
+                    if (list[1][in] < list[1][id]) fits = false;
                     add(m.nb[in * Q + k]);
                 }
             }
             from = to;
         }
-        largest = std::max(largest, nodes.size());
-        if (largest > (size_t)cap) return 0;
-    }
+    });
+    if (!listed || !fits) return 0;
+    size_t largest = 0;
+    for (size_t t = 0; t < own.size(); t++) largest = std::max(largest, (size_t)ends[t * (D + 1) + D]);
     const size_t total = own.size() * largest;
-    if (total > size_t(1) << 23 || D > 250) return 0;
-    const bool any_fixed = thermal && c->order[1];
+    if (total > size_t(1) << 23) return 0;
+    const bool any_fixed = thermal && lists[1];
     std::vector<int16_t> nb(total * Q, -1), inner(any_fixed ? total * Q : 0, 0);
     std::vector<int> gid(total, 0), meta(total, 255 << 24), draw(draws.empty() ? 0 : total);
-    for (size_t t = 0; t < own.size(); t++) {
-        const std::vector<int>& nodes = local[t];
-        const int stamp = (int)(own.size() + t);
-        for (size_t i = 0; i < nodes.size(); i++) {
-            mark[nodes[i]] = stamp;
-            slot[nodes[i]] = (int)i;
+    const bool filled = over_tiles(own.size(), m.N, [&](size_t t, std::vector<int>& mark, std::vector<int>& slot) {
+        const int *nodes = &local[t * cap], *end = &ends[t * (D + 1)];
+        const int count = end[D];
+        for (int i = 0; i < count; i++) {
+            mark[nodes[i]] = (int)t;
+            slot[nodes[i]] = i;
         }
         // neighbours outside the tile belong to its rim and are never followed
-        auto at = [&](int32_t n) { return (int16_t)(n != -1 && mark[n] == stamp ? slot[n] : -1); };
-        for (size_t i = 0; i < nodes.size(); i++) {
+        auto at = [&](int32_t n) { return (int16_t)(n != -1 && mark[n] == (int)t ? slot[n] : -1); };
+        for (int i = 0, depth = 0; i < count; i++) {
+            while (i >= end[depth]) depth++;
             const int64_t id = nodes[i];
             const size_t e = t * largest + i;
             gid[e] = (int)id;
@@ -242,10 +292,11 @@ int tiles_create(mplb_case* c) {
                 }
             }
             meta[e] = list[0][id] | list[1][id] << 8 | (m.onbnd[id] == 0 ? 1 << 16 : 0) | (full ? 1 << 17 : 0) |
-                      level[t][i] << 24;
+                      depth << 24;
             if (!draws.empty()) draw[e] = draws[id];
         }
-    }
+    });
+    if (!filled) return 0;
     Tiles* s = new Tiles();
     c->tiles = s;
     auto put = [&](const void* src, size_t bytes, const void** dst) -> int {
@@ -267,9 +318,6 @@ int tiles_create(mplb_case* c) {
     s->t.total = (int64_t)total;
     s->nodes = (int)largest;
     s->steps = p.steps;
-    // second copies of the macroscopic fields: a launch reads one set and writes the other
-    const int comps[7] = {1, 1, 3, 3, 3, 1, 1};
-    for (int i = 0; i < 7; i++) TCHK(c, hipMalloc(&c->alt[i], c->scalar_bytes * comps[i] * m.N));
     return 0;
 }
 
