@@ -73,4 +73,32 @@ __device__ inline int64_t downstream(const A& a, const NodePos& p, int q) {
     return (int64_t)(p.X[1 + L::t.c[q][0]] + p.Y[1 + L::t.c[q][1]] + p.Z[1 + L::t.c[q][2]]);
 }
 
+// All upstream / downstream nodes in one branch: a branch for each neighbour keeps a node's
+// loads from going out together.
+template <class L, class A>
+__device__ inline void upstreams(const A& a, const NodePos& p, unsigned* up) {
+    if (p.table) {
+#pragma unroll
+        for (int q = 0; q < L::Q; q++) {
+            const int s = a.nb[q * a.N + p.id];
+            up[q] = s == -1 ? (unsigned)p.id : (unsigned)s;
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < L::Q; q++) up[q] = p.X[1 - L::t.c[q][0]] + p.Y[1 - L::t.c[q][1]] + p.Z[1 - L::t.c[q][2]];
+    }
+}
+
+template <class L, class A>
+__device__ inline void downstreams(const A& a, const NodePos& p, int* dn) {
+    if (p.table) {
+#pragma unroll
+        for (int q = 0; q < L::Q; q++) dn[q] = a.nb[L::t.rev[q] * a.N + p.id];
+    } else {
+#pragma unroll
+        for (int q = 0; q < L::Q; q++)
+            dn[q] = (int)(p.X[1 + L::t.c[q][0]] + p.Y[1 + L::t.c[q][1]] + p.Z[1 + L::t.c[q][2]]);
+    }
+}
+
 }  // namespace mplb

@@ -94,24 +94,40 @@ struct FArgs {
     _Float16* rout;
 };
 
-template <typename S>
-__device__ inline float ld(const void* p, int64_t i, float shift) {
-    if constexpr (sizeof(S) == 2) {
-        return (float)((const _Float16*)p)[i] + shift;
+// Element i of an array.  With an int index (the pass kernels, kNarrow nodes at most) the byte
+// offset is one 32-bit value beside a scalar base; a 64-bit address is two or three vector
+// instructions and two registers for each of the thirty to ninety accesses of a node.  Other
+// types address in 64 bits (the thermal march's unsigned indices run over all populations).
+constexpr int64_t kNarrow = int64_t(1) << 30;
+
+template <typename T, typename I>
+__device__ inline T& el(T* p, I i) {
+    if constexpr (std::is_same<I, int>::value) {
+        using C = typename std::conditional<std::is_const<T>::value, const char, char>::type;
+        return *(T*)((C*)p + (unsigned)i * (unsigned)sizeof(T));
     } else {
-        return ((const float*)p)[i];
+        return p[i];
+    }
+}
+
+template <typename S, typename I>
+__device__ inline float ld(const void* p, I i, float shift) {
+    if constexpr (sizeof(S) == 2) {
+        return (float)el((const _Float16*)p, i) + shift;
+    } else {
+        return el((const float*)p, i);
     }
 }
 
 // Population stores: NT = non-temporal (stores_nt has the rule)
-template <typename S, bool NT = true>
-__device__ inline void st(void* p, int64_t i, float v, float shift) {
+template <typename S, bool NT = true, typename I>
+__device__ inline void st(void* p, I i, float v, float shift) {
     if constexpr (sizeof(S) == 2) {
-        if constexpr (NT) __builtin_nontemporal_store((_Float16)(v - shift), (_Float16*)p + i);
-        else ((_Float16*)p)[i] = (_Float16)(v - shift);
+        if constexpr (NT) __builtin_nontemporal_store((_Float16)(v - shift), &el((_Float16*)p, i));
+        else el((_Float16*)p, i) = (_Float16)(v - shift);
     } else {
-        if constexpr (NT) __builtin_nontemporal_store(v, (float*)p + i);
-        else ((float*)p)[i] = v;
+        if constexpr (NT) __builtin_nontemporal_store(v, &el((float*)p, i));
+        else el((float*)p, i) = v;
     }
 }
 
@@ -137,10 +153,10 @@ constexpr float kRefMin = 6.103515625e-05f;     // smallest normal FP16 (R never
 
 // FP16 storage: w_q R of the node a population was stored at (FP16N), or the global
 // shift of population q (FP16S)
-template <class L, typename S>
-__device__ inline float f_wref(const FArgs& a, int64_t node, int q) {
+template <class L, typename S, typename I>
+__device__ inline float f_wref(const FArgs& a, I node, int q) {
     if constexpr (kNodeRef<S>) {
-        return (float)L::t.omega[q] * (float)a.rin[node];
+        return (float)L::t.omega[q] * (float)el(a.rin, node);
     } else if constexpr (sizeof(S) == 2) {
         return a.fshift[q];
     } else {
@@ -149,10 +165,10 @@ __device__ inline float f_wref(const FArgs& a, int64_t node, int q) {
 }
 
 // a stored f population; wref from f_wref
-template <typename S>
-__device__ inline float ldf(const void* p, int64_t i, float wref) {
+template <typename S, typename I>
+__device__ inline float ldf(const void* p, I i, float wref) {
     if constexpr (kNodeRef<S>) {
-        return fmaf((float)((const _Float16*)p)[i], wref, wref);
+        return fmaf((float)el((const _Float16*)p, i), wref, wref);
     } else {
         return ld<S>(p, i, wref);
     }
@@ -160,12 +176,12 @@ __device__ inline float ldf(const void* p, int64_t i, float wref) {
 
 // FP16N: writes node id's reference for the output level (the node's density, at least
 // kRefMin; NaN stays NaN) and returns it with its reciprocal; 0 in the other modes
-template <typename S>
-__device__ inline float put_ref(const FArgs& a, int64_t id, float rho, float& rinv) {
+template <typename S, typename I>
+__device__ inline float put_ref(const FArgs& a, I id, float rho, float& rinv) {
     if constexpr (kNodeRef<S>) {
         const float r = (rho >= kRefMin || rho != rho) ? rho : kRefMin;
         const _Float16 h = (_Float16)r;
-        a.rout[id] = h;
+        el(a.rout, id) = h;
         const float R = (float)h;
         rinv = 1.f / R;
         return R;
@@ -176,12 +192,12 @@ __device__ inline float put_ref(const FArgs& a, int64_t id, float rho, float& ri
 }
 
 // FP16N: stores f population q of a node (reference R and 1 / R = rinv from put_ref)
-template <class L, bool NT = true>
-__device__ inline void stf_ref(void* p, int64_t i, int q, float v, float R, float rinv) {
+template <class L, bool NT = true, typename I>
+__device__ inline void stf_ref(void* p, I i, int q, float v, float R, float rinv) {
     const float wref = (float)L::t.omega[q] * R;
     const float dev = (v - wref) * ((float)(1.0 / L::t.omega[q]) * rinv);
-    if constexpr (NT) __builtin_nontemporal_store((_Float16)dev, (_Float16*)p + i);
-    else ((_Float16*)p)[i] = (_Float16)dev;
+    if constexpr (NT) __builtin_nontemporal_store((_Float16)dev, &el((_Float16*)p, i));
+    else el((_Float16*)p, i) = (_Float16)dev;
 }
 
 // psi = potential(rho, T) (potential.c:7-13) in FP32 with the loop-invariant factors taken
@@ -202,22 +218,15 @@ __device__ inline float fpot(const FArgs& a, float rho, float T) {
     return potential<float>(a.eos, rho, T);
 }
 
-// upstream nodes of a node's populations
-template <class L>
-__device__ inline void upstreams(const FArgs& a, const NodePos& p, unsigned* up) {
-#pragma unroll
-    for (int q = 0; q < L::Q; q++) up[q] = upstream<L>(a, p, q);
-}
-
 // REF: f stored against per-node references (FP16N); otherwise shift holds the storage
 // shifts
-template <class L, typename S, bool REF>
+template <class L, typename S, bool REF, typename I>
 __device__ inline void pull(const FArgs& a, const unsigned* up, const void* src, const float* shift, float* v) {
 #pragma unroll
     for (int q = 0; q < L::Q; q++) {
         const void* plane = (const char*)src + (size_t)q * a.P * sizeof(S);
-        if constexpr (REF && kNodeRef<S>) v[q] = ldf<S>(plane, up[q], f_wref<L, S>(a, up[q], q));
-        else v[q] = ld<S>(plane, up[q], shift[q]);
+        if constexpr (REF && kNodeRef<S>) v[q] = ldf<S>(plane, (I)up[q], f_wref<L, S>(a, (I)up[q], q));
+        else v[q] = ld<S>(plane, (I)up[q], shift[q]);
     }
 }
 
@@ -286,52 +295,52 @@ __device__ inline void bound_g(const FArgs& a, const NodePos& p, float* v) {
     else if (code == FB_FT || code == FB_FRDT) fixed_temperature<L, S>(a, p, v, code, ((a.draw >> (bc >> 4)) & 1) != 0);
 }
 
-template <class L, typename S>
+template <class L, typename S, typename I>
 __device__ inline void pull_f(const FArgs& a, const NodePos& p, float* v) {
     unsigned up[L::Q];
     upstreams<L>(a, p, up);
-    pull<L, S, kNodeRef<S>>(a, up, a.fin, a.fshift, v);
+    pull<L, S, kNodeRef<S>, I>(a, up, a.fin, a.fshift, v);
     bound_f<L>(a, p, v);
 }
 
-template <class L, typename S>
+template <class L, typename S, typename I>
 __device__ inline void pull_g(const FArgs& a, const NodePos& p, float* v) {
     unsigned up[L::Q];
     upstreams<L>(a, p, up);
-    pull<L, S, false>(a, up, a.gin, a.gshift, v);
+    pull<L, S, false, I>(a, up, a.gin, a.gshift, v);
     bound_g<L, S>(a, p, v);
 }
 
 // Both fields, every load issued before a boundary condition branches: pulled one after the
 // other, the second field's loads wait for the first one's (a chain of latencies on the
 // nodes that read the neighbour table).
-template <class L, typename S>
+template <class L, typename S, typename I>
 __device__ inline void pull_fg(const FArgs& a, const NodePos& p, float* v, float* w) {
     unsigned up[L::Q];
     upstreams<L>(a, p, up);
-    pull<L, S, kNodeRef<S>>(a, up, a.fin, a.fshift, v);
-    pull<L, S, false>(a, up, a.gin, a.gshift, w);
+    pull<L, S, kNodeRef<S>, I>(a, up, a.fin, a.fshift, v);
+    pull<L, S, false, I>(a, up, a.gin, a.gshift, w);
     bound_f<L>(a, p, v);
     bound_g<L, S>(a, p, w);
 }
 
-// K1
-template <class L, typename S, bool THERMAL>
+// K1.  I: int (up to kNarrow nodes) or int64_t
+template <class L, typename S, bool THERMAL, typename I>
 __global__ void __launch_bounds__(256) k_fused_density(FArgs a) {
     const NodePos p = node_pos<L>(a);
     if (!p.valid) return;
     float v[L::Q];
     if constexpr (THERMAL) {
         float w[L::Q];
-        pull_fg<L, S>(a, p, v, w);
-        a.rho[p.id] = rho_sym<L, float>(v);
-        a.sumg[p.id] = rho_sym<L, float>(w);
+        pull_fg<L, S, I>(a, p, v, w);
+        el(a.rho, (I)p.id) = rho_sym<L, float>(v);
+        el(a.sumg, (I)p.id) = rho_sym<L, float>(w);
     } else {
-        pull_f<L, S>(a, p, v);
+        pull_f<L, S, I>(a, p, v);
         const float rho = rho_sym<L, float>(v);
-        const float T = a.Tuniform ? a.Tconst : a.Told[p.id];
-        a.psi[p.id] = fpot(a, rho, T);
-        if (a.out_rho) a.out_rho[p.id] = rho;
+        const float T = a.Tuniform ? a.Tconst : el(a.Told, (I)p.id);
+        el(a.psi, (I)p.id) = fpot(a, rho, T);
+        if (a.out_rho) el(a.out_rho, (I)p.id) = rho;
     }
 }
 
@@ -373,39 +382,54 @@ __device__ inline void heat_axis(float Tp, float Tm, float rp, float rm, float u
     divU += dU;
 }
 
-// KH: heatSource.c:26-170 with macroTemperature (myMRTTemperature.c:16-30)
-template <class L>
+// KH: heatSource.c:26-170 with macroTemperature (myMRTTemperature.c:16-30).  Bound by HBM and
+// L2 (rho, T and U of seven nodes): 160^3 47 -> 39 us, 128 x 128 x 384 column 66.8 -> 54.3 with
+// the loads of all axes together.
+template <class L, typename I>
 __global__ void __launch_bounds__(256) k_fused_heat(FArgs a) {
     const NodePos p = node_pos<L>(a);
     if (!p.valid) return;
-    const int64_t id = p.id;
-    const float rho = a.rho[id], Told = a.Told[id];
+    const I id = (I)p.id;
+    const float rho = el(a.rho, id), Told = el(a.Told, id);
     float dot = 0.f, divU = 0.f;
+    if (!p.table) {
+        // every link is there: one branch for the node, so that its loads go out together
+        const I lo[3] = {(I)(p.X[0] + p.Y[1] + p.Z[1]), (I)(p.X[1] + p.Y[0] + p.Z[1]), (I)(p.X[1] + p.Y[1] + p.Z[0])};
+        const I hi[3] = {(I)(p.X[2] + p.Y[1] + p.Z[1]), (I)(p.X[1] + p.Y[2] + p.Z[1]), (I)(p.X[1] + p.Y[1] + p.Z[2])};
 #pragma unroll
-    for (int ax = 0; ax < L::D; ax++) {
-        // a = nb[id][fd_plus] = x + e_ax, b = nb[id][fd_minus] = x - e_ax
-        const int64_t na = downstream<L>(a, p, L::fd_minus[ax]);
-        const int64_t nbb = downstream<L>(a, p, L::fd_plus[ax]);
-        const float* Uax = a.Uold + ax * a.N;
-        if (na != -1 && nbb != -1) {
-            heat_axis(a.Told[na], a.Told[nbb], a.rho[na], a.rho[nbb], Uax[na], Uax[nbb], dot, divU);
-        } else {
-            float gT, gR, dU;
-            if (na == -1 && nbb != -1) {
-                gT = Told - a.Told[nbb];
-                gR = 1.0f / rho - 1.0f / a.rho[nbb];
-                dU = Uax[id] - Uax[nbb];
-            } else if (na != -1 && nbb == -1) {
-                gT = a.Told[na] - Told;
-                gR = 1.0f / a.rho[na] - 1.0f / rho;
-                dU = Uax[na] - Uax[id];
+        for (int ax = 0; ax < L::D; ax++) {
+            const float* Uax = a.Uold + ax * a.N;
+            heat_axis(el(a.Told, hi[ax]), el(a.Told, lo[ax]), el(a.rho, hi[ax]), el(a.rho, lo[ax]), el(Uax, hi[ax]),
+                      el(Uax, lo[ax]), dot, divU);
+        }
+    } else {
+#pragma unroll
+        for (int ax = 0; ax < L::D; ax++) {
+            // a = nb[id][fd_plus] = x + e_ax, b = nb[id][fd_minus] = x - e_ax
+            const int na = (int)downstream<L>(a, p, L::fd_minus[ax]);
+            const int nbb = (int)downstream<L>(a, p, L::fd_plus[ax]);
+            const float* Uax = a.Uold + ax * a.N;
+            if (na != -1 && nbb != -1) {
+                heat_axis(el(a.Told, (I)na), el(a.Told, (I)nbb), el(a.rho, (I)na), el(a.rho, (I)nbb), el(Uax, (I)na), el(Uax, (I)nbb),
+                          dot, divU);
             } else {
-                gT = 0.f;
-                gR = 0.f;
-                dU = 0.f;
+                float gT, gR, dU;
+                if (na == -1 && nbb != -1) {
+                    gT = Told - a.Told[nbb];
+                    gR = 1.0f / rho - 1.0f / a.rho[nbb];
+                    dU = Uax[id] - Uax[nbb];
+                } else if (na != -1 && nbb == -1) {
+                    gT = a.Told[na] - Told;
+                    gR = 1.0f / a.rho[na] - 1.0f / rho;
+                    dU = Uax[na] - Uax[id];
+                } else {
+                    gT = 0.f;
+                    gR = 0.f;
+                    dU = 0.f;
+                }
+                dot += gT * gR;
+                divU += dU;
             }
-            dot += gT * gR;
-            divU += dU;
         }
     }
     const float s = heat_tail<L>(a, rho, Told, dot, divU);
@@ -413,15 +437,15 @@ __global__ void __launch_bounds__(256) k_fused_heat(FArgs a) {
     float Sv;
     if (a.gmodel == 1) {
         Sv = s;
-        T = a.sumg[id] + 0.5f * Sv;
+        T = el(a.sumg, id) + 0.5f * Sv;
     } else {
-        const float old = a.first_call ? 0.f : a.S[id];
+        const float old = a.first_call ? 0.f : el(a.S, id);
         Sv = s + 0.5f * (s - old);
-        T = a.sumg[id];
+        T = el(a.sumg, id);
     }
-    a.S[id] = Sv;
-    a.Tnew[id] = T;
-    a.psi[id] = fpot(a, rho, T);
+    el(a.S, id) = Sv;
+    el(a.Tnew, id) = T;
+    el(a.psi, id) = fpot(a, rho, T);
 }
 
 // Interaction force (interactionForce.c:47-79), velocity (liMRTVelocity.c /
@@ -626,32 +650,49 @@ __device__ inline void collide_g(const FArgs& a, float* v, float T, float Sv, co
     populations_add_sym<L, float>(n, v);
 }
 
-// K2
-template <class L, typename S, bool THERMAL, bool NT>
+// psi at the downstream nodes of node p, whose own is psin[0].  One branch for the node: with
+// a branch for each neighbour the loads do not go out together.
+template <class L, typename I>
+__device__ inline void psi_stencil(const FArgs& a, const NodePos& p, float* psin) {
+    if (p.table) {
+        int n[L::Q];
+#pragma unroll
+        for (int q = 1; q < L::Q; q++) n[q] = el(a.nb + L::t.rev[q] * a.N, (I)p.id);
+#pragma unroll
+        for (int q = 1; q < L::Q; q++) psin[q] = n[q] == -1 ? psin[0] : el(a.psi, (I)n[q]);
+    } else {
+#pragma unroll
+        for (int q = 1; q < L::Q; q++)
+            psin[q] = el(a.psi, (I)(p.X[1 + L::t.c[q][0]] + p.Y[1 + L::t.c[q][1]] + p.Z[1 + L::t.c[q][2]]));
+    }
+}
+
+// K2.  Bound by HBM and by the VALU together (populations read and written once, psi from L2;
+// about 500 instructions a node): with 32-bit indices and every load before the first branch
+// 201 x 150 x 180 FP32 151 -> 137 us, FP16S 105 -> 99, FP16N 126 -> 113; 160^3 FP16N with heat
+// transfer 157 -> 150; 50 x 50 x 160 column FP32 38.5 -> 34.1 (launches timed one by one).
+template <class L, typename S, bool THERMAL, bool NT, typename I>
 __global__ void __launch_bounds__(256) k_fused_collide(FArgs a) {
     const NodePos p = node_pos<L>(a);
     if (!p.valid) return;
-    const int64_t id = p.id, N = a.N;
-    float v[L::Q], w[THERMAL ? L::Q : 1];
-    if constexpr (THERMAL) pull_fg<L, S>(a, p, v, w);
-    else pull_f<L, S>(a, p, v);
+    const I id = (I)p.id;
+    const int64_t N = a.N;
+    float v[L::Q], w[THERMAL ? L::Q : 1], psin[L::Q];
+    unsigned up[L::Q];
+    upstreams<L>(a, p, up);
+    pull<L, S, kNodeRef<S>, I>(a, up, a.fin, a.fshift, v);
+    if constexpr (THERMAL) pull<L, S, false, I>(a, up, a.gin, a.gshift, w);
+    const float psic = psin[0] = el(a.psi, id);
+    const bool interior = !p.table || el(a.onbnd, id) == 0;
+    psi_stencil<L, I>(a, p, psin);
+    bound_f<L>(a, p, v);
+    if constexpr (THERMAL) bound_g<L, S>(a, p, w);
     const float rho = rho_sym<L, float>(v);
-    const float psic = a.psi[id];
-    const bool interior = !p.table || a.onbnd[id] == 0;
-    float psin[L::Q];
-    psin[0] = psic;
-    if (interior || a.surf) {
-#pragma unroll
-        for (int q = 1; q < L::Q; q++) {
-            const int64_t n = downstream<L>(a, p, q);
-            psin[q] = n == -1 ? psic : a.psi[n];
-        }
-    }
     bool full = true;
     if (a.surf && p.table) {
 #pragma unroll
         for (int q = 1; q < L::Q; q++)
-            if (a.nb[q * N + id] == -1) full = false;
+            if (el(a.nb + q * N, id) == -1) full = false;
     }
     float U[3], Fi[3], Ft[3];
     collide_node<L>(a, v, rho, psin, interior, full, U, Fi, Ft);
@@ -659,31 +700,31 @@ __global__ void __launch_bounds__(256) k_fused_collide(FArgs a) {
         float rinv;
         const float R = put_ref<S>(a, id, rho, rinv);
 #pragma unroll
-        for (int q = 0; q < L::Q; q++) stf_ref<L, NT>(a.fout, q * a.P + id, q, v[q], R, rinv);
+        for (int q = 0; q < L::Q; q++) stf_ref<L, NT>((_Float16*)a.fout + q * a.P, id, q, v[q], R, rinv);
     } else {
 #pragma unroll
-        for (int q = 0; q < L::Q; q++) st<S, NT>(a.fout, q * a.P + id, v[q], a.fshift[q]);
+        for (int q = 0; q < L::Q; q++) st<S, NT>((S*)a.fout + q * a.P, id, v[q], a.fshift[q]);
     }
 
     if constexpr (THERMAL) {
-        collide_g<L>(a, w, a.Tnew[id], a.S[id], U);
+        collide_g<L>(a, w, el(a.Tnew, id), el(a.S, id), U);
 #pragma unroll
-        for (int q = 0; q < L::Q; q++) st<S, NT>(a.gout, q * a.P + id, w[q], a.gshift[q]);
-        a.Unew[id] = U[0];
-        a.Unew[N + id] = U[1];
-        a.Unew[2 * N + id] = U[2];
+        for (int q = 0; q < L::Q; q++) st<S, NT>((S*)a.gout + q * a.P, id, w[q], a.gshift[q]);
+        el(a.Unew, id) = U[0];
+        el(a.Unew + N, id) = U[1];
+        el(a.Unew + 2 * N, id) = U[2];
     }
     if (a.out_U) {
-        a.out_U[id] = U[0];
-        a.out_U[N + id] = U[1];
-        a.out_U[2 * N + id] = U[2];
+        el(a.out_U, id) = U[0];
+        el(a.out_U + N, id) = U[1];
+        el(a.out_U + 2 * N, id) = U[2];
     }
-    if (a.out_rho) a.out_rho[id] = rho;
+    if (a.out_rho) el(a.out_rho, id) = rho;
     if (a.out_Fi) {
 #pragma unroll
         for (int d = 0; d < 3; d++) {
-            a.out_Fi[d * N + id] = Fi[d];
-            a.out_Ft[d * N + id] = Ft[d];
+            el(a.out_Fi + d * N, id) = Fi[d];
+            el(a.out_Ft + d * N, id) = Ft[d];
         }
     }
 }
@@ -1781,8 +1822,8 @@ __global__ void __launch_bounds__(256) k_fused_materialize(FArgs a, float* out) 
     const NodePos p = node_pos<L>(a);
     if (!p.valid) return;
     float v[L::Q];
-    if (G) pull_g<L, S>(a, p, v);
-    else pull_f<L, S>(a, p, v);
+    if (G) pull_g<L, S, int64_t>(a, p, v);
+    else pull_f<L, S, int64_t>(a, p, v);
 #pragma unroll
     for (int q = 0; q < L::Q; q++) out[q * a.N + p.id] = v[q];
 }
@@ -1854,6 +1895,7 @@ struct Fused {
     float t_const = 0.f;
     int mtx = 0, mtiles = 0, mitems = 0, mper = 0, mzc = 0;
     bool nt = true;              // population stores are non-temporal
+    bool wide = false;           // the pass kernels index nodes in 64 bits
     float* S = nullptr;          // tiled lattices: the second copy of the heat source
     FTileArgs last{};            // arguments of the last tile launch
 };
@@ -1989,16 +2031,35 @@ void launch_tmarch(mplb_case* c, const FArgs& a) {
     }
 }
 
+// fn with a value of the index type that reaches every node
+template <class Fn>
+void with_index(mplb_case* c, Fn fn) {
+    if (F(c)->wide) fn(int64_t(0));
+    else fn(0);
+}
+
+template <class L, typename S, bool THERMAL>
+void launch_density(mplb_case* c, const FArgs& a) {
+    with_index(c, [&](auto i) {
+        k_fused_density<L, S, THERMAL, decltype(i)><<<(unsigned)a.nblocks, 256, 0, c->stream>>>(a);
+    });
+}
+
+template <class L>
+void launch_heat(mplb_case* c, const FArgs& a) {
+    with_index(c, [&](auto i) { k_fused_heat<L, decltype(i)><<<(unsigned)a.nblocks, 256, 0, c->stream>>>(a); });
+}
+
 template <class L, typename S, bool THERMAL>
 void launch_collide(mplb_case* c, const FArgs& a) {
-    const dim3 grid((unsigned)a.nblocks);
-    if (F(c)->nt) k_fused_collide<L, S, THERMAL, true><<<grid, 256, 0, c->stream>>>(a);
-    else k_fused_collide<L, S, THERMAL, false><<<grid, 256, 0, c->stream>>>(a);
+    with_index(c, [&](auto i) {
+        if (F(c)->nt) k_fused_collide<L, S, THERMAL, true, decltype(i)><<<(unsigned)a.nblocks, 256, 0, c->stream>>>(a);
+        else k_fused_collide<L, S, THERMAL, false, decltype(i)><<<(unsigned)a.nblocks, 256, 0, c->stream>>>(a);
+    });
 }
 
 template <class L, typename S>
 void launch_step(mplb_case* c, FArgs a, bool thermal, bool outputs) {
-    const dim3 grid((unsigned)a.nblocks), block(256);
     if (outputs) {
         a.out_rho = (float*)c->rho;
         a.out_Fi = (float*)c->Fi;
@@ -2008,13 +2069,13 @@ void launch_step(mplb_case* c, FArgs a, bool thermal, bool outputs) {
     if (thermal && F(c)->tmarch) {
         launch_tmarch<L, S, false>(c, a);
     } else if (thermal) {
-        k_fused_density<L, S, true><<<grid, block, 0, c->stream>>>(a);
-        k_fused_heat<L><<<grid, block, 0, c->stream>>>(a);
+        launch_density<L, S, true>(c, a);
+        launch_heat<L>(c, a);
         launch_collide<L, S, true>(c, a);
     } else if (F(c)->march) {
         launch_march<L, S, false>(c, a);
     } else {
-        k_fused_density<L, S, false><<<grid, block, 0, c->stream>>>(a);
+        launch_density<L, S, false>(c, a);
         launch_collide<L, S, false>(c, a);
     }
 }
@@ -2042,7 +2103,6 @@ struct Ev {
 
 template <class L, typename S>
 void launch_step_timed(mplb_case* c, FArgs a, bool thermal, bool outputs) {
-    const dim3 grid((unsigned)a.nblocks), block(256);
     if (outputs) {
         a.out_rho = (float*)c->rho;
         a.out_Fi = (float*)c->Fi;
@@ -2056,11 +2116,11 @@ void launch_step_timed(mplb_case* c, FArgs a, bool thermal, bool outputs) {
     } else if (thermal) {
         {
             Ev e(c, 7);
-            k_fused_density<L, S, true><<<grid, block, 0, c->stream>>>(a);
+            launch_density<L, S, true>(c, a);
         }
         {
             Ev e(c, 5);
-            k_fused_heat<L><<<grid, block, 0, c->stream>>>(a);
+            launch_heat<L>(c, a);
         }
         Ev e(c, 6);
         launch_collide<L, S, true>(c, a);
@@ -2070,7 +2130,7 @@ void launch_step_timed(mplb_case* c, FArgs a, bool thermal, bool outputs) {
     } else {
         {
             Ev e(c, 7);
-            k_fused_density<L, S, false><<<grid, block, 0, c->stream>>>(a);
+            launch_density<L, S, false>(c, a);
         }
         Ev e(c, 6);
         launch_collide<L, S, false>(c, a);
@@ -2390,15 +2450,15 @@ bool in_cache(const Mesh& m, const Fused& z, size_t scalar) {
 // populations twice but leave no lane idle: a march's wavefronts are rows of 64 sites, so on
 // Nx of fill = Nx / (64 x columns) the rest idles.  Per step, single pass against passes:
 //   FP32       0.346 against 0.445 ms on 320 x 200^2 (fill 1), 0.315 / 0.316 on 208^3 (0.81),
-//              0.333 / 0.287 on 200^3 (0.78), 0.195 / 0.145 on 66 x 200 x 300 (0.52).  Rows that
+//              0.333 / 0.282 on 200^3 (0.78), 0.195 / 0.145 on 66 x 200 x 300 (0.52).  Rows that
 //              share 64-byte sectors need more (330 x 200^2, 0.86: 0.532 / 0.465; 180^3, 0.94:
 //              equal; 250^3, 0.98: 0.524 / 0.551).  In cache the passes' launches and psi
 //              cost more than the lanes (130^3, 0.68: 65 / 84 us; 75 x 90 x 120, 0.59: 31 / 36).
-//   FP16S      0.237 / 0.292 on 320 x 200^2, 91 / 96 us on 160^3 (0.83), 0.230 / 0.207 on 208^3,
+//   FP16S      0.237 / 0.292 on 320 x 200^2, 93.5 / 94.3 us on 160^3 (0.83), 0.230 / 0.207 on 208^3,
 //              0.151 / 0.130 on 201 x 150 x 180 (0.79).
-//   FP16N      0.317 / 0.353 on 320 x 200^2, 0.196 / 0.191 on 190^3 (0.99), 0.390 / 0.378 on 240^3
+//   FP16N      0.317 / 0.353 on 320 x 200^2, 0.197 / 0.181 on 190^3 (0.99), 0.390 / 0.378 on 240^3
 //              (0.94), 0.263 / 0.225 on 200^3: the references' loads make its pulls dear.
-//   thermal    FP32 0.863 / 1.052 on 320 x 200^2, 0.335 / 0.353 on 160^3, 0.872 / 0.753 on 208^3,
+//   thermal    FP32 0.863 / 1.052 on 320 x 200^2, 0.334 / 0.342 on 160^3, 0.537 / 0.577 on 192^3, 0.872 / 0.753 on 208^3,
 //              0.551 / 0.480 on 201 x 150 x 180; with FP16 storage the three passes are faster
 //              everywhere (FP16S 255^3 1.024 / 0.945, 160^3 0.305 / 0.230).
 // Below 2^20 nodes a march is a short chain of planes with most of the device idle: the passes
@@ -2409,7 +2469,7 @@ bool march_pays(const Mesh& m, const Fused& z, size_t scalar) {
     const bool sectors = m.nx * scalar % 64 == 0;
     if (!z.thermal && !z.half) return in_cache(m, z, scalar) || fill >= (sectors ? 0.8 : 0.9);
     if (z.thermal && z.half) return false;
-    return m.N >= 1 << 20 && fill >= (z.noderef ? 0.95 : 0.83);
+    return m.N >= 1 << 20 && fill >= (z.noderef ? 1.0 : 0.83);
 }
 
 // Non-temporal or ordinary stores of the new populations.  Non-temporal ones are best when
@@ -2635,6 +2695,9 @@ int fused_create(mplb_case* c) {
         }
     }
     z->nt = stores_nt(m, *z, sb);
+    // (MPLB_INDEX64=1: whatever the size, for tests)
+    const char* ienv = std::getenv("MPLB_INDEX64");
+    z->wide = N > kNarrow || (ienv && std::strcmp(ienv, "1") == 0);
     FCHK(c, hipMalloc(&z->bcf, N));
     FCHK(c, hipMemcpy(z->bcf, bcf.data(), N, hipMemcpyHostToDevice));
     FCHK(c, hipMalloc(&z->bcg, N));
