@@ -434,22 +434,9 @@ int setup_passes(mplb_case* c) {
             }
         }
     }
-    // neighbours are computed from coordinates where the lattice is a box in box order; a
-    // lattice read from files may have odd links or listed nodes off the surface
-    bool box = m.structured;
-    if (box && !m.points.empty()) {
-        const int64_t nxy = (int64_t)m.nx * m.ny;
-        for (int64_t id = 0; id < m.N && box; id++) {
-            const int i = (int)(id % m.nx), j = (int)((id / m.nx) % m.ny), k = (int)(id / nxy);
-            if (i == 0 || i == m.nx - 1 || j == 0 || j == m.ny - 1 || (m.d == 3 && (k == 0 || k == m.nz - 1))) continue;
-            box = !any[id];
-            for (int q = 0; q < m.Q && box; q++) {
-                const int* cq = m.lbmodel == 0 ? D2Q9::t.c[q] : D3Q15::t.c[q];
-                box = m.nb[id * m.Q + q] == id - cq[0] - (int64_t)cq[1] * m.nx - cq[2] * nxy;
-            }
-        }
-    }
-    c->pass_faces = box ? odd_faces(m, any) : kAllTable;
+    // neighbours are computed from coordinates where the lattice is a box in box order, with
+    // the odd links and the listed nodes on its surface
+    c->pass_faces = m.structured && plain_inside(m, any) ? odd_faces(m, any) : kAllTable;
     for (int f = 0; f < 2; f++) {
         if (!lists[f]) continue;
         HIPCHK(c, hipMalloc(&c->order[f], m.N));

@@ -340,4 +340,19 @@ int odd_faces(const Mesh& m, const std::vector<uint8_t>& bc) {
     return best;
 }
 
+bool plain_inside(const Mesh& m, const std::vector<uint8_t>& bc) {
+    const int64_t nx = m.nx, nxy = nx * m.ny;
+    for (int k = m.d == 3 ? 1 : 0; k < (m.d == 3 ? m.nz - 1 : 1); k++)
+        for (int j = 1; j < m.ny - 1; j++)
+            for (int64_t id = 1 + j * nx + k * nxy; id < nx - 1 + j * nx + k * nxy; id++) {
+                if (bc[id]) return false;
+                if (m.points.empty()) continue;
+                for (int q = 0; q < m.Q; q++) {
+                    const int* cq = m.lbmodel == 0 ? kC2[q] : kC3[q];
+                    if (m.nb[id * m.Q + q] != id - cq[0] - cq[1] * nx - cq[2] * nxy) return false;
+                }
+            }
+    return true;
+}
+
 }  // namespace mplb

@@ -43,4 +43,9 @@ inline int wrap_dup(int u, int n) { return u < 0 ? u + (n - 1) : (u > n - 1 ? u 
 // condition.
 int odd_faces(const Mesh& m, const std::vector<uint8_t>& bc);
 
+// Whether the nodes off the surface of a structured box need no table: none is marked in bc
+// and, in a lattice read from files, all their links go to the box neighbours (a built box
+// has no other links inside, but its lists can leave the surface: Y1 of the 2D generic box).
+bool plain_inside(const Mesh& m, const std::vector<uint8_t>& bc);
+
 }  // namespace mplb
