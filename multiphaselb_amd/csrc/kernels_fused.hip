@@ -42,7 +42,7 @@ struct FArgs {
     int64_t N, nxy;
     int64_t P;                                  // pitch between population planes (>= N)
     int nblocks;                                // 256-node blocks
-    int face_table;                             // faces (x0 x1 y0 y1 z0 z1 bits) read through the table
+    int face_table;                             // faces read through the table (boxidx.h)
     const int* nb;                              // [Q][N]
     const uint8_t* onbnd;
     int lists_f, lists_g;                       // nodes carry boundary codes
@@ -1882,7 +1882,7 @@ struct Fused {
     int last_draw = 0;             // fixedRandomT drawing lists of the last step (bit per slot)
     float rho0_built = 0.f;        // rho_0 the post-collision buffers were computed with
     int64_t P = 0;                 // population plane pitch
-    int face_table = 0;            // faces whose links differ from the periodic wrap
+    int face_table = 0;            // faces read through the table (kAllTable: every node)
     float fshift[15] = {0}, gshift[15] = {0};
     bool noderef = false;          // FP16N: f against per-node references
     _Float16* ra = nullptr;        // FP16N: per-node references of fa and fb
@@ -2611,7 +2611,7 @@ int fused_create(mplb_case* c) {
     {
         std::vector<uint8_t> bc(N);
         for (int64_t id = 0; id < N; id++) bc[id] = bcf[id] != FB_NONE || bcg[id] != FB_NONE;
-        z->face_table = odd_faces(m, bc);
+        z->face_table = plain_inside(m, bc) ? odd_faces(m, bc) : kAllTable;
     }
     // single-pass kernel: isothermal D3Q15 with every link the periodic wrap and no
     // boundary node (MPLB_FUSED_KERNEL=twopass keeps the two-pass kernels, =march takes the
