@@ -44,6 +44,25 @@ struct Timer {
 namespace mplb {
 struct HostStage;
 struct Tiles;
+
+// Makes dev the calling thread's device, and its own again at the end: events and
+// allocations belong to the current device, which need not be the case's.
+class DeviceScope {
+public:
+    explicit DeviceScope(int dev) {
+        if (hipGetDevice(&before_) != hipSuccess || before_ == dev) before_ = -1;
+        err = hipSetDevice(dev);
+    }
+    ~DeviceScope() {
+        if (before_ >= 0) (void)hipSetDevice(before_);
+    }
+    DeviceScope(const DeviceScope&) = delete;
+    DeviceScope& operator=(const DeviceScope&) = delete;
+    hipError_t err;
+
+private:
+    int before_ = -1;
+};
 }
 
 struct mplb_case {

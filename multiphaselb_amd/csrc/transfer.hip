@@ -87,6 +87,8 @@ void stage_free(mplb_case* c) {
 bool stage_wanted(int64_t N, int comps) { return (size_t)N * comps * sizeof(double) >= 2 * kBufBytes; }
 
 int stage_transfer(mplb_case* c, void* planes, int64_t N, int comps, double* host, bool to_device) {
+    const DeviceScope device(c->opts.device);
+    if (device.err != hipSuccess) return stage_fail(c, device.err, "field transfer");
     const int rc = stage_ready(c);
     if (rc) return rc;
     HostStage* s = c->stage;

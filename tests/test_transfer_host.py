@@ -1,0 +1,18 @@
+"""Host side of the large field transfers, on a HIP runtime without a GPU (_fakehip)."""
+from _fakehip import run
+
+OPEN = """
+c = M.Case(make_case_dir(d2(nx=723, ny=725, btype=3)), heat_transfer=False, device=0)
+a = np.random.default_rng(1).standard_normal(c._shape("U"))
+"""
+
+
+def test_transfers_do_not_depend_on_the_current_device(tmp_path):
+    """A case on device 0 while the caller's current device is 1: no event of another device is
+    recorded on the case's stream, and the caller's device stays."""
+    print(run(tmp_path, OPEN + """
+device.value = 1
+c.set("U", a)
+c.get("U")
+assert device.value == 1
+"""))
