@@ -861,7 +861,7 @@ int copy_field(mplb_case* c, const std::string& name, double* host, size_t n, bo
     if (field_layout(c, name, &d, &comps)) return fail(c, MPLB_E_ARG, "Unknown field " + name);
     const int64_t N = c->mesh.N;
     if (n != (size_t)(N * comps)) return fail(c, MPLB_E_ARG, "Field " + name + ": wrong element count");
-    if (stage_wanted(N, comps)) {
+    if (stage_wanted(c, N, comps)) {
         const int rc = stage_transfer(c, d, N, comps, host, to_device);
         if (!rc && to_device && (name == "rho" || name == "T")) c->psi_valid = false;
         return rc;

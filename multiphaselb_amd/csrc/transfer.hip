@@ -62,18 +62,6 @@ static int stage_fail(mplb_case* c, hipError_t e, const char* what) {
     return MPLB_E_HIP;
 }
 
-static int stage_ready(mplb_case* c) {
-    if (!c->stage) c->stage = new HostStage();
-    HostStage* s = c->stage;
-    for (int i = 0; i < kBuffers; i++) {
-        hipError_t e = hipSuccess;
-        if (!s->buf[i]) e = hipHostMalloc((void**)&s->buf[i], kBufBytes, hipHostMallocDefault);
-        if (e == hipSuccess && !s->ev[i]) e = hipEventCreateWithFlags(&s->ev[i], hipEventDisableTiming);
-        if (e != hipSuccess) return stage_fail(c, e, "pinned transfer buffer");
-    }
-    return 0;
-}
-
 void stage_free(mplb_case* c) {
     if (!c->stage) return;
     for (int i = 0; i < kBuffers; i++) {
@@ -84,13 +72,25 @@ void stage_free(mplb_case* c) {
     c->stage = nullptr;
 }
 
-bool stage_wanted(int64_t N, int comps) { return (size_t)N * comps * sizeof(double) >= 2 * kBufBytes; }
+bool stage_wanted(mplb_case* c, int64_t N, int comps) {
+    if ((size_t)N * comps * sizeof(double) < 2 * kBufBytes) return false;
+    if (c->stage) return true;
+    const DeviceScope device(c->opts.device);
+    c->stage = new HostStage();
+    hipError_t e = device.err;
+    for (int i = 0; i < kBuffers && e == hipSuccess; i++) {
+        e = hipHostMalloc((void**)&c->stage->buf[i], kBufBytes, hipHostMallocDefault);
+        if (e == hipSuccess) e = hipEventCreateWithFlags(&c->stage->ev[i], hipEventDisableTiming);
+    }
+    if (e == hipSuccess) return true;
+    (void)hipGetLastError();        // (not an error of the next launch)
+    stage_free(c);
+    return false;
+}
 
 int stage_transfer(mplb_case* c, void* planes, int64_t N, int comps, double* host, bool to_device) {
     const DeviceScope device(c->opts.device);
     if (device.err != hipSuccess) return stage_fail(c, device.err, "field transfer");
-    const int rc = stage_ready(c);
-    if (rc) return rc;
     HostStage* s = c->stage;
     const int64_t total = N * comps, per = kBufBytes / sizeof(double);
     const int64_t chunks = (total + per - 1) / per;

@@ -16,3 +16,14 @@ c.set("U", a)
 c.get("U")
 assert device.value == 1
 """))
+
+
+def test_without_pinned_memory_fields_go_through_pageable_copies(tmp_path):
+    print(run(tmp_path, OPEN + """
+pinned_fails.value = 1
+c.set("U", a)
+assert np.array_equal(c.get("U"), a)
+pinned_fails.value = 0
+c.set("U", a)
+c.close()
+"""))
