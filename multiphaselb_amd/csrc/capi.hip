@@ -450,7 +450,7 @@ int setup_passes(mplb_case* c) {
                                            : PassOps<float>::march_plan(c->opts.device, m.nx, m.ny, m.nz, &c->march);
         if (e) return fail(c, MPLB_E_HIP, std::string("march plan: ") + hipGetErrorString((hipError_t)e));
     }
-    return tiles_create(c);
+    return 0;
 }
 
 template <typename T>
@@ -835,8 +835,16 @@ int init_t(mplb_case* c) {
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->initialized = true;
     c->snap_valid = false;
-    if (c->fused) return fused_after_init(c);
-    return 0;
+    if (c->fused) {
+        rc = fused_after_init(c);
+        if (rc) return rc;
+    }
+    // tiles are for cases that step: a case that is only opened does not wait for their tables
+    if (c->tiles_tried) return 0;
+    c->tiles_tried = true;
+    const DeviceScope device(c->opts.device);
+    HIPCHK(c, device.err);
+    return c->fused ? fused_tiles(c) : tiles_create(c);
 }
 
 int field_layout(const mplb_case* c, const std::string& name, void** dptr, int* comps) {

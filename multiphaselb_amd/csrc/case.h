@@ -114,6 +114,7 @@ struct mplb_case {
     // several steps per launch on small lattices (tiles.hip): rho, T, U, Fi, Ft, ss and psi
     // of the level being written
     mplb::Tiles* tiles = nullptr;
+    bool tiles_tried = false;                   // at the first init
     void* alt[7] = {nullptr};
 
     // fused structured-box path

@@ -13,18 +13,18 @@ SOURCE = r"""
 #include <new>
 extern "C" {
 int fake_device = 0, fake_pinned_fails = 0;
-long fake_mallocs = 0, fake_fail_from = -1;      // device allocations so far; those from this one on fail
+long fake_live = 0, fake_peak = 0, fake_most = -1;    // device allocations, and how many there may be
 size_t fake_new_limit = 0;                       // host allocations of more bytes fail (0: none)
 struct Dev { int device; };
 int hipGetDevice(int* d) { *d = fake_device; return 0; }
 int hipSetDevice(int d) { fake_device = d; return 0; }
 int hipDeviceGetAttribute(int* v, int, int) { *v = 256; return 0; }
 int hipMalloc(void** p, size_t n) {
-    if (fake_fail_from >= 0 && fake_mallocs >= fake_fail_from) return *p = nullptr, 2;
-    fake_mallocs++;
+    if (fake_most >= 0 && fake_live >= fake_most) return *p = nullptr, 2;
+    if (++fake_live > fake_peak) fake_peak = fake_live;
     return (*p = std::calloc(n ? n : 1, 1)) ? 0 : 2;
 }
-int hipFree(void* p) { std::free(p); return 0; }
+int hipFree(void* p) { fake_live -= p != nullptr; std::free(p); return 0; }
 int hipHostMalloc(void** p, size_t n, unsigned) { return fake_pinned_fails ? 2 : (*p = std::malloc(n)) ? 0 : 2; }
 int hipHostFree(void* p) { std::free(p); return 0; }
 int hipMemcpy(void* d, const void* s, size_t n, int) { std::memcpy(d, s, n); return 0; }
@@ -64,7 +64,8 @@ PRELUDE = """
 import ctypes as C, sys
 import numpy as np
 fake = C.CDLL(%r, mode=C.RTLD_GLOBAL)
-device, mallocs, fail_from = C.c_int.in_dll(fake, "fake_device"), C.c_long.in_dll(fake, "fake_mallocs"), C.c_long.in_dll(fake, "fake_fail_from")
+device, live, peak, most = (t.in_dll(fake, "fake_" + n) for t, n in
+                            ((C.c_int, "device"), (C.c_long, "live"), (C.c_long, "peak"), (C.c_long, "most")))
 pinned_fails, new_limit = C.c_int.in_dll(fake, "fake_pinned_fails"), C.c_size_t.in_dll(fake, "fake_new_limit")
 sys.path[:0] = [%r, %r]
 import multiphaselb_amd as M
