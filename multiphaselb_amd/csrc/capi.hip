@@ -844,7 +844,9 @@ int init_t(mplb_case* c) {
     c->tiles_tried = true;
     const DeviceScope device(c->opts.device);
     HIPCHK(c, device.err);
-    return c->fused ? fused_tiles(c) : tiles_create(c);
+    if (c->fused) fused_tiles(c);
+    else tiles_create(c);
+    return 0;
 }
 
 int field_layout(const mplb_case* c, const std::string& name, void** dptr, int* comps) {

@@ -13,8 +13,9 @@ bool fused_supported(const mplb_case* c, std::string* why);
 int fused_create(mplb_case* c);
 void fused_destroy(mplb_case* c);
 int fused_after_init(mplb_case* c);
-// tiles of a small D2Q9 lattice, where they are the faster way (after the first init)
-int fused_tiles(mplb_case* c);
+// tiles of a small D2Q9 lattice, where they are the faster way and memory allows (after the
+// first init)
+void fused_tiles(mplb_case* c);
 // m steps; level0: the time level before the first of them
 int fused_steps(mplb_case* c, int m, int level0);
 // make the generic device arrays (rho, T, U, f, g ...) describe the current time level

@@ -2525,25 +2525,27 @@ static double tile_passes_us(const Mesh& m, const Fused& z) {
     return z.thermal ? 11.7 + 51e-6 * (double)m.N : 9.2 + 18.5e-6 * (double)m.N;
 }
 
-int fused_tiles(mplb_case* c) {
+void fused_tiles(mplb_case* c) {
     Fused* z = F(c);
     const Mesh& m = c->mesh;
-    if (z->lb != 0 || m.N > 1 << 20 || m.bd.size() >= 255) return 0;
+    if (z->lb != 0 || m.N > 1 << 20 || m.bd.size() >= 255) return;
     const int H = z->thermal ? 3 : 2, n[2] = {m.nx, m.ny};
     int cus = 256;
-    FCHK(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->opts.device));
+    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->opts.device);
     std::vector<int> sizes;
     for (int b = 1; b <= 128; b += b < 32 ? 1 : b < 64 ? 4 : 32) sizes.push_back(b);
     TilePlan p = tile_choose(c, sizes, 0.95 * tile_passes_us(m, *z), [&](const TilePlan& q) {
         return tile_plan_us(q, n, *z, H, cus);
     });
     tile_override(&p);
-    if (p.steps <= 0) return 0;
+    if (p.steps <= 0) return;
     const bool lists[2] = {z->lists[0] != 0, z->lists[1] != 0};
-    const int rc = tile_tables(c, p, H * p.steps, kTileThreads, lists);
-    if (rc || !c->tiles) return rc;
-    if (z->thermal) FCHK(c, hipMalloc(&z->S, sizeof(float) * m.N));
-    return 0;
+    if (!tile_tables(c, p, H * p.steps, kTileThreads, lists)) return;
+    if (z->thermal && hipMalloc(&z->S, sizeof(float) * m.N) != hipSuccess) {
+        (void)hipGetLastError();
+        z->S = nullptr;
+        tiles_destroy(c);
+    }
 }
 
 int fused_create(mplb_case* c) {

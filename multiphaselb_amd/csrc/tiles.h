@@ -80,12 +80,14 @@ TilePlan tile_choose(const mplb_case* c, const std::vector<int>& sizes, double l
                      const std::function<double(const TilePlan&)>& us);
 // MPLB_TILES=bx,by,bz,steps sets the plan (steps 0: no tiles), for tests and timing sweeps
 void tile_override(TilePlan* p);
-// Builds the tables of a plan whose halo is `depth` levels (c->tiles); leaves the case
-// without when a tile has more than cap nodes.  lists: the field has boundary lists.
-int tile_tables(mplb_case* c, const TilePlan& p, int depth, int cap, const bool lists[2]);
+// Builds the tables of a plan whose halo is `depth` levels (c->tiles); false, and the case
+// without, when a tile has more than cap nodes or memory runs out.  lists: the field has
+// boundary lists.
+bool tile_tables(mplb_case* c, const TilePlan& p, int depth, int cap, const bool lists[2]);
 // Chooses tiles for a case that runs in fused passes and builds their tables (c->tiles);
-// leaves the case without when more launches over the whole lattice are the faster way.
-int tiles_create(mplb_case* c);
+// leaves the case without when more launches over the whole lattice are the faster way or
+// memory runs out.
+void tiles_create(mplb_case* c);
 void tiles_destroy(mplb_case* c);
 // m steps from and to the per-routine state (psi valid on entry); level0: the time level
 // before the first of them

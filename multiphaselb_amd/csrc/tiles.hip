@@ -20,14 +20,13 @@ namespace mplb {
 
 namespace {
 
-#define TCHK(c, call)                                                           \
-    do {                                                                        \
-        hipError_t _e = (call);                                                 \
-        if (_e != hipSuccess) {                                                 \
-            (c)->err = std::string(#call) + ": " + hipGetErrorString(_e);       \
-            return MPLB_E_HIP;                                                  \
-        }                                                                       \
-    } while (0)
+// An allocation that fails is no error: the case goes without tiles
+bool device_alloc(void** p, size_t bytes) {
+    if (hipMalloc(p, bytes ? bytes : 1) == hipSuccess) return true;
+    (void)hipGetLastError();
+    *p = nullptr;
+    return false;
+}
 
 int tile_reverse(const Mesh& m, int k) { return m.lbmodel == 0 ? D2Q9::t.rev[k] : D3Q15::t.rev[k]; }
 
@@ -108,7 +107,8 @@ void tile_override(TilePlan* p) {
 
 void tiles_destroy(mplb_case* c) {
     if (!c->tiles) return;
-    for (void* p : c->tiles->owned) (void)hipFree(p);
+    for (void* p : c->tiles->owned)
+        if (p) (void)hipFree(p);
     delete c->tiles;
     c->tiles = nullptr;
     for (void*& p : c->alt) {
@@ -140,6 +140,7 @@ bool over_tiles(size_t tiles, int64_t N, const Fn& fn) {
         }
     };
     std::vector<std::thread> pool;
+    pool.reserve(8);
     for (size_t i = 1; i < std::min<size_t>(8, tiles / 8); i++) {
         try {
             pool.emplace_back(work);
@@ -154,10 +155,10 @@ bool over_tiles(size_t tiles, int64_t N, const Fn& fn) {
 
 }  // namespace
 
-int tiles_create(mplb_case* c) {
+void tiles_create(mplb_case* c) {
     const Mesh& m = c->mesh;
     const bool thermal = c->fc[1].present && c->update[1], fp64 = c->scalar_bytes == 8;
-    if (!c->passes || m.N > 1 << 20 || m.bd.size() > (size_t)kTileLists) return 0;
+    if (!c->passes || m.N > 1 << 20 || m.bd.size() > (size_t)kTileLists) return;
     const int cap = fp64 ? TileOps<double>::max_nodes(m.lbmodel, thermal) : TileOps<float>::max_nodes(m.lbmodel, thermal);
     const int H = thermal ? 3 : 2, extra = c->fc[0].mp.surf ? 1 : 0;
     const int n[3] = {m.nx, m.ny, m.nz};
@@ -168,17 +169,34 @@ int tiles_create(mplb_case* c) {
         return plan_us(q, n, thermal, m.d == 3, fp64, cap, extra, cus);
     });
     tile_override(&p);
-    if (p.steps <= 0) return 0;
+    if (p.steps <= 0) return;
     const bool lists[2] = {c->order[0] != nullptr, c->order[1] != nullptr};
-    const int rc = tile_tables(c, p, H * p.steps + extra, cap, lists);
-    if (rc || !c->tiles) return rc;
+    if (!tile_tables(c, p, H * p.steps + extra, cap, lists)) return;
     // second copies of the macroscopic fields: a launch reads one set and writes the other
     const int comps[7] = {1, 1, 3, 3, 3, 1, 1};
-    for (int i = 0; i < 7; i++) TCHK(c, hipMalloc(&c->alt[i], c->scalar_bytes * comps[i] * m.N));
-    return 0;
+    for (int i = 0; i < 7; i++)
+        if (!device_alloc(&c->alt[i], c->scalar_bytes * comps[i] * m.N)) return tiles_destroy(c);
 }
 
-int tile_tables(mplb_case* c, const TilePlan& p, int D, int cap, const bool lists[2]) {
+namespace {
+
+bool build_tables(mplb_case* c, const TilePlan& p, int D, int cap, const bool lists[2]);
+
+}  // namespace
+
+bool tile_tables(mplb_case* c, const TilePlan& p, int depth, int cap, const bool lists[2]) {
+    try {
+        if (build_tables(c, p, depth, cap, lists)) return true;
+    } catch (const std::bad_alloc&) {
+        // host memory ran out: without tiles as well
+    }
+    tiles_destroy(c);
+    return false;
+}
+
+namespace {
+
+bool build_tables(mplb_case* c, const TilePlan& p, int D, int cap, const bool lists[2]) {
     const Mesh& m = c->mesh;
     const int Q = m.Q;
     const bool thermal = c->fc[1].present && c->update[1];
@@ -223,7 +241,7 @@ int tile_tables(mplb_case* c, const TilePlan& p, int D, int cap, const bool list
                 }
     }
     // tile t's nodes from local[t * cap], level d ending at ends[t * (D + 1) + d]
-    if (own.size() * (size_t)cap > size_t(1) << 26 || D > 250) return 0;
+    if (own.size() * (size_t)cap > size_t(1) << 26 || D > 250) return false;
     const std::unique_ptr<int[]> local(new int[own.size() * cap]), ends(new int[own.size() * (D + 1)]);
     std::atomic<bool> fits{true};
     const bool listed = over_tiles(own.size(), m.N, [&](size_t t, std::vector<int>& mark, std::vector<int>&) {
@@ -256,11 +274,11 @@ int tile_tables(mplb_case* c, const TilePlan& p, int D, int cap, const bool list
             from = to;
         }
     });
-    if (!listed || !fits) return 0;
+    if (!listed || !fits) return false;
     size_t largest = 0;
     for (size_t t = 0; t < own.size(); t++) largest = std::max(largest, (size_t)ends[t * (D + 1) + D]);
     const size_t total = own.size() * largest;
-    if (total > size_t(1) << 23) return 0;
+    if (total > size_t(1) << 23) return false;
     const bool any_fixed = thermal && lists[1];
     std::vector<int16_t> nb(total * Q, -1), inner(any_fixed ? total * Q : 0, 0);
     std::vector<int> gid(total, 0), meta(total, 255 << 24), draw(draws.empty() ? 0 : total);
@@ -296,30 +314,32 @@ int tile_tables(mplb_case* c, const TilePlan& p, int D, int cap, const bool list
             if (!draws.empty()) draw[e] = draws[id];
         }
     });
-    if (!filled) return 0;
+    if (!filled) return false;
     Tiles* s = new Tiles();
     c->tiles = s;
-    auto put = [&](const void* src, size_t bytes, const void** dst) -> int {
+    auto put = [&](const void* src, size_t bytes, const void** dst) {
         void* q = nullptr;
-        TCHK(c, hipMalloc(&q, bytes ? bytes : 1));
-        s->owned.push_back(q);
-        TCHK(c, hipMemcpy(q, src, bytes, hipMemcpyHostToDevice));
+        s->owned.push_back(nullptr);
+        if (!device_alloc(&q, bytes)) return false;
+        s->owned.back() = q;
         *dst = q;
-        return 0;
+        return hipMemcpy(q, src, bytes, hipMemcpyHostToDevice) == hipSuccess;
     };
-    int rc = put(gid.data(), sizeof(int) * total, (const void**)&s->t.gid);
-    if (!rc) rc = put(nb.data(), sizeof(int16_t) * nb.size(), (const void**)&s->t.nb);
-    if (!rc && any_fixed) rc = put(inner.data(), sizeof(int16_t) * inner.size(), (const void**)&s->t.inner);
-    if (!rc) rc = put(meta.data(), sizeof(int) * total, (const void**)&s->t.meta);
-    if (!rc && !draw.empty()) rc = put(draw.data(), sizeof(int) * total, (const void**)&s->t.draw);
-    if (rc) return rc;
+    if (!put(gid.data(), sizeof(int) * total, (const void**)&s->t.gid) ||
+        !put(nb.data(), sizeof(int16_t) * nb.size(), (const void**)&s->t.nb) ||
+        (any_fixed && !put(inner.data(), sizeof(int16_t) * inner.size(), (const void**)&s->t.inner)) ||
+        !put(meta.data(), sizeof(int) * total, (const void**)&s->t.meta) ||
+        (!draw.empty() && !put(draw.data(), sizeof(int) * total, (const void**)&s->t.draw)))
+        return false;
     s->t.tiles = (int)own.size();
     s->t.stride = (int)largest;
     s->t.total = (int64_t)total;
     s->nodes = (int)largest;
     s->steps = p.steps;
-    return 0;
+    return true;
 }
+
+}  // namespace
 
 template <typename T>
 void tiles_run(mplb_case* c, int m, int level0) {
