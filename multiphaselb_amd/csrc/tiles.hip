@@ -28,6 +28,9 @@ bool device_alloc(void** p, size_t bytes) {
     return false;
 }
 
+// rho, T, U, Fi, Ft, ss, psi (mplb_case::alt): those that change with heat transfer only
+constexpr bool kHeatField[7] = {false, true, false, false, false, true, false};
+
 int tile_reverse(const Mesh& m, int k) { return m.lbmodel == 0 ? D2Q9::t.rev[k] : D3Q15::t.rev[k]; }
 
 // Time of one step with a plan, in microseconds: a launch with the load of its state, then
@@ -173,9 +176,10 @@ void tiles_create(mplb_case* c) {
     const bool lists[2] = {c->order[0] != nullptr, c->order[1] != nullptr};
     if (!tile_tables(c, p, H * p.steps + extra, cap, lists)) return;
     // second copies of the macroscopic fields: a launch reads one set and writes the other
+    // (T and the heat source change with heat transfer only)
     const int comps[7] = {1, 1, 3, 3, 3, 1, 1};
     for (int i = 0; i < 7; i++)
-        if (!device_alloc(&c->alt[i], c->scalar_bytes * comps[i] * m.N)) return tiles_destroy(c);
+        if ((thermal || !kHeatField[i]) && !device_alloc(&c->alt[i], c->scalar_bytes * comps[i] * m.N)) return tiles_destroy(c);
 }
 
 namespace {
@@ -380,7 +384,7 @@ void tiles_run(mplb_case* c, int m, int level0) {
         TileOps<T>::run(c->mesh.lbmodel, c->stream, a, thermal, s->nodes);
         for (int f = 0; f < (thermal ? 2 : 1); f++) std::swap(c->f[f], c->f_alt[f]);
         for (int i = 0; i < 7; i++)
-            if (thermal || (i != 1 && i != 5)) std::swap(*cur[i], c->alt[i]);
+            if (thermal || !kHeatField[i]) std::swap(*cur[i], c->alt[i]);
         done += a.steps;
     }
 }

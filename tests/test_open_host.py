@@ -32,3 +32,19 @@ for tiles in ("0", ""):
     n.append((opened, inited))
 assert n[0][0] == n[0][1] == n[1][0] < n[1][1], n
 """ % kind))
+
+
+def test_isothermal_tiles_keep_no_second_temperature_and_heat_source(tmp_path):
+    """Second copies are for the fields a launch writes: five of them beside the three tables
+    without heat transfer, all seven with it."""
+    print(run(tmp_path, """
+for ht, extra in ((False, 3 + 5), (True, 3 + 7)):
+    c = M.Case(make_case_dir(d2(nx=128, ny=128, btype=3)), device=0, heat_transfer=ht)
+    opened = live.value
+    for name in ("rho", "T"):
+        c.set(name, np.ones(c.N))
+    c.init()
+    assert live.value - opened == extra, (ht, live.value - opened)
+    c.step(9)
+    c.close()
+"""))
