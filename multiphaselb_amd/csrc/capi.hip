@@ -437,12 +437,13 @@ int setup_passes(mplb_case* c) {
     // neighbours are computed from coordinates where the lattice is a box in box order, with
     // the odd links and the listed nodes on its surface
     c->pass_faces = m.structured && plain_inside(m, any) ? odd_faces(m, any) : kAllTable;
+    // (without memory for the tables the case keeps one kernel per routine)
     for (int f = 0; f < 2; f++) {
         if (!lists[f]) continue;
-        HIPCHK(c, hipMalloc(&c->order[f], m.N));
+        if (!device_alloc((void**)&c->order[f], m.N)) return 0;
         HIPCHK(c, hipMemcpy(c->order[f], order[f].data(), m.N, hipMemcpyHostToDevice));
     }
-    if (c->fc[1].present && c->update[1]) HIPCHK(c, hipMalloc(&c->sumg, c->scalar_bytes * m.N));
+    if (c->fc[1].present && c->update[1] && !device_alloc(&c->sumg, c->scalar_bytes * m.N)) return 0;
     c->passes = true;
     const bool thermal = c->fc[1].present && c->update[1];
     if (m.d == 3 && !thermal && c->pass_faces == 0) {

@@ -63,6 +63,14 @@ public:
 private:
     int before_ = -1;
 };
+
+// Device memory that a case can do without: a failure is no error of the call
+inline bool device_alloc(void** p, size_t bytes) {
+    if (hipMalloc(p, bytes ? bytes : 1) == hipSuccess) return true;
+    (void)hipGetLastError();
+    *p = nullptr;
+    return false;
+}
 }
 
 struct mplb_case {

@@ -2541,11 +2541,7 @@ void fused_tiles(mplb_case* c) {
     if (p.steps <= 0) return;
     const bool lists[2] = {z->lists[0] != 0, z->lists[1] != 0};
     if (!tile_tables(c, p, H * p.steps, kTileThreads, lists)) return;
-    if (z->thermal && hipMalloc(&z->S, sizeof(float) * m.N) != hipSuccess) {
-        (void)hipGetLastError();
-        z->S = nullptr;
-        tiles_destroy(c);
-    }
+    if (z->thermal && !device_alloc((void**)&z->S, sizeof(float) * m.N)) tiles_destroy(c);
 }
 
 int fused_create(mplb_case* c) {

@@ -20,14 +20,6 @@ namespace mplb {
 
 namespace {
 
-// An allocation that fails is no error: the case goes without tiles
-bool device_alloc(void** p, size_t bytes) {
-    if (hipMalloc(p, bytes ? bytes : 1) == hipSuccess) return true;
-    (void)hipGetLastError();
-    *p = nullptr;
-    return false;
-}
-
 // rho, T, U, Fi, Ft, ss, psi (mplb_case::alt): those that change with heat transfer only
 constexpr bool kHeatField[7] = {false, true, false, false, false, true, false};
 

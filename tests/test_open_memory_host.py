@@ -42,3 +42,22 @@ for limit in (1 << 20, 3 << 18):
     opened(%s)
     new_limit.value = 0
 """ % (kind, kind)))
+
+
+def test_no_device_memory_for_the_passes(tmp_path):
+    """The per-node list numbers and the new temperature of the fused passes: without them the
+    case runs one kernel per routine."""
+    print(run(tmp_path, """
+from multiphaselb_amd.casefiles import BC
+spec = d2(nx=5, ny=40, btype=1, f_bc={"Y0": BC("bounceBack"), "Y1": BC("bounceBack")},
+          g_bc={"Y0": BC("fixedT", (0.95 * TC,)), "Y1": BC("fixedT", (0.8 * TC,))})
+M.Case(make_case_dir(spec), device=0).close()
+for most.value in range(peak.value - 3, peak.value + 1):
+    c = M.Case(make_case_dir(spec), device=0)
+    for name in ("rho", "T"):
+        c.set(name, np.ones(c.N))
+    c.init()
+    assert c.step(3) == 3
+    c.close()
+    assert live.value == 0
+"""))
