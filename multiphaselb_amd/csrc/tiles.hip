@@ -6,10 +6,10 @@
 #include <atomic>
 #include <cstdio>
 #include <cstdlib>
+#include <exception>
 #include <memory>
 #include <new>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -135,11 +135,10 @@ bool over_tiles(size_t tiles, int64_t N, const Fn& fn) {
         }
     };
     std::vector<std::thread> pool;
-    pool.reserve(8);
     for (size_t i = 1; i < std::min<size_t>(8, tiles / 8); i++) {
         try {
             pool.emplace_back(work);
-        } catch (const std::system_error&) {
+        } catch (const std::exception&) {
             break;                       // fewer threads do the same
         }
     }

@@ -14,8 +14,8 @@
 #include <atomic>
 #include <condition_variable>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -141,7 +141,7 @@ int stage_transfer(mplb_case* c, void* planes, int64_t N, int comps, double* hos
     std::vector<std::thread> pool;
     try {
         for (int w = 0; w < (int)std::min<int64_t>(kWorkers, chunks); w++) pool.emplace_back(work);
-    } catch (const std::system_error&) {
+    } catch (const std::exception&) {
         // fewer threads than asked for; with none at all this thread copies
     }
     hipError_t e = hipSuccess;

@@ -27,3 +27,14 @@ pinned_fails.value = 0
 c.set("U", a)
 c.close()
 """))
+
+
+def test_a_transfer_that_cannot_start_threads_copies_by_itself(tmp_path):
+    """Worker threads fail to start for want of memory as well as of threads."""
+    print(run(tmp_path, OPEN + """
+c.set("U", a)
+new_limit.value = 20
+c.set("U", a)
+c.get("U")
+new_limit.value = 0
+"""))
