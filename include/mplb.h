@@ -277,7 +277,8 @@ int mplb_mlp_gradient(mplb_mlp* n, const float* x, const float* t, float* loss, 
  * call starts a fresh Adam run: moments zeroed, bias-correction step count from 1. */
 int mplb_mlp_train(mplb_mlp* n, const float* X, const float* T, int nsamples, const int32_t* idx, int iters,
                    float lr, float beta1, float beta2, float eps, float* loss_hist);
-/* intermediate tensors of the last gradient call as FP32: "a" (level j BF16 input/
+/* intermediate tensors of the last forward, gradient or training call (its last batch; a
+ * forward call leaves "dz" and "dzb" as they were) as FP32: "a" (level j BF16 input/
  * activation), "a32", "y", "dz", "dzb", "wb" (layer j BF16 weights [in_padded][out]) */
 int mplb_mlp_tensor(mplb_mlp* n, const char* name, int j, float* out, size_t count);
 

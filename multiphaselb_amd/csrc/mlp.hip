@@ -287,12 +287,14 @@ struct Net {
     const float* T;
     const int* idx;
     int* counter;                      // [0] iteration of the next k_rows, [1] of the last one
-    float* y;                          // forward only
+    float* y;                          // forward only: all rows' outputs
     float* rowsum;
     __bf16* abt[kNetLayers];           // BF16 activations of levels 0..L-1, rows: channels (frag)
     __bf16* dzt[kNetLayers + 1];       // BF16 dL/dz of levels 1..L, rows: channels (frag)
     float* dz32[kNetLayers + 1];       // [B][w]
-    // KEEP: the row-major copies mplb_mlp_tensor hands out
+    // KEEP: the row-major copies mplb_mlp_tensor hands out, of the rows from keep0 on
+    int keep0;
+    float* ykeep;
     __bf16* ab[kNetLayers];
     float* a32[kNetLayers + 1];
     __bf16* dzb[kNetLayers + 1];
@@ -356,6 +358,8 @@ __global__ void __launch_bounds__(kRowThreads) k_rows(Net g) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int r = lane & 15, kq = (lane >> 4) * 8, m0 = (lane >> 4) * 4;
     const int b0 = blockIdx.x * kRows, B = g.B;
+    const int k0 = b0 - g.keep0;                         // first kept row (KEEP; below 0: none)
+    const bool keep = KEEP && k0 >= 0;
     constexpr int kWaves = kRowThreads / 64, kHeld = 8, kTargets = 4;
     bf16x8 held[kHeld];
     float held_bias = 0.f;
@@ -385,7 +389,7 @@ __global__ void __launch_bounds__(kRowThreads) k_rows(Net g) {
         const float x = c < g.w[0] && row < g.rows ? g.X[(size_t)row * g.w[0] + c] : 0.f;
         buf[m * ld + c] = bf(x);
         if (BWD) g.abt[0][frag(c, b0 + m, B)] = bf(x);
-        if (KEEP) g.ab[0][(size_t)(b0 + m) * kInPad + c] = bf(x);
+        if (keep) g.ab[0][(size_t)(k0 + m) * kInPad + c] = bf(x);
     }
     float target[kTargets];
     if constexpr (BWD) {
@@ -427,10 +431,11 @@ __global__ void __launch_bounds__(kRowThreads) k_rows(Net g) {
                     v = tanhf(v);
                     t[e] = bf(v);
                     to[m * ld + n] = t[e];
-                    if (KEEP) g.ab[l + 1][(size_t)(b0 + m) * N + n] = t[e];
-                    if (KEEP) g.a32[l + 1][(size_t)(b0 + m) * N + n] = v;
-                } else if (!BWD || KEEP) {
-                    if (b0 + m < B) g.y[(size_t)(b0 + m) * N + n] = v;
+                    if (keep) g.ab[l + 1][(size_t)(k0 + m) * N + n] = t[e];
+                    if (keep) g.a32[l + 1][(size_t)(k0 + m) * N + n] = v;
+                } else {
+                    if (!BWD && b0 + m < B) g.y[(size_t)(b0 + m) * N + n] = v;
+                    if (keep) g.ykeep[(size_t)(k0 + m) * N + n] = v;
                 }
                 if (BWD) level[m * stride + n] = v;
             }
@@ -457,7 +462,7 @@ __global__ void __launch_bounds__(kRowThreads) k_rows(Net g) {
             level[m * (n + 1) + c] = d;
             to[m * ld + c] = bf(dz);
             g.dz32[g.L][(size_t)(b0 + m) * n + c] = dz;
-            if (KEEP) g.dzb[g.L][(size_t)(b0 + m) * n + c] = bf(dz);
+            if (keep) g.dzb[g.L][(size_t)(k0 + m) * n + c] = bf(dz);
         };
 #pragma unroll
         for (int j = 0; j < kTargets; j++) {
@@ -499,7 +504,7 @@ __global__ void __launch_bounds__(kRowThreads) k_rows(Net g) {
                     t[e] = bf(dz);
                     out[m * ld + c] = t[e];
                     g.dz32[l][(size_t)(b0 + m) * N + c] = dz;
-                    if (KEEP) g.dzb[l][(size_t)(b0 + m) * N + c] = t[e];
+                    if (keep) g.dzb[l][(size_t)(k0 + m) * N + c] = t[e];
                 }
                 *(bf16x4*)(g.dzt[l] + frag(c, b0 + m0, B)) = t;
             }
@@ -839,7 +844,7 @@ Net net_args(mplb_mlp* n) {
     g.X = n->X;
     g.T = n->T;
     g.counter = n->counter;
-    g.y = n->y;
+    g.ykeep = n->y;
     g.rowsum = n->rowsum;
     return g;
 }
@@ -943,7 +948,7 @@ int mplb_mlp_create(int nlayers, const int* widths, int batch, int device, mplb_
     if (nlayers <= kNetLayers && lds <= kRowsLds) {
         n->lds_bwd = lds;
         n->lds_fwd = rows_lds(nlayers, n->w.data(), n->wp.data(), false);
-        MCHK(n, hipFuncSetAttribute((const void*)k_rows<false, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        MCHK(n, hipFuncSetAttribute((const void*)k_rows<false, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)kRowsLds));
         MCHK(n, hipFuncSetAttribute((const void*)k_rows<true, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)kRowsLds));
@@ -998,18 +1003,20 @@ int mplb_mlp_forward(mplb_mlp* n, const float* x, int rows, float* y) {
     MCHK(n, hipSetDevice(n->dev));
     const int din = n->w[0], dout = n->w[n->L], B = n->B;
     if (n->lds_bwd) {
-        constexpr int kChunk = 65536;          // rows on the device at a time
-        const size_t most = (size_t)std::min(rows, kChunk);
+        const int chunk = std::max(1, 65536 / B) * B;    // rows on the device at a time
+        const size_t most = (size_t)std::min(rows, chunk);
         int rc = ensure(n, &n->X, &n->X_cap, most * din);
         if (!rc) rc = ensure(n, &n->Y, &n->Y_cap, most * dout);
         if (rc) return rc;
         Net g = net_args(n);
         g.y = n->Y;
-        for (int r0 = 0; r0 < rows; r0 += kChunk) {
-            g.B = g.rows = std::min(kChunk, rows - r0);
+        for (int r0 = 0; r0 < rows; r0 += chunk) {
+            g.B = g.rows = std::min(chunk, rows - r0);
+            // the last batch of rows stays for mplb_mlp_tensor, filled up with empty ones
+            g.keep0 = (g.rows - 1) / B * B;
             MCHK(n, hipMemcpyAsync(n->X, x + (size_t)r0 * din, sizeof(float) * g.rows * din, hipMemcpyHostToDevice,
                                    n->stream));
-            k_rows<false, false><<<(unsigned)((g.rows + kRows - 1) / kRows), kRowThreads, n->lds_fwd, n->stream>>>(g);
+            k_rows<false, true><<<(unsigned)((g.keep0 + B) / kRows), kRowThreads, n->lds_fwd, n->stream>>>(g);
             MCHK(n, hipGetLastError());
             MCHK(n, hipMemcpyAsync(y + (size_t)r0 * dout, n->Y, sizeof(float) * g.rows * dout, hipMemcpyDeviceToHost,
                                    n->stream));
@@ -1091,7 +1098,8 @@ int mplb_mlp_train(mplb_mlp* n, const float* X, const float* T, int nsamples, co
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     MCHK(n, hipStreamBeginCapture(n->stream, hipStreamCaptureModeThreadLocal));
-    if (n->lds_bwd) {
+    // the last iteration of the two-launch path also leaves its tensors for mplb_mlp_tensor
+    auto rows_and_weights = [&](bool keep) {
         int blocks = 0;
         Grads gr = grad_args(n, &blocks);
         gr.hist = n->hist;
@@ -1099,8 +1107,13 @@ int mplb_mlp_train(mplb_mlp* n, const float* X, const float* T, int nsamples, co
         Net g = net_args(n);
         g.idx = n->idx;
         g.rows = nsamples;
-        k_rows<true, false><<<(unsigned)(B / kRows + 8 * kHelpers), kRowThreads, n->lds_bwd, n->stream>>>(g);
+        const unsigned row_blocks = (unsigned)(B / kRows + 8 * kHelpers);
+        if (keep) k_rows<true, true><<<row_blocks, kRowThreads, n->lds_bwd, n->stream>>>(g);
+        else k_rows<true, false><<<row_blocks, kRowThreads, n->lds_bwd, n->stream>>>(g);
         k_weights<true><<<(unsigned)blocks, 256, 0, n->stream>>>(gr);
+    };
+    if (n->lds_bwd) {
+        rows_and_weights(false);
     } else {
         k_gather<<<B, 64, 0, n->stream>>>(n->X, n->T, n->idx, n->counter, B, din, dout, n->ab[0], n->abt[0], n->tgt);
         forward(n);
@@ -1112,7 +1125,11 @@ int mplb_mlp_train(mplb_mlp* n, const float* X, const float* T, int nsamples, co
     }
     MCHK(n, hipStreamEndCapture(n->stream, &graph));
     MCHK(n, hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
-    for (int it = 0; it < iters; it++) MCHK(n, hipGraphLaunch(exec, n->stream));
+    for (int it = n->lds_bwd ? 1 : 0; it < iters; it++) MCHK(n, hipGraphLaunch(exec, n->stream));
+    if (n->lds_bwd) {
+        rows_and_weights(true);
+        MCHK(n, hipGetLastError());
+    }
     MCHK(n, hipStreamSynchronize(n->stream));
     MCHK(n, hipGraphExecDestroy(exec));
     MCHK(n, hipGraphDestroy(graph));
@@ -1120,7 +1137,7 @@ int mplb_mlp_train(mplb_mlp* n, const float* X, const float* T, int nsamples, co
     return 0;
 }
 
-// Intermediate tensors of the last forward/backward, as FP32 (BF16 ones widened):
+// Intermediate tensors of the last forward, gradient or training call (its last batch), as FP32 (BF16 ones widened):
 // "x" level-0 BF16 input [B][32]; "a" level j BF16 activation [B][w_j] (j = 0..L-1);
 // "a32" FP32 activation (1..L-1); "y" output [B][w_L]; "dz" FP32 dL/dz of level j
 // (1..L); "dzb" its BF16 copy; "wb" BF16 weights of layer j [32 or w_j][w_j+1].
