@@ -206,7 +206,7 @@ int mplb_batch_run_to_steady(mplb_batch* b, double threshold, int check_every, i
 /* "rho" or "p" (macroPressure.c:20-65, liMRT form) of case i at its current level. */
 int mplb_batch_get_field(mplb_batch* b, int i, const char* name, double* out, size_t n);
 int64_t mplb_batch_case_steps(const mplb_batch* b, int i);
-/* Autotuner: times the single-pass kernel at 16/32/64 rows per work item (when every
+/* Autotuner: times the single-pass kernel at 8/16/32 rows per work item (when every
  * case is at most 256 nodes wide) and the two-pass kernels at 64..1024 nodes per
  * workgroup, each with and without the XCD-ordered work table, over steps_per_trial
  * steps each on the current cases (which advance meanwhile), and keeps the fastest.

@@ -1067,7 +1067,10 @@ int mplb_batch_tune(mplb_batch* b, int steps_per_trial, int* chosen_block, int* 
     const int trial = std::max(2, steps_per_trial & ~1);    // even: the buffers end where they started
     // candidates: rows per single-pass item (when every case fits a workgroup row), then
     // nodes per workgroup of the two-pass kernels
-    const int rows_cand[] = {16, 32, 64};
+    // (64 rows per item are the fastest of no batch that was timed; us per step at 8 / 16 / 32 / 64
+    // rows, FP32: 4096 cases of 64^2 245 / 316 / 327 / 326, 1024 of 64 to 256 nodes 481 / 483 / 527 / 534,
+    // 500 of 256^2 482 / 512 / 516 / 570, FP64 953 / 1038 / 995 / 978, FP16S 349 / 339 / 344 / 400)
+    const int rows_cand[] = {8, 16, 32};
     int best_r = b->mrows;
     const int bs0 = b->bsize;
     for (int xo = 0; xo < 2; xo++) {
