@@ -1,7 +1,6 @@
-// Neighbours of a node of a structured box: computed from wrapped coordinates, or read
-// from the neighbour table on the faces of the box whose links are not the duplicate-node
-// periodic wrap or that carry a boundary condition (odd_faces,
-// mesh.h).
+// Neighbours of a node of a structured box: computed from wrapped coordinates, or read from
+// the neighbour table: on the faces that cover the nodes with odd links or a boundary
+// condition (odd_faces, mesh.h), or everywhere where such nodes lie inside (plain_inside).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -10,13 +9,13 @@
 
 namespace mplb {
 
-// face_table of a lattice whose nodes are all read through the table
+// bits of face_table: the faces x0 x1 y0 y1 z0 z1, and this one for all nodes
 constexpr int kAllTable = 64;
 
 struct NodePos {
     int i, j, k;
     int64_t id;
-    bool table;         // on a face whose links must be read from the neighbour table
+    bool table;         // links and boundary conditions come from the tables
     bool valid;
     unsigned X[3], Y[3], Z[3];   // wrapped coordinates u-1, u, u+1 premultiplied by the strides
 };

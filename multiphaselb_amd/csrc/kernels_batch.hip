@@ -411,8 +411,9 @@ __device__ inline int wrap_dup(int u, int n) { return u < 0 ? u + (n - 1) : (u >
 // psi never goes to memory.  Per node and step the populations are read once and written
 // once.  LDS hazards: row y + 1 goes to slot (y + 2 - y0) & 3, which no lane reads while
 // colliding row y - 1 or y, and one barrier per row publishes it.
-// Bound: memory (256 cases of 64 to 256 nodes in FP32: 1.10 x the 72 B per node and step at
-// 3.9 TB/s, VALU issue 45% busy).  Six waves per SIMD in FP32 and FP16 (79 VGPRs), four in
+// Bound: memory and VALU issue together, at the latency of a row's chain (256 cases of 64 to
+// 256 nodes in FP32, 140 us per launch: 45 B read and 36 B written per node, 4.7 TB/s, VALU
+// issue 52% busy).  Six waves per SIMD in FP32 and FP16 (79 VGPRs), four in
 // FP64 (127): with the model constants converted in the kernel they held 20 vector registers
 // and, with 64-bit addresses, the FP32 kernel ran four, 197 us per step at 32 rows per item
 // against 152.  Issuing row y + 2's pulls before row y collides (108 VGPRs) was slower, 171

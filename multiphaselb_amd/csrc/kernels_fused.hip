@@ -1,20 +1,24 @@
 // Fused structured-box path: FP32 arithmetic, FP32 or FP16-deviation population storage.
 //
-// The state between steps is the post-collision population set of the current step.
-// Isothermal D3Q15 boxes (FP32 or FP16 storage) whose links are all the periodic wrap take
-// one single-pass kernel per step (k_fused_march: pull-stream, psi in an LDS ring of
-// planes, force, velocity and collision).  Other boxes take two node-parallel passes (three with heat
-// transfer):
-//   K1  pull-stream f (and g) from the post-collision buffers, apply the boundary
-//       conditions of the node in registers, and write what the neighbours' stencils
-//       need: psi = potential(rho, T) (isothermal) or rho and sum g (thermal);
-//   KH  (thermal) heat source from the rho / T / U stencils, new T, psi;
-//   K2  pull again (the same addresses K1 touched), psi stencil -> interaction force ->
-//       velocity, then the MRT collisions of the next step, written to the other buffer.
-// Interior nodes compute the pull source as a fixed offset; nodes on the box surface
-// read the neighbour table, so the reference's duplicate-node periodic links and wall
-// links are followed exactly.  Block b of K1/K2 covers the 256 consecutive node ids
-// [256 b, 256 b + 256).
+// The state between steps is the post-collision population set of the current step.  A step
+// is one of
+//   - several steps per launch in overlapping tiles on small D2Q9 lattices (k_fused_tile, where
+//     tile_plan_us finds it faster than the passes);
+//   - one single-pass kernel on D3Q15 boxes whose links are all the periodic wrap, where
+//     march_pays finds it faster (k_fused_march: pull-stream, psi in an LDS ring of planes,
+//     force, velocity and collision; k_fused_tmarch with heat transfer);
+//   - two node-parallel passes (three with heat transfer) on all other boxes:
+//     K1  pull-stream f (and g) from the post-collision buffers, apply the boundary
+//         conditions of the node in registers, and write what the neighbours' stencils
+//         need: psi = potential(rho, T) (isothermal) or rho and sum g (thermal);
+//     KH  (thermal) heat source from the rho / T / U stencils, new T, psi;
+//     K2  pull again (the same addresses K1 touched), psi stencil -> interaction force ->
+//         velocity, then the MRT collisions of the next step, written to the other buffer.
+// The passes compute neighbours from coordinates, periodic wrap included; nodes on the faces
+// that odd_faces (mesh.h) picks read the neighbour table and their boundary codes, so that
+// wall links are followed exactly, and so does the whole lattice where nodes off the surface
+// carry a condition or odd links (plain_inside).  Block b of K1/K2 covers the 256
+// consecutive node ids [256 b, 256 b + 256).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -1558,9 +1562,6 @@ k_fused_march_lds(FArgs a) {
     store_post(z1 - 1);
 }
 
-// Post-stream, post-boundary populations of the current time level (what the
-// reference holds in f.value after updateBoundaries), FP32 SoA.
-
 // ---------------------------------------------------------------------------
 // Several steps per launch on small D2Q9 lattices.  A step of a lattice of some ten thousand
 // nodes is two or three launches of about 5 us each, whatever the nodes cost.  Here a
@@ -1601,7 +1602,7 @@ __device__ inline void tile_fixed_temperature(const FArgs& a, int64_t id, const 
         if (!(miss >> q & 1) || (miss >> L::t.rev[q] & 1)) continue;
         const int n = at[L::t.rev[q]];
         const float gnb = gs[q][inner[e + q * total]];
-        const float U[3] = {sU[0][n], sU[1][n], L::D == 3 ? sU[L::D - 1][n] : 0.f};
+        const float U[3] = {sU[0][n], sU[1][n], 0.f};
         float geq[L::Q];
         if (a.gmodel == 1) my_geq<L, float>(sT[n], U, a1, a2, geq);
         else litemp_geq<L, float>(sT[n], U, geq);
@@ -1631,6 +1632,7 @@ __device__ inline void tile_bounce_back(unsigned miss, float* v) {
 
 template <class L, typename S, bool THERMAL, int NT>
 __global__ void __launch_bounds__(NT) k_fused_tile(FArgs a, FTileArgs p) {
+    static_assert(L::D == 2, "D2Q9");
     __shared__ float fs[L::Q][NT], s_psi[NT];
     __shared__ float gs[THERMAL ? L::Q : 1][THERMAL ? NT : 1];
     __shared__ float s_rho[THERMAL ? NT : 1], s_T[THERMAL ? NT : 1], s_U[L::D][THERMAL ? NT : 1];
@@ -1817,6 +1819,8 @@ __global__ void __launch_bounds__(NT) k_fused_tile(FArgs a, FTileArgs p) {
     }
 }
 
+// Post-stream, post-boundary populations of the current time level (what the
+// reference holds in f.value after updateBoundaries), FP32 SoA.
 template <class L, typename S, bool G>
 __global__ void __launch_bounds__(256) k_fused_materialize(FArgs a, float* out) {
     const NodePos p = node_pos<L>(a);

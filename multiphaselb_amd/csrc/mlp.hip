@@ -477,8 +477,8 @@ __global__ void __launch_bounds__(kRowThreads) k_rows(Net g) {
             g.dzt[g.L][frag(c, b0 + m, B)] = to[m * ld + c];
         }
         // row sums of squared errors: 256 partial sums over every 256th column, added in
-        // order, by one lane per row of the last wave (which for a 256-wide layer has a tile of
-        // its own to finish, so the sums come after the backward pass)
+        // order, by one lane per row of the first wave after the backward pass (in which every
+        // wave of a 256-wide layer has a tile to finish)
         const float* diff = level;
         for (int l = g.L - 1; l > 0; l--) {
             const int N = g.wp[l], K = g.w[l + 1];
